@@ -32,7 +32,11 @@ namespace dsa {
 
 // rowinfo[b][h][i] = (lse_i * log2 e, dO_i . O_i) for i < LqP: D / VEC lanes
 // per row, one 16-byte load each, then a butterfly sum.  Rows past Lq get
-// (inf, 0); dead rows already have lse = inf.  Block blk of 256 threads.
+// (inf, 0); dead rows already have lse = inf.  With far blocks (FarSpan) two
+// more planes hold the same with lse * log2 e less a_i * scale * log2 e, a_i
+// the c2p term of the far blocks of either side: dkdv then has P = exp2(y *
+// scale * log2 e - lse') of a far tile from the plane of its side, with no
+// addition per element.  Block blk of 256 threads.
 template <typename T, int D>
 DSA_DEV void prep_delta(const BwdParams& bp, int blk) {
   constexpr int VEC = 16 / sizeof(T);
@@ -42,7 +46,7 @@ DSA_DEV void prep_delta(const BwdParams& bp, int blk) {
   const int64_t n = (int64_t)p.B * p.H * p.LqP;
   const int64_t row = ((int64_t)blk * 256 + threadIdx.x) / LPR;
   const int part = threadIdx.x % LPR;
-  float acc = 0.f;
+  float acc = 0.f, fa[2] = {0.f, 0.f};
   int i = 0, h = 0, b = 0;
   if (row < n) {
     i = (int)(row % p.LqP);
@@ -62,21 +66,38 @@ DSA_DEV void prep_delta(const BwdParams& bp, int blk) {
 #pragma unroll
         for (int e = 0; e < VEC; ++e) acc += (float)lv[e] * (float)dv[e];
       }
+      if (p.far && (p.flags & 1)) {
+        const T* q = p.qc ? (const T*)p.qc + (int64_t)b * p.qcs[0] + (int64_t)i * p.qcs[1] + (int64_t)h * p.qcs[2]
+                          : (const T*)p.q + (int64_t)b * p.qs[0] + (int64_t)i * p.qs[1] + (int64_t)h * p.qs[2];
+        const vecT qv = *reinterpret_cast<const vecT*>(q + part * VEC);
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          const int r = offset_row(p.rel, far_offset(p, s), p.Lq, p.Lk, p.A, false);
+          const vecT kv = *reinterpret_cast<const vecT*>((const T*)p.kr + (int64_t)h * p.krs[0] + (int64_t)r * p.krs[1] + part * VEC);
+#pragma unroll
+          for (int e = 0; e < VEC; ++e) fa[s] += (float)qv[e] * (float)kv[e];
+        }
+      }
     }
   }
 #pragma unroll
   for (int m = LPR / 2; m >= 1; m >>= 1) acc += __shfl_xor(acc, m);
+  if (p.far) {
+#pragma unroll
+    for (int m = LPR / 2; m >= 1; m >>= 1) {
+      fa[0] += __shfl_xor(fa[0], m);
+      fa[1] += __shfl_xor(fa[1], m);
+    }
+  }
   if (row < n && part == 0) {
     const float lse2 = (i < p.Lq) ? p.lse[((int64_t)b * p.H + h) * p.Lq + i] * kLog2e : INFINITY;
     *reinterpret_cast<float2*>(bp.rowinfo + 2 * row) = make_float2(lse2, acc);
+    if (p.far) {
+      const float sl2 = p.scale * kLog2e;
+      *reinterpret_cast<float2*>(bp.rowinfo + 2 * (n + row)) = make_float2(lse2 - fa[0] * sl2, acc);
+      *reinterpret_cast<float2*>(bp.rowinfo + 2 * (2 * n + row)) = make_float2(lse2 - fa[1] * sl2, acc);
+    }
   }
-}
-
-// Table row of offset d (clamped into the relative-position table's range).
-DSA_DEV int offset_row(const int32_t* rel, int d, int Lq, int Lk, int A, bool p2c) {
-  d = min(max(d, -(Lk - 1)), Lq - 1);
-  const int t = min(max(rel[d + Lk - 1], -A), A);
-  return p2c ? p2c_row(t, A) : c2p_row(t, A);
 }
 
 // krgt[h][d][t] = Kr[h][c(t' - OFF)][d] with t' = t ^ (VEC - 1) (each
@@ -192,6 +213,10 @@ __global__ __launch_bounds__(256) void dsa_bwd_prep_kernel(BwdParams bp, PrepBlo
   if (blk < nb.gather) {
     prep_gather<T, D>(bp, blk);
   } else if (blk < nb.gather + nb.seg) {
+    if (bp.f.far && blk == nb.gather && threadIdx.x < 64) {
+      const FarSpan fs = far_span(bp.f);
+      if (threadIdx.x == 0) bp.farspan[0] = fs.pos, bp.farspan[1] = fs.neg;
+    }
     prep_segments(bp, blk - nb.gather);
   } else if (blk < nb.gather + nb.seg + nb.chunk) {
     prep_chunks(bp, blk - nb.gather - nb.seg);

@@ -41,7 +41,9 @@ constexpr int NW = 4, WK = 32, BKW = 128, BQ = 32;
 // DROP: attention dropout with the forward's keep bits p.drop
 // (dsa_dropout.h): dV sums the kept probabilities, scaled by p.drop_scale,
 // and dP keeps the kept pairs' dO . v, scaled the same way.
-template <typename T, int D, int MASK, bool DROP = false>
+// FAR: calls that can have far blocks (FarSpan, p.far); kept out of the others'
+// code, whose registers are all taken (252 of 256).
+template <typename T, int D, int MASK, bool DROP, bool FAR>
 __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
   using namespace kvcfg;
   using M = Mfma<T>;
@@ -61,7 +63,8 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
   // next row's leading ones.
   constexpr int ZL = 32;
   constexpr int SROW = sizeof(T) == 2 ? 72 : 76;         // few bank conflicts for 16-byte row reads
-  constexpr int SW = (WK + 1) * SROW;
+  // (the last row's right-hand zeros: the walk reads up to 26 elements past it)
+  constexpr int SW = WK * SROW + 32;
   // qrgt ring: NRB blocks of 32 offsets, each stored [chunk c][d][VEC] so that
   // a fragment read (one chunk of 16 consecutive d rows) is contiguous.
   constexpr int NRB = 6, RBE = 32 * D;
@@ -84,23 +87,42 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
   constexpr bool SEGM = seg_mode(MASK);
   constexpr int MAXQT = 1024;  // query tiles (Lq <= 32768)
   // segment masks: the active query tiles in order (tile | 0x4000 if it
-  // needs no masking); query segments of MASK_SEG tiles
+  // needs no masking), FAR: the far ones of either side, then the near ones;
+  // query segments of MASK_SEG tiles
   __shared__ short qlist[SEGM ? MAXQT : 1];
-  __shared__ int qlen;
+  __shared__ int qlen[3];
   __shared__ __align__(16) int qsg[MASK == MASK_SEG ? 2 : 1][MASK == MASK_SEG ? BQ : 1];
   // dense pair masks: the current tile's mask, one bit per (query, key),
   // 16 keys a word (read once per tile with 16-byte loads)
   __shared__ uint16_t pmask[MASK == MASK_PAIR ? BQ : 1][MASK == MASK_PAIR ? BKW / 16 : 1];
 
   const int tid = threadIdx.x, lane = tid & 63;
-  const int w = tid >> 6, g = (tid & 63) >> 4, c16 = tid & 15;
+  // SCAL: the wave index is known to the compiler as uniform, and the copies'
+  // addresses are scalar bases and small per-lane offsets: 20 to 30 vector
+  // registers fewer, which the far loops (with 64-bit addresses a lane they
+  // spilled in the near loop: 339 against 276 us at B=4, L=2048, H=16) and the
+  // kernels with per-element mask tests need, for more scalar ones, which
+  // spill to vector lanes and cost the others up to 6% (dropout at B=12,
+  // L=512: 85.7 against 80.8 us).
+  constexpr bool SCAL = FAR || MASK == MASK_SEG || MASK == MASK_PAIR;
+  const int w = SCAL ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
+  const int g = (tid & 63) >> 4, c16 = tid & 15;
+  // one 16-byte LDS copy: byte offset off (lane part) from the uniform base
+  auto copy16 = [&](const void* base, unsigned off, void* lds_wave) {
+    if constexpr (SCAL) lds_dma16_s(base, off, lds_wave);
+    else lds_dma16((const char*)base + off, lds_wave);
+  };
+  auto copy16_nt = [&](const void* base, unsigned off, void* lds_wave) {
+    if constexpr (SCAL) lds_dma16_s_nt(base, off, lds_wave);
+    else lds_dma16_nt((const char*)base + off, lds_wave);
+  };
   const int Lq = p.Lq, Lk = p.Lk;
   const int NKT = p.LkP / BKW;
   // (b, h, kt), kt fastest; with an order (masks), item order[r / H] and
   // head r % H, heaviest first
   int kt, h, b;
   if (bp.korder) {
-    const int it = bp.korder[blockIdx.x / p.H];
+    const int it = __builtin_amdgcn_readfirstlane(bp.korder[blockIdx.x / p.H]);
     h = blockIdx.x % p.H, kt = it % NKT, b = it / NKT;
   } else {
     const int m = xcd_remap(blockIdx.x, gridDim.x);
@@ -118,6 +140,10 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
   const T* dobase = (const T*)bp.dout + (int64_t)b * bp.dos[0] + (int64_t)h * bp.dos[2];
   const BT* biasb = (const BT*)p.bias;
   const float* rib = bp.rowinfo + (int64_t)(b * p.H + h) * p.LqP * 2;
+  const int64_t riplane = (int64_t)p.B * p.H * p.LqP * 2;  // far blocks: the planes of the two sides follow
+  FarSpan fs{kNoFar, -kNoFar};
+  if constexpr (FAR) fs = far_span_of(bp);
+  auto is_far = [&](int qi) { return FAR && fs.far(qi / (128 / BQ) - kt); };
   const uint8_t* pkb = (MASK == MASK_PAIR) ? p.pk + (int64_t)b * p.pkb + (int64_t)h * p.pkh : nullptr;
   const SegView<MASK> sv(p, b);
   T* dsw = (T*)bp.ds + (int64_t)(b * p.H + h) * p.LqP * p.LkP + jw;  // dS column jw, row 0
@@ -139,28 +165,46 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
   // Segment masks: the query tiles that meet this key tile (ChunkRange),
   // listed by wave 0 (one chunk per lane); the others are neither computed
   // nor written.
+  // FAR: the far tiles past neg (queries before the keys) come first, then
+  // the far ones past pos, then the near ones: n1, n2 and nlist end the three
+  // parts, each a loop of its own.  The near loop's registers are all taken
+  // (a spill in it waits for the next tile's copies), and last it carries
+  // nothing of the others.
   bool any_key;
-  int nlist = nqt;
+  int nlist = nqt, n1 = 0, n2 = 0, qhi = 0;
   if constexpr (SEGM) {
     const ChunkRange kr = key_tile_range(bp.cinfo + (int64_t)b * nqt, kt, nqt);
     if (w == 0) {
       int n = 0;
-      for (int c0 = 0; c0 < nqt; c0 += 64) {
-        const int c = c0 + lane;
-        bool act = false, full = false;
-        if (c < nqt) {
-          const ChunkRange x = chunk_range(bp.cinfo + (int64_t)b * nqt, c);
-          act = x.meets(kr);
-          full = act && x.all && kr.all && x.lo == x.hi && kr.lo == kr.hi && x.lo == kr.lo;
+#pragma unroll 1
+      for (int part = 0; part < (FAR ? 3 : 1); ++part) {
+        for (int c0 = 0; c0 < nqt; c0 += 64) {
+          const int c = c0 + lane;
+          bool act = false, full = false;
+          if (c < nqt) {
+            const ChunkRange x = chunk_range(bp.cinfo + (int64_t)b * nqt, c);
+            act = x.meets(kr);
+            full = act && x.all && kr.all && x.lo == x.hi && kr.lo == kr.hi && x.lo == kr.lo;
+            if (FAR) act = act && part == (!is_far(c) ? 2 : c / (128 / BQ) < kt ? 0 : 1);
+          }
+          n = wave_append(act, (short)(c | (full ? 0x4000 : 0)), qlist, n);
         }
-        n = wave_append(act, (short)(c | (full ? 0x4000 : 0)), qlist, n);
+        if (lane == 0) qlen[part] = n;
       }
-      if (lane == 0) qlen = n;
     }
     __syncthreads();
-    nlist = __builtin_amdgcn_readfirstlane(qlen);
+    if constexpr (FAR) {
+      n1 = __builtin_amdgcn_readfirstlane(qlen[0]);
+      n2 = __builtin_amdgcn_readfirstlane(qlen[1]);
+    }
+    nlist = __builtin_amdgcn_readfirstlane(qlen[FAR ? 2 : 0]);
     any_key = nlist > 0;
   } else {
+    if constexpr (FAR) {
+      n1 = min(max((128 / BQ) * (kt + fs.neg + 1), 0), nqt);
+      qhi = min(max((128 / BQ) * (kt + fs.pos), 0), nqt);
+      n2 = n1 + nqt - qhi;
+    }
     any_key = __syncthreads_or(tid < BKW && j0 + tid < Lk);
   }
 
@@ -175,10 +219,10 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
     T* slot = Ring + (rb % NRB) * RBE;
 #pragma unroll
     for (int k = 0; k < (RCPB + 255) / 256; ++k) {
-      const int pc = 256 * k + w * 64 + lane;
       if (256 * k + w * 64 < RCPB) {
-        const int c = pc / D, d = pc % D;
-        lds_dma16(qrg + (int64_t)d * bp.TGP + 32 * rb + c * VEC, (char*)(slot + (256 * k + w * 64) * VEC));
+        const int c = (256 * k + w * 64) / D + lane / D, d = lane % D;  // D divides 64
+        copy16(qrg + 32 * rb, (unsigned)((d * bp.TGP + c * VEC) * (int)sizeof(T)),
+                    (char*)(slot + (256 * k + w * 64) * VEC));
       }
     }
   };
@@ -198,7 +242,9 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
   // (whose ring slot was last read two tiles earlier); with dropout, the
   // wave's keep words.
   int qseg_next = 0;  // MASK_SEG: query segment of lane (w = 1, lane < 32) in the next tile
-  auto issue = [&](int qi, bool ring, T* Qd, T* dOd, BT* Bd, float* Rd, uint32_t* Dd) {
+  // nring: the last blocks of the tile's qrgt window to copy; side: the far
+  // side of a far tile, or -1.
+  auto issue = [&](int qi, int nring, int side, T* Qd, T* dOd, BT* Bd, float* Rd, uint32_t* Dd) {
     const int i0 = qi * BQ;
     if (MASK == MASK_SEG && w == 1 && lane < BQ) qseg_next = (i0 + lane < Lq) ? sv(i0 + lane) : 0;
 #pragma unroll
@@ -211,22 +257,28 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
         lds_dma16(dobase + i * bp.dos[1] + lc * SQ::VEC, (char*)dOd + (w * QCW + 64 * k) * 16);
       }
     }
-    if (p.flags) {
+    if (p.flags && side < 0) {
       // two 2048-element blocks of the saved term: forward wave block
       // (i0 % 128) / 32 of forward key tiles j0/64 and j0/64 + 1
       constexpr int CPB = 2048 * (int)sizeof(BT) / 16;
 #pragma unroll
       for (int k = 0; k < BCW / 64; ++k) {
-        const int pc = w * BCW + 64 * k + lane;
-        const int kk = pc / CPB;
-        const BT* src = biasb + bias_tile_offset(b, h, p.H, i0 / 128, j0 / 64 + kk, p.LqP, p.LkP) +
+        const int pc = w * BCW + 64 * k;  // of lane 0; a wave's 64 chunks lie in one block
+        const BT* src = biasb + bias_tile_offset(b, h, p.H, i0 / 128, j0 / 64 + pc / CPB, p.LqP, p.LkP) +
                         ((i0 % 128) / 32) * 2048 + (pc % CPB) * (16 / (int)sizeof(BT));
-        lds_dma16_nt(src, (char*)Bd + (w * BCW + 64 * k) * 16);  // read once: non-temporal
+        copy16_nt(src, lane * 16, (char*)Bd + pc * 16);  // read once: non-temporal
       }
     }
-    if (w == 0 && lane < 2 * BQ * 4 / 16) lds_dma16(rib + 2 * i0 + 4 * lane, (char*)Rd);
-    if (p2c && ring) issue_ring(tw0 / 32 + qi + 4);
-    if (DROP && lane < 16) lds_dma16(dropw + (int64_t)qi * NKT64 * 64 + 4 * lane, (char*)(Dd + w * 64));
+    if (w == 0 && lane < 2 * BQ * 4 / 16)
+      copy16(rib + (FAR ? (1 + side) * riplane : 0) + 2 * i0, lane * 16, (char*)Rd);
+    if (p2c) {
+      if constexpr (FAR) {
+        for (int r = 5 - nring; r < 5; ++r) issue_ring(tw0 / 32 + qi + r);
+      } else {
+        if (nring) issue_ring(tw0 / 32 + qi + 4);
+      }
+    }
+    if (DROP && lane < 16) copy16(dropw + (int64_t)qi * NKT64 * 64, lane * 16, (char*)(Dd + w * 64));
   };
 
   // dS rows i of the wave's 32 keys: lane (g, c16) writes keys jw + 16 kk +
@@ -283,14 +335,30 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
     // The qrgt ring holds blocks [qi, qi + 4] of the window (relative to
     // tw0 / 32) while tile qi is computed; block qi + 5 lands in the sixth
     // slot meanwhile when the next tile is qi + 1.  The first window:
-    const int qfirst = SEGM ? (__builtin_amdgcn_readfirstlane(qlist[0]) & 0x3ff) : 0;
-    if (p2c)
-      for (int r = 0; r < 4; ++r) issue_ring(tw0 / 32 + qfirst + r);
-    issue(qfirst, true, Qs0, dOs0, Bs0, Rs0, Dk0);
+    auto entry = [&](int n) {
+      if constexpr (SEGM) return __builtin_amdgcn_readfirstlane(qlist[n]);
+      if constexpr (!FAR) return n;
+      return n < n1 ? n : n < n2 ? qhi + n - n1 : n1 + n - n2;
+    };
+    const int qfirst = entry(0) & 0x3ff;
+    if (!FAR || n2 == 0) {
+      if (p2c)
+        for (int r = 0; r < 4; ++r) issue_ring(tw0 / 32 + qfirst + r);
+      issue(qfirst, 1, -1, Qs0, dOs0, Bs0, Rs0, Dk0);
+    } else {
+      // the near part's first tile is to find its buffers first
+      if (n2 & 1) issue(qfirst, 0, n1 > 0 ? 1 : 0, Qs1, dOs1, Bs1, Rs1, Dk1);
+      else issue(qfirst, 0, n1 > 0 ? 1 : 0, Qs0, dOs0, Bs0, Rs0, Dk0);
+    }
     lds_dma_wait();
-    auto tile = [&](int n, const T* Q, const T* dO, const BT* Bt, const float* R, const uint32_t* Dw, T* nQ, T* ndO,
+    // Far tiles, one side at a time: the p2c term of the lane's keys and the
+    // column sums of dS (every row of the A operand is ones).
+    float fb[2] = {0.f, 0.f};
+    f32x4 fcs[2] = {zero4(), zero4()};
+    auto tile = [&](auto farkind, int n, const T* Q, const T* dO, const BT* Bt, const float* R, const uint32_t* Dw, T* nQ, T* ndO,
                     BT* nBt, float* nR, uint32_t* nDw) {
-      const int ent = SEGM ? __builtin_amdgcn_readfirstlane(qlist[n]) : n;
+      constexpr bool far = decltype(farkind)::value;
+      const int ent = entry(n);
       const int qi = ent & 0x3ff, i0 = qi * BQ;
       // This wave's copies of tile qi have landed: they were issued before
       // the previous tile's NST dS stores, its last vector-memory
@@ -298,7 +366,7 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
       vm_wait<NST>();
       if (MASK == MASK_SEG && w == 1 && lane < BQ) qsg[n & 1][lane] = qseg_next;
       __syncthreads();  // ... every wave's, and the previous tile is no longer read
-      if (SEGM && p2c && n > 0) {
+      if (SEGM && !far && p2c && n > n2) {
         // after skipped tiles: the blocks of this tile's window not in the
         // ring yet (their slots hold blocks no longer needed)
         const int pv = __builtin_amdgcn_readfirstlane(qlist[n - 1]) & 0x3ff;
@@ -309,8 +377,9 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
         }
       }
       if (n + 1 < nlist) {
-        const int qn = SEGM ? (__builtin_amdgcn_readfirstlane(qlist[n + 1]) & 0x3ff) : n + 1;
-        issue(qn, qn == qi + 1, nQ, ndO, nBt, nR, nDw);
+        const int qn = entry(n + 1) & 0x3ff;
+        if constexpr (far) issue(qn, n + 1 == n2 ? 5 : 0, n + 1 < n1 ? 1 : n + 1 < n2 ? 0 : -1, nQ, ndO, nBt, nR, nDw);
+        else issue(qn, qn == qi + 1, -1, nQ, ndO, nBt, nR, nDw);
       }
       // With segments, a tile whose queries all share the workgroup's single
       // key segment needs no masking beyond the dead-row test.  Other modes:
@@ -358,11 +427,13 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
         for (int s = 0; s < NS; ++s) qa[s] = SQ::row_frag(Q, 16 * ib + c16, s, g);
 #pragma unroll
         for (int jb = 0; jb < 2; ++jb) {
-          f32x4 acc = zero4();
+          // a far tile: the p2c term of the lane's keys starts the products
+          // (the c2p term is in the plane of rowinfo that the tile reads)
+          f32x4 acc = far ? f32x4{fb[jb], fb[jb], fb[jb], fb[jb]} : zero4();
 #pragma unroll
           for (int s = 0; s < NS; ++s)
             acc = M::mma(qa[s], kf[jb][s], acc);
-          {
+          if constexpr (!far) {
             // rows 16*ib + 4*g + e of key column 32w + 16*jb + c16 (forward
             // tile order); without relative terms the buffer holds zeros
             const int jl = WK * w + 16 * jb;
@@ -483,6 +554,12 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
         for (int jb = 0; jb < 2; ++jb) {
           pf[jb] = M::from_acc(pp[jb], s);
           df[jb] = M::from_acc(dsh[jb], s);
+          if constexpr (far) {
+            frag ones;
+#pragma unroll
+            for (int e = 0; e < FE; ++e) ones[e] = (T)1.0f;
+            fcs[jb] = M::mma(ones, df[jb], fcs[jb]);
+          }
         }
 #pragma unroll
         for (int db = 0; db < ND; ++db) {
@@ -497,7 +574,7 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
       }
 
       // ---- p2c: dK^T += qrgt[t0 + x]^T F[x] ------------------------------------------------
-      if (p2c) {
+      if (!far && p2c) {
         // qrgt column of x = 0 for this wave: i0 - jw - 31 + OFF (a multiple of 32)
         const int t0 = tw0 + i0 + BKW - WK - WK * w;
 #pragma unroll
@@ -522,9 +599,72 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
       }
       __builtin_amdgcn_s_setprio(0);
     };
-    for (int n = 0; n < nlist; n += 2) {
-      tile(n, Qs0, dOs0, Bs0, Rs0, Dk0, Qs1, dOs1, Bs1, Rs1, Dk1);
-      if (n + 1 < nlist) tile(n + 1, Qs1, dOs1, Bs1, Rs1, Dk1, Qs0, dOs0, Bs0, Rs0, Dk0);
+    if constexpr (FAR) {
+      float cs[2][2] = {{0.f, 0.f}, {0.f, 0.f}};  // column sums of dS per side
+      int n = 0;
+#pragma unroll
+      for (int side = 1; side >= 0; --side) {
+        const int hi = side ? n1 : n2;
+        if (n >= hi) continue;
+        const T* row = (const T*)p.qr + (int64_t)h * p.qrs[0] +
+                       (p2c ? (int64_t)offset_row(p.rel, far_offset(p, side), Lq, Lk, p.A, true) * p.qrs[1] : 0);
+        fcs[0] = fcs[1] = zero4();
+        if (p2c) {
+          f32x4 acc[2] = {zero4(), zero4()};
+#pragma unroll
+          for (int s = 0; s < NS; ++s) {
+            const frag af = M::load_contig(row, s, g);  // every row of the A operand
+#pragma unroll
+            for (int jb = 0; jb < 2; ++jb) acc[jb] = M::mma(af, kf[jb][s], acc[jb]);
+          }
+          fb[0] = acc[0][0], fb[1] = acc[1][0];
+        }
+#pragma unroll 1
+        for (; n < hi; ++n) {
+          // the parity picks the buffers at run time (the copies are issued
+          // from assembly, so the compiler waits for none of them)
+          const bool o = (n ^ n2) & 1;
+          tile(std::true_type{}, n, o ? Qs1 : Qs0, o ? dOs1 : dOs0, o ? Bs1 : Bs0, o ? Rs1 : Rs0, o ? Dk1 : Dk0,
+               o ? Qs0 : Qs1, o ? dOs0 : dOs1, o ? Bs0 : Bs1, o ? Rs0 : Rs1, o ? Dk0 : Dk1);
+        }
+        if (p2c) {
+          cs[side][0] = fcs[0][0], cs[side][1] = fcs[1][0];
+#pragma unroll
+          for (int db = 0; db < ND; ++db)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const float r = (float)row[16 * db + 4 * g + e];
+#pragma unroll
+              for (int jb = 0; jb < 2; ++jb) dka[db][jb][e] = __builtin_fmaf(r, cs[side][jb], dka[db][jb][e]);
+            }
+        }
+      }
+      if (p2c && n2 > 0) {
+        // and to the table gradient row: the waves' sums meet in their dS^T
+        // tiles' space, which the near tiles then need zeroed again
+        float* red = reinterpret_cast<float*>(stg);
+        static_assert(SW * sizeof(T) >= 2 * D * sizeof(float), "both sides' sums in a wave's tile");
+        wave_lds_sync();
+#pragma unroll
+        for (int side = 0; side < 2; ++side) far_row_sum<T, NS>(red + side * D, cs[side], kf, g, c16);
+        __syncthreads();
+        if (tid < 2 * D) {
+          const int side = tid / D, d = tid % D;
+          float v = 0.f;
+#pragma unroll
+          for (int u = 0; u < NW; ++u) v += reinterpret_cast<const float*>(Stg + u * SW)[side * D + d];
+          far_part(bp.farpart, p, h, 1, side, D)[((int64_t)b * NKT + kt) * D + d] = v;
+        }
+        __syncthreads();
+        for (int c = lane; c < 2 * D * (int)sizeof(float) / 16; c += 64)
+          reinterpret_cast<f32x4*>(stg)[c] = zero4();
+        wave_lds_sync();
+      }
+    }
+    using near_t = std::false_type;
+    for (int n = n2; n < nlist; n += 2) {
+      tile(near_t{}, n, Qs0, dOs0, Bs0, Rs0, Dk0, Qs1, dOs1, Bs1, Rs1, Dk1);
+      if (n + 1 < nlist) tile(near_t{}, n + 1, Qs1, dOs1, Bs1, Rs1, Dk1, Qs0, dOs0, Bs0, Rs0, Dk0);
     }
   }
 

@@ -46,8 +46,8 @@ struct DqLds {
 // Workgroup blk of nblk (the logical index, whose remainder mod 8 is the
 // XCD it runs on).  QC: the c2p part (the gradient of the c2p term's query
 // rows qc) is accumulated apart and written to dqc; dq then holds the
-// content part.
-template <typename T, int D, bool QC>
+// content part.  FAR: calls that can have far blocks (FarSpan).
+template <typename T, int D, bool QC, bool FAR>
 DSA_DEV void dq_body(const BwdParams& bp, int blk, int nblk, DqLds<T, D>& L) {
   using namespace dqcfg;
   using M = Mfma<T>;
@@ -94,6 +94,9 @@ DSA_DEV void dq_body(const BwdParams& bp, int blk, int nblk, DqLds<T, D>& L) {
   const T* kbase = (const T*)p.k + (int64_t)b * p.ks[0] + (int64_t)h * p.ks[2];
   const T* dsb = (const T*)bp.ds + ((int64_t)(b * p.H + h) * bp.f.LqP + i0) * bp.f.LkP;
   const T* krg = c2p ? (const T*)bp.krgt + (int64_t)h * D * bp.TGP : nullptr;
+  FarSpan fs{kNoFar, -kNoFar};
+  if constexpr (FAR) fs = far_span_of(bp);
+  auto is_far = [&](int kt) { return FAR && fs.far(qt - kt / (128 / BK)); };
 
   // zeros everywhere; the key columns are overwritten per tile
   {
@@ -146,7 +149,7 @@ DSA_DEV void dq_body(const BwdParams& bp, int blk, int nblk, DqLds<T, D>& L) {
       for (int e = 0; e < VEC; ++e) kr[k][e] = (T)0.0f;
       if (c < KV && j < p.Lk) kr[k] = *reinterpret_cast<const vecT*>(kbase + (int64_t)j * p.ks[1] + (c % (D / VEC)) * VEC);
     }
-    if (c2p) {
+    if (c2p && !is_far(kt)) {
       const int tw = i0 - j0 - 63 + bp.OFF;  // window column 0 (a multiple of 32)
 #pragma unroll
       for (int k = 0; k < GCH; ++k) {
@@ -185,7 +188,18 @@ DSA_DEV void dq_body(const BwdParams& bp, int blk, int nblk, DqLds<T, D>& L) {
     for (int t = tid; t < nkt; t += 256) klist[t] = (short)(t | (0xf << 10));
     __syncthreads();
   }
+  // Far tiles: row sums of dS (every row of the A operand is ones, so each
+  // lane holds its queries' sums), one side at a time (tiles come in key
+  // order: the far side past pos, the near tiles, the far side past neg).
+  f32x4 frs[2] = {zero4(), zero4()};
+  int fside = -1;
+  frag ones;
+#pragma unroll
+  for (int e = 0; e < FE; ++e) ones[e] = (T)1.0f;
+  float rs[2][2] = {{0.f, 0.f}, {0.f, 0.f}};  // per side
   auto tile = [&](int n, Regs& r) {
+    const int kt = klist[n] & 1023;
+    const bool far = is_far(kt);
     __syncthreads();  // previous tile's readers are done
 #pragma unroll
     for (int k = 0; k < SCH; ++k) {
@@ -197,7 +211,7 @@ DSA_DEV void dq_body(const BwdParams& bp, int blk, int nblk, DqLds<T, D>& L) {
       const int c = tid + 256 * k;
       if (c < KV) *reinterpret_cast<vecT*>(Ks + (c / (D / VEC)) * KSTR + (c % (D / VEC)) * VEC) = r.k[k];
     }
-    if (c2p) {
+    if (c2p && !far) {
 #pragma unroll
       for (int k = 0; k < GCH; ++k) {
         const int c = tid + 256 * k;
@@ -207,6 +221,16 @@ DSA_DEV void dq_body(const BwdParams& bp, int blk, int nblk, DqLds<T, D>& L) {
     __syncthreads();
     if (n + 2 < nkt) fetch(klist[n + 2], r);
 
+    if (FAR && far && c2p) {
+      const int side = fs.side(qt - kt / (128 / BK));
+      if (side != fside) {
+        if (fside == 0) {
+          rs[0][0] = frs[0][0], rs[0][1] = frs[1][0];
+          frs[0] = frs[1] = zero4();
+        }
+        fside = side;
+      }
+    }
     // ---- dQ^T += K^T dS^T: B = dS row i, keys KSTEP*s + FE*g + [0, FE) -----------------------
 #pragma unroll
     for (int s = 0; s < BK / M::KSTEP; ++s) {
@@ -214,6 +238,9 @@ DSA_DEV void dq_body(const BwdParams& bp, int blk, int nblk, DqLds<T, D>& L) {
 #pragma unroll
       for (int ib = 0; ib < 2; ++ib)
         bfr[ib] = *reinterpret_cast<const frag*>(Ss + (WQ * w + 16 * ib + c16) * SSTR + ZC + M::KSTEP * s + FE * g);
+#pragma unroll
+      for (int ib = 0; ib < 2; ++ib)
+        if (FAR && far) frs[ib] = M::mma(ones, bfr[ib], frs[ib]);
 #pragma unroll
       for (int db = 0; db < ND; ++db) {
         const frag af = tr_contig<T>(Ks, KSTR, s * M::KSTEP, 16 * db, g, c16);
@@ -223,7 +250,7 @@ DSA_DEV void dq_body(const BwdParams& bp, int blk, int nblk, DqLds<T, D>& L) {
     }
 
     // ---- c2p: dQ^T += krgt[t0 + x]^T E[x] ---------------------------------------------------
-    if (c2p) {
+    if (c2p && !far) {
       // krgt column of x = 0 for this wave: iw - j0 - 63 + OFF, i.e. window
       // column 32w.  Element e of the fragment whose first offset is
       // xb = KSTEP*s + FE*g holds offset x = xb + FE - 1 - e, i.e. key
@@ -256,6 +283,52 @@ DSA_DEV void dq_body(const BwdParams& bp, int blk, int nblk, DqLds<T, D>& L) {
     tile(n, ra);
     if (n + 1 < nkt) tile(n + 1, rb);
   }
+  if (FAR && fside >= 0) {
+    // the row sums of both sides to dQ and, beside a table kernel that leaves
+    // the far blocks out, to the table gradient rows
+    if (fside == 0) rs[0][0] = frs[0][0], rs[0][1] = frs[1][0];
+    else rs[1][0] = frs[0][0], rs[1][1] = frs[1][0];
+    constexpr int NSD = D / M::KSTEP;
+    const T* qb = QC ? (const T*)p.qc + (int64_t)b * p.qcs[0] + (int64_t)h * p.qcs[2]
+                     : (const T*)p.q + (int64_t)b * p.qs[0] + (int64_t)h * p.qs[2];
+    const int64_t qrs = QC ? p.qcs[1] : p.qs[1];
+    frag qv[2][NSD];
+#pragma unroll
+    for (int ib = 0; ib < 2; ++ib)
+#pragma unroll
+      for (int s = 0; s < NSD; ++s) {
+        const int i = iw + 16 * ib + c16;
+        qv[ib][s] = i < p.Lq ? M::load_contig(qb + (int64_t)i * qrs, s, g) : M::zero();
+      }
+    float* red = reinterpret_cast<float*>(Ks);
+    static_assert(BK * KSTR * sizeof(T) >= NW * 2 * D * sizeof(float), "the waves' sums in the K tile");
+    __syncthreads();  // the last tile is no longer read
+#pragma unroll
+    for (int side = 0; side < 2; ++side) {
+      const T* row = (const T*)p.kr + (int64_t)h * p.krs[0] +
+                     (int64_t)offset_row(p.rel, far_offset(p, side), p.Lq, p.Lk, p.A, false) * p.krs[1];
+#pragma unroll
+      for (int db = 0; db < ND; ++db)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float x = (float)row[16 * db + 4 * g + e];
+#pragma unroll
+          for (int ib = 0; ib < 2; ++ib) {
+            f32x4& a = QC ? dqca[QC ? db : 0][ib] : dqa[db][ib];
+            a[e] = __builtin_fmaf(x, rs[side][ib], a[e]);
+          }
+        }
+      far_row_sum<T, NSD>(red + (w * 2 + side) * D, rs[side], qv, g, c16);
+    }
+    __syncthreads();
+    if (bp.fardq && tid < 2 * D) {
+      const int side = tid / D, d = tid % D;
+      float v = 0.f;
+#pragma unroll
+      for (int u = 0; u < NW; ++u) v += red[(u * 2 + side) * D + d];
+      far_part(bp.farpart, p, h, 0, side, D)[((int64_t)b * NQT + qt) * D + d] = v;
+    }
+  }
 
   // ---- dQ ---------------------------------------------------------------------------------
   T* dqbase = (T*)bp.dq + (int64_t)b * bp.dqs[0] + (int64_t)h * bp.dqs[2];
@@ -287,10 +360,10 @@ DSA_DEV void dq_body(const BwdParams& bp, int blk, int nblk, DqLds<T, D>& L) {
   }
 }
 
-template <typename T, int D, bool QC = false>
+template <typename T, int D, bool QC, bool FAR>
 __global__ __launch_bounds__(256, 2) void dsa_bwd_dq_kernel(BwdParams bp) {
   __shared__ DqLds<T, D> L;
-  dq_body<T, D, QC>(bp, blockIdx.x, gridDim.x, L);
+  dq_body<T, D, QC, FAR>(bp, blockIdx.x, gridDim.x, L);
 }
 
 }  // namespace dsa

@@ -24,7 +24,7 @@
 
 namespace dsa {
 
-template <typename T, int D, bool LISTED, bool QC>
+template <typename T, int D, bool LISTED, bool QC, bool FAR>
 __global__ __launch_bounds__(256, 2) void dsa_bwd_dqtab_kernel(BwdParams bp, BwdParams tp, int ntab, int nt8, int ndq) {
   __shared__ union Lds {
     DqLds<T, D> dq;
@@ -32,9 +32,9 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dqtab_kernel(BwdParams bp, Bwd
   } L;
   const int n = blockIdx.x;
   if (n < nt8) {
-    if (n < ntab) table_body<T, D, LISTED>(tp, n, ntab, L.tab);
+    if (n < ntab) table_body<T, D, LISTED, FAR>(tp, n, ntab, L.tab);
   } else {
-    dq_body<T, D, QC>(bp, n - nt8, ndq, L.dq);
+    dq_body<T, D, QC, FAR>(bp, n - nt8, ndq, L.dq);
   }
 }
 

@@ -114,7 +114,7 @@ struct TabLds {
 // XCD it runs on).  LISTED: a key-padding or segment mask is given
 // (bp.cinfo): items without an active part are skipped and partials carry
 // flags.
-template <typename T, int D, bool LISTED>
+template <typename T, int D, bool LISTED, bool FAR>
 DSA_DEV void table_body(const BwdParams& bp, int blk, int nblk, TabLds<T, D>& L) {
   using namespace tbcfg;
   using M = Mfma<T>;
@@ -171,7 +171,14 @@ DSA_DEV void table_body(const BwdParams& bp, int blk, int nblk, TabLds<T, D>& L)
   block_items(dblk, p.LkP, p.Lq, p.Lk, p2c, &rstart, &nch);
   // The block's items of one kind, (batch, 32-row chunk) batch-major, are
   // split into NPG contiguous ranges; partial group pg takes range pg.
-  const int total = active ? p.B * nch : 0;
+  // Far blocks (FarSpan) are left out: their pairs' sums come from the dkdv
+  // kernel (Gp) and the dq kernel (Gc, when it runs beside this one).  The
+  // offset block holds pairs of the block diagonals dd and dd + 1.
+  const bool exf = FAR && (p2c || bp.fardq);
+  FarSpan fs{kNoFar, -kNoFar};
+  if constexpr (FAR) fs = far_span_of(bp);
+  const int dd0 = d0 / DBW;  // exact: d0 is a multiple of DBW
+  const int total = active && !(exf && (dd0 >= fs.pos || dd0 + 1 <= fs.neg)) ? p.B * nch : 0;
   const int per = (total + bp.NPG - 1) / bp.NPG;
   const int it_lo = min(total, pg * per), nitems = min(total, it_lo + per) - it_lo;
   // A block whose offsets all lie in the offset range of one table row of
@@ -234,24 +241,28 @@ DSA_DEV void table_body(const BwdParams& bp, int blk, int nblk, TabLds<T, D>& L)
     // item without active parts is skipped.
     const int nqc = p.LqP / 32, nkt128 = p.LkP / 128;
     auto item_mask = [&](int b, int r0) -> int {
-      if (!LISTED) return 0xff;
-      const int4* ci = bp.cinfo + (int64_t)b * nqc;
+      if (!LISTED && !FAR) return 0xff;
+      const int4* ci = LISTED ? bp.cinfo + (int64_t)b * nqc : nullptr;
       int m = 0;
       if constexpr (!P) {
         const int jc0 = r0 - d0 - DBW, kA = (jc0 >= 0 ? jc0 : jc0 - 127) / 128;
-        const ChunkRange qc = chunk_range(ci, r0 / 32);
+        ChunkRange qc{0, 0, 0};
+        if constexpr (LISTED) qc = chunk_range(ci, r0 / 32);
 #pragma unroll
         for (int u = 0; u < 3; ++u) {
           const int k = kA + u;
-          if (k >= 0 && k < nkt128 && 128 * k < jc0 + DBW + CH && qc.meets(key_tile_range(ci, k, nqc))) m |= 1 << u;
+          if (k < 0 || k >= nkt128 || 128 * k >= jc0 + DBW + CH || (exf && fs.far(r0 / 128 - k))) continue;
+          if (!LISTED || qc.meets(key_tile_range(ci, k, nqc))) m |= 1 << u;
         }
       } else {
-        const ChunkRange kr = key_tile_range(ci, r0 / 128, nqc);
+        ChunkRange kr{0, 0, 0};
+        if constexpr (LISTED) kr = key_tile_range(ci, r0 / 128, nqc);
         const int cA = (r0 + d0) / 32;  // r0 + d0 is a multiple of 32 (may be negative)
 #pragma unroll
         for (int u = 0; u < PR / 32; ++u) {
           const int c = cA + u;
-          if (c >= 0 && c < nqc && chunk_range(ci, c).meets(kr)) m |= 1 << u;
+          if (c < 0 || c >= nqc || (exf && fs.far(c / 4 - r0 / 128))) continue;
+          if (!LISTED || chunk_range(ci, c).meets(kr)) m |= 1 << u;
         }
       }
       return m;
@@ -340,7 +351,7 @@ DSA_DEV void table_body(const BwdParams& bp, int blk, int nblk, TabLds<T, D>& L)
     const int ncand = nitems > sub ? (nitems - sub + 1) / 2 : 0;
     for (int base = 0; base < ncand; base += 64) {
       int cnt = min(64, ncand - base);
-      if (LISTED) {
+      if (LISTED || exf) {
         const int c = base + lane, it = sub + 2 * c;
         int m = 0;
         if (c < ncand) {
@@ -352,7 +363,7 @@ DSA_DEV void table_body(const BwdParams& bp, int blk, int nblk, TabLds<T, D>& L)
       }
       nact += cnt;
       auto entry = [&](int n) {
-        return LISTED ? __builtin_amdgcn_readfirstlane(lst[n]) : ((sub + 2 * (base + n)) << 8) | 0xff;
+        return (LISTED || exf) ? __builtin_amdgcn_readfirstlane(lst[n]) : ((sub + 2 * (base + n)) << 8) | 0xff;
       };
       if constexpr (PREFETCH) {
         if (cnt > 0) fetch(entry(0));
@@ -449,10 +460,10 @@ DSA_DEV void table_body(const BwdParams& bp, int blk, int nblk, TabLds<T, D>& L)
   }
 }
 
-template <typename T, int D, bool LISTED>
+template <typename T, int D, bool LISTED, bool FAR>
 __global__ __launch_bounds__(256, 2) void dsa_bwd_table_kernel(BwdParams bp) {
   __shared__ TabLds<T, D> L;
-  table_body<T, D, LISTED>(bp, blockIdx.x, gridDim.x, L);
+  table_body<T, D, LISTED, FAR>(bp, blockIdx.x, gridDim.x, L);
 }
 
 // tab[h][r][:] (+)= s * sum over offsets d with row(d) = r of the block
@@ -505,6 +516,22 @@ __global__ __launch_bounds__(256) void dsa_bwd_fold_kernel(BwdParams bp) {
     for (int u = 0; u < 4; ++u) a4[u] += pair_val(it + u * NP);
   }
   for (; it < npairs; it += NP) a4[0] += pair_val(it);
+  if (p.far) {
+    // the far blocks' partials of the rows they read
+    const int n = p.B * (t ? p.LkP : p.LqP) / 128;
+#pragma unroll
+    for (int side = 0; side < 2; ++side) {
+      const int e = far_offset(p, side);
+      if (e < beg || e >= end) continue;
+      const float* fp = far_part(bp.farpart, p, h, t, side, D) + 4 * c4;
+      int u = part;
+      for (; u + 3 * NP < n; u += 4 * NP) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) a4[k] += *reinterpret_cast<const f32x4*>(fp + (int64_t)(u + k * NP) * D);
+      }
+      for (; u < n; u += NP) a4[0] += *reinterpret_cast<const f32x4*>(fp + (int64_t)u * D);
+    }
+  }
   f32x4 acc = (a4[0] + a4[1]) + (a4[2] + a4[3]);
 #pragma unroll
   for (int m = Q4; m < 64; m <<= 1)

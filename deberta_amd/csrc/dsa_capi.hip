@@ -16,14 +16,7 @@
 #include "../../include/dsa.h"
 #include "../../include/dsa_block.h"
 #include "dsa_bias.h"
-#include "dsa_bwd.h"
-#include "dsa_bwd_dkdv.h"
-#include "dsa_bwd_dq.h"
-#include "dsa_bwd_dqtab.h"
-#include "dsa_bwd_table.h"
-#include "dsa_dropout.h"
-#include "dsa_order.h"
-#include "dsa_fwd.h"
+#include "dsa_launch.h"
 #include "dsa_rows.h"
 
 // Library-owned scratch of dsa_fwd_static: the launch order's cost and
@@ -35,28 +28,23 @@
 constexpr size_t kStaticScratchBytes = 512 * 1024;
 static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
 
+using namespace dsa::host;
+
+// Compiled in translation units of their own (dsa_inst.hip).
+namespace dsa {
+namespace host {
+#define DSA_EXTERN(T, D)                                                      \
+  extern template int fwd_mask<T, D>(const FwdParams&, int, hipStream_t); \
+  extern template int launch_bwd<T, D>(const dsa_bwd_args*, const WsLayout&, int, hipStream_t);
+DSA_EXTERN(bf16, 64)
+DSA_EXTERN(bf16, 32)
+DSA_EXTERN(float, 64)
+DSA_EXTERN(float, 32)
+#undef DSA_EXTERN
+}  // namespace host
+}  // namespace dsa
+
 namespace {
-
-thread_local std::string g_err;
-
-int fail(const char* fmt, ...) __attribute__((format(printf, 1, 2)));
-int fail(const char* fmt, ...) {
-  char buf[512];
-  va_list ap;
-  va_start(ap, fmt);
-  vsnprintf(buf, sizeof(buf), fmt, ap);
-  va_end(ap);
-  g_err = buf;
-  return 1;
-}
-
-bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
-
-size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
-
-int round_up(int x, int a) { return (x + a - 1) / a * a; }
-
-int elem_bytes(int dtype) { return dtype == DSA_BF16 ? 2 : 4; }
 
 // The c2p term's query rows (qc, optional): c2p on, aligned like q.
 int check_qc(const dsa_fwd_args* a) {
@@ -126,410 +114,6 @@ int check_fwd(const dsa_fwd_args* a) {
   if ((a->flags & DSA_P2C) && (!aligned16(a->qr) || a->qr_strides[0] % vec || a->qr_strides[1] % vec))
     return fail("dsa: qr must be 16-byte aligned with strides that are multiples of %d", vec);
   return check_qc(a);
-}
-
-dsa::FwdParams to_params(const dsa_fwd_args* a) {
-  dsa::FwdParams p;
-  p.q = a->q;
-  p.k = a->k;
-  p.v = a->v;
-  p.kr = a->kr;
-  p.qr = a->qr;
-  p.rel = a->rel_table;
-  p.kk = a->key_keep;
-  p.pk = a->pair_keep;
-  p.out = a->out;
-  p.lse = a->lse;
-  p.bias = a->bias;
-  for (int s = 0; s < 3; ++s) {
-    p.qs[s] = a->q_strides[s];
-    p.ks[s] = a->k_strides[s];
-    p.vs[s] = a->v_strides[s];
-    p.os[s] = a->o_strides[s];
-  }
-  for (int s = 0; s < 2; ++s) {
-    p.krs[s] = a->kr_strides[s];
-    p.qrs[s] = a->qr_strides[s];
-  }
-  p.krk = p.qrk = 64 / elem_bytes(a->dtype);  // rows contiguous: k-steps adjacent
-  p.kkb = a->key_keep_stride_b;
-  p.pkb = a->pair_keep_strides[0];
-  p.pkq = a->pair_keep_strides[1];
-  p.pkh = a->pair_keep ? a->pair_keep_stride_h : 0;
-  p.seg = a->seg;
-  p.segb = a->seg_stride_b;
-  p.order = nullptr;
-  p.qc = a->qc;
-  for (int s = 0; s < 3; ++s) p.qcs[s] = a->qc ? a->qc_strides[s] : 0;
-  p.B = a->B;
-  p.H = a->H;
-  p.Lq = a->Lq;
-  p.Lk = a->Lk;
-  p.A = a->flags ? a->att_span : 1;
-  p.flags = a->flags;
-  p.LqP = round_up(a->Lq, 128);
-  p.LkP = round_up(a->Lk, 128);
-  p.scale = a->scale;
-  p.drop = nullptr;  // set where the keep bits are generated
-  p.drop_scale = 1.f;
-  p.olo = a->dtype == DSA_BF16 ? a->out_lo : nullptr;
-  return p;
-}
-
-int mask_mode(const dsa_fwd_args* a) {
-  return a->pair_keep ? dsa::MASK_PAIR : a->key_keep ? dsa::MASK_KEY : a->seg ? dsa::MASK_SEG : dsa::MASK_NONE;
-}
-
-int launch_check(const char* what) {
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return fail("dsa: %s launch failed: %s", what, hipGetErrorString(e));
-  return 0;
-}
-
-// Heaviest-first order (dsa_order.h) of B * ntiles items: cost and order
-// arrays of that many ints each.  Used under key_keep / seg masks only, and
-// for at most this many items (one block sorts them).
-constexpr int64_t kMaxOrderItems = 65536;
-
-size_t order_bytes(const dsa_fwd_args* a, int ntiles) {
-  const int64_t n = (int64_t)a->B * ntiles;
-  if (!(a->key_keep || a->seg) || n > kMaxOrderItems) return 0;
-  return align_up((size_t)2 * n * sizeof(int), 256);
-}
-
-// Up to two heaviest-first orders (dsa_order.h): each job a buffer of cost
-// then order (B * ntiles ints each), its tiles per row and its cost kind.
-// fill_orders sets up the launches' parameters and the number of cost
-// blocks (batch row fastest, then the tile group, then the job);
-// launch_orders runs the cost and sort kernels, a caller that runs the cost
-// blocks inside another launch only the sort (launch_order_sort).
-int fill_orders(const dsa::FwdParams& p, int njobs, int* const* bufs, const int* ntiles, const bool* fwd,
-                dsa::OrderParams2& op, int& ny) {
-  op.f = p;
-  op.njobs = njobs;
-  int maxt = 0;
-  for (int j = 0; j < 2; ++j) {
-    const int jj = j < njobs ? j : 0;
-    op.job[j].cost = bufs[jj];
-    op.job[j].order = bufs[jj] + (int64_t)p.B * ntiles[jj];
-    op.job[j].ntiles = ntiles[jj];
-    op.job[j].fwd = fwd[jj] ? 1 : 0;
-    maxt = std::max(maxt, ntiles[jj]);
-  }
-  ny = (maxt + dsa::ORDER_TPB - 1) / dsa::ORDER_TPB;
-  return p.B * ny * njobs;
-}
-
-int launch_order_sort(const dsa::OrderParams2& op, hipStream_t st) {
-  hipLaunchKernelGGL(dsa::dsa_order_sort_kernel, dim3(1), dim3(1024), 0, st, op);
-  return launch_check("dsa_order_sort_kernel");
-}
-
-int launch_orders(const dsa::FwdParams& p, int njobs, int* const* bufs, const int* ntiles, const bool* fwd,
-                  hipStream_t st) {
-  dsa::OrderParams2 op;
-  int ny = 0;
-  fill_orders(p, njobs, bufs, ntiles, fwd, op, ny);
-  const dim3 grid((unsigned)p.B, (unsigned)ny, (unsigned)njobs);
-  hipLaunchKernelGGL(dsa::dsa_order_cost_kernel, grid, dim3(256), 0, st, op);
-  if (launch_check("dsa_order_cost_kernel")) return 1;
-  return launch_order_sort(op, st);
-}
-
-int fwd_tiles(const dsa_fwd_args* a) { return (a->Lq + dsa::dcfg::BQ - 1) / dsa::dcfg::BQ; }
-
-// ---- attention dropout (dsa_dropout.h) ----
-// Bytes of the keep bits (0 without dropout).
-size_t drop_bits_bytes(const dsa_fwd_args* a) {
-  if (!a->dropout_threshold) return 0;
-  return dsa::dropout_bits_bytes(a->B, a->H, round_up(a->Lq, 128), round_up(a->Lk, 128));
-}
-// Bytes of them in the forward's or the backward's workspace: none when the
-// caller keeps them (dropout_bits).
-size_t drop_bytes(const dsa_fwd_args* a) {
-  return a->dropout_bits ? 0 : align_up(drop_bits_bytes(a), 256);
-}
-float drop_scale(const dsa_fwd_args* a) { return 65536.f / (float)(65536u - a->dropout_threshold); }
-
-// Generates the call's keep bits into `bits` and points the kernels'
-// parameters at them.
-int launch_dropout_bits(const dsa_fwd_args* a, uint32_t* bits, dsa::FwdParams& p, hipStream_t st) {
-  dsa::DropParams d;
-  d.bits = bits;
-  d.B = a->B;
-  d.H = a->H;
-  d.NQB = round_up(a->Lq, 128) / 32;
-  d.NKT = round_up(a->Lk, 128) / 64;
-  d.t = a->dropout_threshold;
-  d.k0 = (uint32_t)(a->dropout_seed & 0xffffffffu);
-  d.k1 = (uint32_t)(a->dropout_seed >> 32);
-  const dim3 grid((unsigned)((d.NKT + 3) / 4 * d.NQB), (unsigned)d.H, (unsigned)d.B);
-  hipLaunchKernelGGL(dsa::dsa_dropout_bits_kernel, grid, dim3(256), 0, st, d);
-  if (launch_check("dsa_dropout_bits_kernel")) return 1;
-  p.drop = bits;
-  p.drop_scale = drop_scale(a);
-  return 0;
-}
-
-
-template <typename T, int D, int MASK, bool DROP>
-int launch_fwd(const dsa::FwdParams& p, hipStream_t st) {
-  dim3 grid((unsigned)((p.Lq + dsa::dcfg::BQ - 1) / dsa::dcfg::BQ * p.H * p.B));
-  if (p.qc)
-    hipLaunchKernelGGL((dsa::dsa_fwd_kernel<T, D, MASK, true, DROP>), grid, dim3(256), 0, st, p);
-  else
-    hipLaunchKernelGGL((dsa::dsa_fwd_kernel<T, D, MASK, false, DROP>), grid, dim3(256), 0, st, p);
-  return launch_check("dsa_fwd_kernel");
-}
-
-template <typename T, int D, int MASK>
-int launch_fwd(const dsa::FwdParams& p, hipStream_t st) {
-  return p.drop ? launch_fwd<T, D, MASK, true>(p, st) : launch_fwd<T, D, MASK, false>(p, st);
-}
-
-template <typename T, int D>
-int fwd_mask(const dsa::FwdParams& p, int mode, hipStream_t st) {
-  switch (mode) {
-    case dsa::MASK_KEY: return launch_fwd<T, D, dsa::MASK_KEY>(p, st);
-    case dsa::MASK_PAIR: return launch_fwd<T, D, dsa::MASK_PAIR>(p, st);
-    case dsa::MASK_SEG: return launch_fwd<T, D, dsa::MASK_SEG>(p, st);
-    default: return launch_fwd<T, D, dsa::MASK_NONE>(p, st);
-  }
-}
-
-// Compute units of the current device (queried once per device).
-int device_cus() {
-  static std::atomic<int> cached[16] = {};
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return 256;
-  if (dev >= 0 && dev < 16 && (cus = cached[dev].load(std::memory_order_relaxed)) > 0) return cus;
-  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) return 256;
-  if (dev >= 0 && dev < 16) cached[dev].store(cus, std::memory_order_relaxed);
-  return cus;
-}
-
-// Workspace of the backward (offsets 256-byte aligned) and the padded
-// extents the kernels share.
-struct WsLayout {
-  int LqP, LkP, TGP, OFF, NDB, NPG;
-  size_t rowinfo, krgt, qrgt, ds, gpart, seg, cinfo, korder, qorder, drop, total;
-};
-
-WsLayout ws_layout(const dsa_bwd_args* a) {
-  const dsa_fwd_args& f = a->fwd;
-  const size_t es = (size_t)elem_bytes(f.dtype);
-  WsLayout w;
-  w.LqP = round_up(f.Lq, 128);
-  w.LkP = round_up(f.Lk, 128);
-  w.OFF = w.LkP - 1;            // offset origin: t = d + OFF, 32-aligned tile starts
-  w.TGP = w.LqP + w.LkP;        // offsets [-(LkP - 1), LqP] of every band window
-  w.NDB = (w.LqP + w.LkP) / dsa::tbcfg::DBW;
-  // Partial groups of the table kernel (ranges of an offset block's items
-  // of one kind; a central block has about B * L / 32): about one and a
-  // half workgroups per CU, whose fp32 atomics into the block accumulators
-  // stay few and which leave room for dq beside them (B=32, L=512, the two
-  // in one launch: backward 312 us with one workgroup per CU, 305 with one
-  // and a half, 307 with two, 319 with three).  Long sequences and masks concentrate the work in the
-  // central blocks, whose workgroups then bound the launch: those get at
-  // most 64 items of a kind each.
-  const int per = f.H * w.NDB;
-  const int64_t items = (int64_t)f.B * ((w.LqP > w.LkP ? w.LqP : w.LkP) / 32);
-  int64_t groups = (3 * device_cus() / 2 + per - 1) / per;
-  if (w.NDB > 16 || f.key_keep || f.seg) groups = std::max<int64_t>(groups, (items + 63) / 64);
-  w.NPG = (int)std::min<int64_t>(std::max<int64_t>(groups, 1), items);
-  size_t off = 0;
-  w.rowinfo = off;
-  off = align_up(off + (size_t)f.B * f.H * w.LqP * 2 * sizeof(float), 256);
-  w.krgt = off;
-  if (f.flags & DSA_C2P) off = align_up(off + (size_t)f.H * f.D * w.TGP * es, 256);
-  w.qrgt = off;
-  if (f.flags & DSA_P2C) off = align_up(off + (size_t)f.H * f.D * w.TGP * es, 256);
-  w.ds = off;
-  off = align_up(off + (size_t)f.B * f.H * w.LkP * w.LqP * es, 256);
-  w.gpart = off;
-  if (f.flags) off = align_up(off + (size_t)f.H * w.NDB * 2 * dsa::tbcfg::DBW * f.D * sizeof(float), 256);
-  w.seg = off;
-  if (f.flags) off = align_up(off + (size_t)2 * 2 * (2 * f.att_span) * sizeof(int), 256);
-  w.cinfo = off;
-  if (f.key_keep || f.seg) off = align_up(off + (size_t)f.B * (w.LqP / 32) * 4 * sizeof(int), 256);
-  w.korder = off;  // dkdv launch order (cost, order), under key_keep / seg
-  off += order_bytes(&f, w.LkP / dsa::kvcfg::BKW);
-  w.qorder = off;  // dq launch order
-  off += order_bytes(&f, w.LqP / dsa::dqcfg::BQ);
-  w.drop = off;  // attention dropout's keep bits, regenerated by PREP
-  off += drop_bytes(&f);
-  w.total = off;
-  return w;
-}
-
-template <typename T, int D, bool DROP>
-int launch_dkdv(const dsa::BwdParams& bp, const WsLayout& ws, int mode, hipStream_t st) {
-  const dsa::FwdParams& f = bp.f;
-  dim3 grid((unsigned)(ws.LkP / dsa::kvcfg::BKW * f.H * f.B));
-  switch (mode) {
-    case dsa::MASK_KEY:
-      hipLaunchKernelGGL((dsa::dsa_bwd_dkdv_kernel<T, D, dsa::MASK_KEY, DROP>), grid, dim3(256), 0, st, bp);
-      break;
-    case dsa::MASK_PAIR:
-      hipLaunchKernelGGL((dsa::dsa_bwd_dkdv_kernel<T, D, dsa::MASK_PAIR, DROP>), grid, dim3(256), 0, st, bp);
-      break;
-    case dsa::MASK_SEG:
-      hipLaunchKernelGGL((dsa::dsa_bwd_dkdv_kernel<T, D, dsa::MASK_SEG, DROP>), grid, dim3(256), 0, st, bp);
-      break;
-    default:
-      hipLaunchKernelGGL((dsa::dsa_bwd_dkdv_kernel<T, D, dsa::MASK_NONE, DROP>), grid, dim3(256), 0, st, bp);
-  }
-  return launch_check("dsa_bwd_dkdv_kernel");
-}
-
-template <typename T, int D>
-int launch_bwd(const dsa_bwd_args* a, const WsLayout& ws, int mode, hipStream_t st) {
-  const dsa_fwd_args& f = a->fwd;
-  dsa::BwdParams bp;
-  bp.f = to_params(&f);
-  bp.dout = a->dout;
-  for (int s = 0; s < 3; ++s) {
-    bp.dos[s] = a->do_strides[s];
-    bp.dqs[s] = a->dq_strides[s];
-    bp.dks[s] = a->dk_strides[s];
-    bp.dvs[s] = a->dv_strides[s];
-  }
-  bp.dq = a->dq;
-  bp.dk = a->dk;
-  bp.dv = a->dv;
-  bp.dqc = f.qc ? a->dqc : nullptr;
-  for (int s = 0; s < 3; ++s) bp.dqcs[s] = f.qc ? a->dqc_strides[s] : 0;
-  bp.dkr = a->dkr;
-  bp.dqr = a->dqr;
-  bp.dtab_bf16 = a->dtab_dtype == DSA_BF16;
-  bp.dtab_overwrite = a->dtab_overwrite != 0;
-  char* base = static_cast<char*>(a->workspace);
-  bp.rowinfo = reinterpret_cast<float*>(base + ws.rowinfo);
-  bp.krgt = base + ws.krgt;
-  bp.qrgt = base + ws.qrgt;
-  bp.ds = base + ws.ds;
-  bp.gpart = reinterpret_cast<float*>(base + ws.gpart);
-  bp.rowseg = reinterpret_cast<int*>(base + ws.seg);
-  bp.cinfo = (f.key_keep || f.seg) ? reinterpret_cast<int4*>(base + ws.cinfo) : nullptr;
-  const int nkt = ws.LkP / dsa::kvcfg::BKW;
-  int* kbuf = order_bytes(&f, nkt) ? reinterpret_cast<int*>(base + ws.korder) : nullptr;
-  bp.korder = kbuf ? kbuf + (int64_t)f.B * nkt : nullptr;
-  const int nqt = ws.LqP / dsa::dqcfg::BQ;
-  int* qbuf = order_bytes(&f, nqt) ? reinterpret_cast<int*>(base + ws.qorder) : nullptr;
-  bp.qorder = qbuf ? qbuf + (int64_t)f.B * nqt : nullptr;
-  bp.TGP = ws.TGP;
-  bp.OFF = ws.OFF;
-  bp.NDB = ws.NDB;
-  bp.NPG = ws.NPG;
-  const int stages =
-      a->stages ? a->stages : (DSA_STAGE_PREP | DSA_STAGE_DQ | DSA_STAGE_DKDV | DSA_STAGE_FOLD);
-  if (f.dropout_threshold) {
-    if (f.dropout_bits) {
-      // the forward's keep bits, kept by the caller
-      bp.f.drop = static_cast<const uint32_t*>(f.dropout_bits);
-      bp.f.drop_scale = drop_scale(&f);
-    } else {
-      // PREP regenerates them (same seed, same bits) into the workspace; a
-      // DKDV run in a later call reads the ones an earlier PREP left
-      uint32_t* dbits = reinterpret_cast<uint32_t*>(base + ws.drop);
-      if (stages & DSA_STAGE_PREP) {
-        if (launch_dropout_bits(&f, dbits, bp.f, st)) return 1;
-      } else {
-        bp.f.drop = dbits;
-        bp.f.drop_scale = drop_scale(&f);
-      }
-    }
-  }
-
-  if (stages & DSA_STAGE_PREP) {
-    // dkdv's key tiles against 32-query chunks; dq's tiles (128 queries
-    // against 64-key tiles) weigh as the forward's.  Their cost blocks run
-    // first in the prep launch, the sort after it.
-    int* bufs[2];
-    int nts[2];
-    bool kinds[2];
-    int nj = 0;
-    if (kbuf) bufs[nj] = kbuf, nts[nj] = nkt, kinds[nj++] = false;
-    if (qbuf) bufs[nj] = qbuf, nts[nj] = nqt, kinds[nj++] = true;
-    dsa::OrderParams2 op;
-    op.f = bp.f;
-    op.njobs = 0;
-    dsa::PrepBlocks nb;
-    nb.order = 0;
-    nb.order_ny = 1;
-    if (nj) nb.order = fill_orders(bp.f, nj, bufs, nts, kinds, op, nb.order_ny);
-    const int64_t n = (int64_t)f.B * f.H * ws.LqP * (D / (16 / (int)sizeof(T)));
-    nb.delta = (int)((n + 255) / 256);
-    nb.gather = nb.seg = nb.chunk = nb.zero = 0;
-    nb.gacc_floats = 0;
-    if (f.key_keep || f.seg) nb.chunk = (int)(((int64_t)f.B * (ws.LqP / 32) + 255) / 256);
-    if (f.flags) {
-      const int64_t m = 2 * (int64_t)f.H * D * (ws.TGP / (16 / (int)sizeof(T)));
-      nb.gather = (int)((m + 255) / 256);
-      const int64_t ns = 2 * (int64_t)(f.Lq + f.Lk);
-      nb.seg = (int)((ns + 255) / 256);
-      // the table kernel's block accumulators, added to in FOLD
-      nb.gacc_floats = (int64_t)f.H * ws.NDB * 2 * dsa::tbcfg::DBW * D;
-      nb.zero = (int)((nb.gacc_floats / 4 + 255) / 256);
-    }
-    hipLaunchKernelGGL((dsa::dsa_bwd_prep_kernel<T, D>),
-                       dim3((unsigned)(nb.order + nb.gather + nb.seg + nb.chunk + nb.zero + nb.delta)), dim3(256), 0, st,
-                       bp, nb, op);
-    if (launch_check("dsa_bwd_prep_kernel")) return 1;
-    if (nj && launch_order_sort(op, st)) return 1;
-  }
-  if (stages & DSA_STAGE_DKDV) {
-    if (bp.f.drop ? launch_dkdv<T, D, true>(bp, ws, mode, st) : launch_dkdv<T, D, false>(bp, ws, mode, st)) return 1;
-  }
-  // DQ and FOLD both only read dS: with both requested, the dq and table
-  // workgroups run in one launch (dsa_bwd_dqtab.h) and share the GPU.
-  // FOLD is TABLE (the table kernel) followed by SUM (the fold kernel).
-  const bool fold = (stages & (DSA_STAGE_FOLD | DSA_STAGE_TABLE)) && f.flags;
-  const bool sum = (stages & (DSA_STAGE_FOLD | DSA_STAGE_SUM)) && f.flags;
-  const bool dq = (stages & DSA_STAGE_DQ) != 0;
-  // dKr sums dS_ij times the c2p term's query rows: qc when it is given
-  dsa::BwdParams tp = bp;
-  if (f.qc) {
-    tp.f.q = f.qc;
-    for (int s = 0; s < 3; ++s) tp.f.qs[s] = f.qc_strides[s];
-  }
-  const int ntab = ws.NDB * f.H * ws.NPG;
-  const int ndq = ws.LqP / dsa::dqcfg::BQ * f.H * f.B;
-  if (fold && dq) {
-    const int nt8 = (ntab + 7) / 8 * 8;
-    const dim3 grid((unsigned)(nt8 + ndq));
-    const bool listed = bp.cinfo != nullptr;
-    if (listed && f.qc)
-      hipLaunchKernelGGL((dsa::dsa_bwd_dqtab_kernel<T, D, true, true>), grid, dim3(256), 0, st, bp, tp, ntab, nt8, ndq);
-    else if (listed)
-      hipLaunchKernelGGL((dsa::dsa_bwd_dqtab_kernel<T, D, true, false>), grid, dim3(256), 0, st, bp, tp, ntab, nt8, ndq);
-    else if (f.qc)
-      hipLaunchKernelGGL((dsa::dsa_bwd_dqtab_kernel<T, D, false, true>), grid, dim3(256), 0, st, bp, tp, ntab, nt8, ndq);
-    else
-      hipLaunchKernelGGL((dsa::dsa_bwd_dqtab_kernel<T, D, false, false>), grid, dim3(256), 0, st, bp, tp, ntab, nt8, ndq);
-    if (launch_check("dsa_bwd_dqtab_kernel")) return 1;
-  } else if (fold) {
-    if (bp.cinfo)
-      hipLaunchKernelGGL((dsa::dsa_bwd_table_kernel<T, D, true>), dim3(ntab), dim3(256), 0, st, tp);
-    else
-      hipLaunchKernelGGL((dsa::dsa_bwd_table_kernel<T, D, false>), dim3(ntab), dim3(256), 0, st, tp);
-    if (launch_check("dsa_bwd_table_kernel")) return 1;
-  } else if (dq) {
-    if (f.qc)
-      hipLaunchKernelGGL((dsa::dsa_bwd_dq_kernel<T, D, true>), dim3(ndq), dim3(256), 0, st, bp);
-    else
-      hipLaunchKernelGGL((dsa::dsa_bwd_dq_kernel<T, D, false>), dim3(ndq), dim3(256), 0, st, bp);
-    if (launch_check("dsa_bwd_dq_kernel")) return 1;
-  }
-  if (sum) {
-    const int rows = 2 * f.H * (2 * f.att_span);
-    if (f.Lq + f.Lk > 2048)  // long rows of saturated relative positions: four waves a row
-      hipLaunchKernelGGL((dsa::dsa_bwd_fold_kernel<D, 4>), dim3((unsigned)rows), dim3(256), 0, st, bp);
-    else  // one wave a row, four rows a workgroup
-      hipLaunchKernelGGL((dsa::dsa_bwd_fold_kernel<D, 1>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, st, bp);
-    if (launch_check("dsa_bwd_fold_kernel")) return 1;
-  }
-  return 0;
 }
 
 static_assert(kStaticScratchBytes == 2 * kMaxOrderItems * sizeof(int), "the static scratch holds one launch order");

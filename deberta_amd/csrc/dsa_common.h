@@ -266,6 +266,29 @@ DSA_DEV void lds_dma16_nt(const void* src, void* lds_wave) {
       __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(__attribute__((address_space(3))) void*)lds_wave);
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt" ::"v"(src), "s"(lds) : "memory", "m0");
 }
+// The same copies from a wave-uniform base and a 32-bit byte offset per lane
+// (global_load_lds_dwordx4 with a scalar base: no 64-bit address per lane).
+template <typename P>
+DSA_DEV P* uniform_ptr(P* p) {
+  const uintptr_t a = (uintptr_t)p;
+  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)a);
+  const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(a >> 32));
+  return (P*)(((uintptr_t)hi << 32) | lo);
+}
+DSA_DEV void lds_dma16_s(const void* base, unsigned off, void* lds_wave) {
+  base = uniform_ptr(base);
+  const unsigned lds =
+      __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(__attribute__((address_space(3))) void*)lds_wave);
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds)
+               : "memory", "m0");
+}
+DSA_DEV void lds_dma16_s_nt(const void* base, unsigned off, void* lds_wave) {
+  base = uniform_ptr(base);
+  const unsigned lds =
+      __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(__attribute__((address_space(3))) void*)lds_wave);
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(off), "s"(base), "s"(lds)
+               : "memory", "m0");
+}
 // Waits until at most N of this wave's vector-memory instructions are
 // outstanding (they complete in issue order).
 template <int N>

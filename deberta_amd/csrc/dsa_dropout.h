@@ -104,7 +104,7 @@ inline size_t dropout_bits_bytes(int B, int H, int LqP, int LkP) {
 // key group's 16 keys).  Grid (ceil(NKT / 4) * NQB, H, B): a workgroup takes
 // four 64-key tiles of one 32-query block, one wave per tile (a wave past
 // NKT ends at once); consecutive threads write consecutive words.
-__global__ __launch_bounds__(256) void dsa_dropout_bits_kernel(DropParams d) {
+static __global__ __launch_bounds__(256) void dsa_dropout_bits_kernel(DropParams d) {
   const int nx = (d.NKT + 3) / 4;
   const int qb = blockIdx.x / nx;
   const int kt = (blockIdx.x % nx) * 4 + (threadIdx.x >> 6);

@@ -29,7 +29,8 @@ namespace dsa {
 // instead of q.  DROP: attention dropout with the keep bits p.drop
 // (dsa_dropout.h): dropped probabilities leave the PV product, the row sums
 // (and so the lse) keep them, and the output is scaled by p.drop_scale.
-template <typename T, int D, int MASK, bool QC = false, bool DROP = false>
+// FAR: calls that can have far blocks (FarSpan, p.far).
+template <typename T, int D, int MASK, bool QC, bool DROP, bool FAR>
 __global__ __launch_bounds__(256, 2) void dsa_fwd_kernel(FwdParams p) {
   using namespace dcfg;
   using M = Mfma<T>;
@@ -58,6 +59,9 @@ __global__ __launch_bounds__(256, 2) void dsa_fwd_kernel(FwdParams p) {
   __shared__ unsigned char kflag[SEGM ? MAXKT : 1];
   __shared__ short klist[SEGM ? MAXKT : 1];
   __shared__ int klen;
+  // far blocks (FarSpan), per side: the p2c row, and each query's c2p term
+  __shared__ __align__(16) T farq[2][FAR ? D : VEC];
+  __shared__ float fara[2][FAR ? BQ : 1];
 
   const int tid = threadIdx.x;
   const int w = tid >> 6, g = (tid & 63) >> 4, c16 = tid & 15;
@@ -125,6 +129,37 @@ __global__ __launch_bounds__(256, 2) void dsa_fwd_kernel(FwdParams p) {
 #pragma unroll
       for (int s = 0; s < NS; ++s)
         qcf[ib][s] = (irow[ib] < Lq) ? M::load_contig(qcbase + (int64_t)irow[ib] * p.qcs[1], s, g) : M::zero();
+  }
+
+  FarSpan fs{kNoFar, -kNoFar};
+  if constexpr (FAR) {
+    fs = far_span(p);
+#pragma unroll
+    for (int side = 0; side < 2; ++side) {
+      const int e = far_offset(p, side);
+      if (tid < D / VEC) {
+        vecT x;
+#pragma unroll
+        for (int u = 0; u < VEC; ++u) x[u] = (T)0.0f;  // without p2c
+        if (p.flags & 2)
+          x = *reinterpret_cast<const vecT*>(qrh + (int64_t)offset_row(p.rel, e, Lq, Lk, A, true) * p.qrs[1] +
+                                             (tid * VEC / M::KSTEP) * p.qrk + tid * VEC % M::KSTEP);
+        *reinterpret_cast<vecT*>(&farq[side][tid * VEC]) = x;
+      }
+      f32x4 a2[2] = {zero4(), zero4()};
+      if (p.flags & 1) {
+        // every row of the A operand is the far row: the result's rows all
+        // hold the queries' terms
+        const T* row = krh + (int64_t)offset_row(p.rel, e, Lq, Lk, A, false) * p.krs[1];
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+          const frag af = *reinterpret_cast<const frag*>(row + s * p.krk + M::FRAG_ELEMS * g);
+#pragma unroll
+          for (int ib = 0; ib < 2; ++ib) a2[ib] = M::mma(af, pick<QC>(qcf, qf)[ib][s], a2[ib]);
+        }
+      }
+      if (g == 0) fara[side][w * WQ + c16] = a2[0][0], fara[side][w * WQ + 16 + c16] = a2[1][0];
+    }
   }
 
   float mref[2] = {-INFINITY, -INFINITY};  // reference max of the unscaled scores
@@ -267,6 +302,7 @@ __global__ __launch_bounds__(256, 2) void dsa_fwd_kernel(FwdParams p) {
       }
       if (!__syncthreads_or(keep != 0)) continue;
     }
+    const bool far = FAR && fs.far(qt - kt / 2);
     __syncthreads();  // previous tile's LDS reads are done
     // Everything this wave requested in the previous tile has landed or been
     // written by now (the prefetch and the saved-term stores were issued
@@ -288,7 +324,7 @@ __global__ __launch_bounds__(256, 2) void dsa_fwd_kernel(FwdParams p) {
       }
     }
     if (SEGM && tid < BK) ksg[tid] = ksn;
-    if (p.flags) store_row_tables(crow, prow, relv, A, (int)p.krs[1], (int)p.qrs[1], tid);
+    if (p.flags && !far) store_row_tables(crow, prow, relv, A, (int)p.krs[1], (int)p.qrs[1], tid);
     __syncthreads();
 
     // ---- y = K Q^T + c2p + p2c (unscaled) -------------------------------------
@@ -301,27 +337,52 @@ __global__ __launch_bounds__(256, 2) void dsa_fwd_kernel(FwdParams p) {
     // raised wave priority, so that the SIMD's other wave fills in with its
     // softmax (VALU) work (forward 144.8 -> 143.7 us in one process).
     f32x4 st[2][4];
+    float fa[2] = {0.f, 0.f};  // a far tile's c2p term of the lane's queries
     __builtin_amdgcn_s_setprio(1);
+    if (FAR && far) {
+      // the p2c term is the keys' products with one row (every column of
+      // the B operand), the start of the score products; the c2p term, one
+      // value a query, joins at the softmax
+      const int side = fs.side(qt - kt / 2);
+      frag qb[NS];
 #pragma unroll
-    for (int jb = 0; jb < 4; ++jb)
+      for (int s = 0; s < NS; ++s) qb[s] = M::load_contig(&farq[side][0], s, g);
+      fa[0] = fara[side][w * WQ + c16], fa[1] = fara[side][w * WQ + 16 + c16];
 #pragma unroll
-      for (int ib = 0; ib < 2; ++ib) {
-        f32x4 acc = zero4();
+      for (int jb = 0; jb < 4; ++jb) {
+        f32x4 bj = zero4();
 #pragma unroll
-        for (int s = 0; s < NS; ++s) acc = M::mma(kf[jb][s], qf[ib][s], acc);
-        st[ib][jb] = acc;
+        for (int s = 0; s < NS; ++s) bj = M::mma(kf[jb][s], qb[s], bj);
+#pragma unroll
+        for (int ib = 0; ib < 2; ++ib) {
+          f32x4 acc = bj;
+#pragma unroll
+          for (int s = 0; s < NS; ++s) acc = M::mma(kf[jb][s], qf[ib][s], acc);
+          st[ib][jb] = acc;
+        }
       }
+    } else {
+#pragma unroll
+      for (int jb = 0; jb < 4; ++jb)
+#pragma unroll
+        for (int ib = 0; ib < 2; ++ib) {
+          f32x4 acc = zero4();
+#pragma unroll
+          for (int s = 0; s < NS; ++s) acc = M::mma(kf[jb][s], qf[ib][s], acc);
+          st[ib][jb] = acc;
+        }
+    }
     // The next tile is requested only after this tile's band rows have been
     // waited for (a wave's vector-memory requests complete in issue order,
     // so a request issued before them would be waited for with them) and
     // before the saved-term stores (with stores outstanding the compiler
     // cannot order the counts and waits for everything).  It has the gather,
     // the softmax and the PV product to land.
-    if (p.flags)
+    if (p.flags && !far)
       band_products_T<T, D, MASK == MASK_PAIR ? 3 : 6>(kf, pick<QC>(qcf, qf), cb, pb, crow, prow, w, g, c16, krh, qrh,
                                                        p.krk, p.qrk, p.flags);
     if (n + 1 < nlist) fetch(SEGM ? __builtin_amdgcn_readfirstlane(klist[n + 1]) : n + 1);
-    if (p.flags) band_gather_T<T, D>(st, cb, pb, w, g, c16, p.flags, biasl ? biasl + (int64_t)kt * 8192 : nullptr);
+    if (p.flags && !far) band_gather_T<T, D>(st, cb, pb, w, g, c16, p.flags, biasl ? biasl + (int64_t)kt * 8192 : nullptr);
     __builtin_amdgcn_s_setprio(0);
 
     // ---- mask: only where a key or query of the tile can be masked out ------
@@ -368,6 +429,7 @@ __global__ __launch_bounds__(256, 2) void dsa_fwd_kernel(FwdParams p) {
       for (int jb = 0; jb < 4; ++jb)
 #pragma unroll
         for (int e = 0; e < 4; ++e) mt = fmaxf(mt, st[ib][jb][e]);
+      mt += fa[ib];
       lm[ib] = mt;
       raise = raise || mt > mref[ib] + thr;
     }
@@ -384,7 +446,7 @@ __global__ __launch_bounds__(256, 2) void dsa_fwd_kernel(FwdParams p) {
     }
 #pragma unroll
     for (int ib = 0; ib < 2; ++ib) {
-      const float mb = (mref[ib] == -INFINITY) ? 0.f : mref[ib] * sl2;
+      const float mb = (mref[ib] == -INFINITY) ? 0.f : (mref[ib] - fa[ib]) * sl2;
       float ls = 0.f;
 #pragma unroll
       for (int jb = 0; jb < 4; ++jb)

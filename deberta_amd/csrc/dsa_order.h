@@ -169,7 +169,7 @@ DSA_DEV void order_cost_block(const OrderParams2& op2, int b, int by, int jb) {
   if (lane == 0) op.cost[(int64_t)b * op.ntiles + i] = min(n, ORDER_MAX_COST);
 }
 
-__global__ __launch_bounds__(256) void dsa_order_cost_kernel(OrderParams2 op2) {
+static __global__ __launch_bounds__(256) void dsa_order_cost_kernel(OrderParams2 op2) {
   order_cost_block(op2, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
@@ -177,7 +177,7 @@ __global__ __launch_bounds__(256) void dsa_order_cost_kernel(OrderParams2 op2) {
 // (ncost of them, batch row fastest; none without an order) first, then the
 // k-step copies of the relative tables (ncopy blocks per table; none
 // without the copies).  The sort runs after it (dsa_order_sort_kernel).
-__global__ __launch_bounds__(256) void dsa_fwd_pre_kernel(TableKs t, OrderParams2 op2, int ncost, int ncopy) {
+static __global__ __launch_bounds__(256) void dsa_fwd_pre_kernel(TableKs t, OrderParams2 op2, int ncost, int ncopy) {
   const int blk = blockIdx.x;
   if (blk < ncost) {
     order_cost_block(op2, blk % op2.f.B, blk / op2.f.B, 0);
@@ -187,7 +187,7 @@ __global__ __launch_bounds__(256) void dsa_fwd_pre_kernel(TableKs t, OrderParams
   }
 }
 
-__global__ __launch_bounds__(1024) void dsa_order_sort_kernel(OrderParams2 op) {
+static __global__ __launch_bounds__(1024) void dsa_order_sort_kernel(OrderParams2 op) {
   // cost c sits at position ORDER_MAX_COST - c (heaviest first); thread t
   // owns positions 2t and 2t + 1
   __shared__ int hist[2 * 1024];

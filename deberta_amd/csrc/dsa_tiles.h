@@ -38,6 +38,7 @@ struct FwdParams {
   const uint32_t* drop;
   float drop_scale;
   void* olo;        // bf16 only: O's rounding residual, with out's strides, or null
+  int far;          // far blocks are looked for (FarSpan)
 };
 
 struct BwdParams {
@@ -54,7 +55,7 @@ struct BwdParams {
   void* dqr;
   int dtab_bf16, dtab_overwrite;
   // workspace
-  float* rowinfo;   // [B, H, LqP, 2]: lse*log2e (inf: dead or padding row), dO . O
+  float* rowinfo;   // [B, H, LqP, 2]: lse*log2e (inf: dead or padding row), dO . O; three planes with far blocks
   void* ds;         // dS [B, H, f.LqP, f.LkP] (rows = queries), zero outside [0, Lq) x [0, Lk)
   void* krgt;       // [H, D, TGP]: krgt[h][d][t] = Kr[h][c(t - OFF)][d]
   void* qrgt;       // [H, D, TGP]: qrgt[h][d][t] = Qr[h][p(t - OFF)][d]
@@ -65,7 +66,10 @@ struct BwdParams {
   const int* korder;  // dkdv launch order of the (batch row, key tile) items, or null (dsa_order.h)
   const int* qorder;  // dq launch order of the (batch row, query tile) items, or null
   int TGP, OFF;     // row length and offset origin of krgt / qrgt
+  float* farpart;   // far blocks' table gradient partials (far_part)
+  int* farspan;     // the call's FarSpan, found by the prep kernel
   int NDB, NPG;     // offset blocks, partial groups per block (item ranges)
+  int fardq;        // the dq kernel adds the far blocks' dKr sums (it runs beside the table kernel, which leaves them out)
 };
 
 // Segment view of the key-padding (MASK_KEY) and segment-id (MASK_SEG)
@@ -162,6 +166,109 @@ DSA_DEV SegRange wg_seg_range(int s, bool has, int* red) {
     r.all = r.all && red[3 * k + 2] != 0;
   }
   return r;
+}
+
+// Far blocks: the 128-query x 128-key blocks (query block qt, key block kt)
+// whose offsets all read one c2p row and one p2c row, because the relative
+// position saturates there.  The rows are monotone in the offset, so block
+// diagonal delta = qt - kt >= 1 is far iff its smallest offset, 128 delta -
+// 127, has the rows of the largest offset of the call, Lq - 1; then every
+// larger delta is far too, and likewise for delta <= -1 with -(Lk - 1).  In
+// a far block the relative term of pair (i, j) is a_i + b_j with a_i = q_i .
+// Kr[c] and b_j = k_j . Qr[p] of the one row pair, so no band is computed,
+// gathered, saved or read back: the products of a tile fall to those of
+// plain attention, its gradients to one row and one column sum of dS (s_i,
+// t_j):
+//   dQ_i += s_i Kr[c],  dKr[c] += sum_i s_i q_i,  and so for K and Qr.
+// At position buckets 256 / max_position 512 delta >= 5 is far: 52% of the
+// blocks at L = 2048, 74% at L = 4096.  Whether blocks can be far is decided
+// on the host from the extents (far_wanted), so shorter calls search nothing.
+// The forward finds the span itself, the backward's prep kernel finds the
+// same one from the same table for the kernels after it.
+constexpr int kNoFar = 1 << 26;  // a block diagonal past every call's (and 4x it, the 32-query tiles, in range)
+struct FarSpan {
+  int pos, neg;  // far iff delta >= pos or delta <= neg
+  DSA_DEV bool far(int delta) const { return delta >= pos || delta <= neg; }
+  DSA_DEV int side(int delta) const { return delta > 0 ? 0 : 1; }  // of a far delta: 0 past pos, 1 past neg
+};
+// The host's rule: the furthest block diagonal's smallest offset is at least
+// the 2 att_span rows of a table.  An unbucketed table saturates att_span
+// offsets out, the log-bucketed ones of max_position = 2 att_span about 2
+// att_span out; nearer searches would find nothing or a corner block.
+inline bool far_wanted(int flags, int LqP, int LkP, int A) {
+  return flags != 0 && (LqP > LkP ? LqP : LkP) - 128 - 127 >= 2 * A;
+}
+// Offset whose table rows a far block of this side reads.
+DSA_DEV int far_offset(const FwdParams& p, int side) { return side == 0 ? p.Lq - 1 : -(p.Lk - 1); }
+
+// Table row of offset d (clamped into the relative-position table's range).
+DSA_DEV int offset_row(const int32_t* rel, int d, int Lq, int Lk, int A, bool p2c) {
+  d = min(max(d, -(Lk - 1)), Lq - 1);
+  const int t = min(max(rel[d + Lk - 1], -A), A);
+  return p2c ? p2c_row(t, A) : c2p_row(t, A);
+}
+
+// Every lane of the wave calls it (one block diagonal a lane); the result is
+// uniform.
+DSA_DEV FarSpan far_span(const FwdParams& p) {
+  FarSpan s{kNoFar, -kNoFar};
+  if (!p.far) return s;
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int side = 0; side < 2; ++side) {
+    const int n = (side == 0 ? p.LqP : p.LkP) / 128;
+    const int e = far_offset(p, side);
+    const int ce = offset_row(p.rel, e, p.Lq, p.Lk, p.A, false), pe = offset_row(p.rel, e, p.Lq, p.Lk, p.A, true);
+    for (int d0 = 1; d0 < n; d0 += 64) {
+      const int d = d0 + lane;
+      const int o = side == 0 ? 128 * d - 127 : -(128 * d - 127);
+      const bool ok = d < n && (!(p.flags & 1) || offset_row(p.rel, o, p.Lq, p.Lk, p.A, false) == ce) &&
+                      (!(p.flags & 2) || offset_row(p.rel, o, p.Lq, p.Lk, p.A, true) == pe);
+      const unsigned long long m = __ballot(ok);
+      if (m) {
+        const int f = d0 + __builtin_ctzll(m);
+        if (side == 0) s.pos = f;
+        else s.neg = -f;
+        break;
+      }
+    }
+  }
+  return s;
+}
+
+// The span the prep kernel left for the backward's kernels.
+DSA_DEV FarSpan far_span_of(const BwdParams& bp) {
+  return FarSpan{__builtin_amdgcn_readfirstlane(bp.farspan[0]), __builtin_amdgcn_readfirstlane(bp.farspan[1])};
+}
+
+// Rows summed into a far block's table gradient row: out[k] (k = 0 .. D - 1,
+// LDS, this wave's) = sum over the wave's 32 columns (two 16-wide tiles,
+// column c16 of tile t in the lanes c16 of every group g) of coef[t] *
+// rows[t][..][k], rows the columns' operand fragments (CONTIG k-set), coef the
+// same in the four lane groups.
+template <typename T, int NS>
+DSA_DEV void far_row_sum(float* out, const float (&coef)[2], const typename Mfma<T>::frag (&rows)[2][NS], int g,
+                         int c16) {
+  using M = Mfma<T>;
+#pragma unroll
+  for (int s = 0; s < NS; ++s)
+#pragma unroll
+    for (int e = 0; e < M::FRAG_ELEMS; ++e) {
+      float v = coef[0] * (float)rows[0][s][e] + coef[1] * (float)rows[1][s][e];
+#pragma unroll
+      for (int o = 1; o < 16; o <<= 1) v += __shfl_xor(v, o);
+      if (c16 == 0) out[M::KSTEP * s + M::FRAG_ELEMS * g + e] = v;
+    }
+}
+// The far partials of a call, [H][kind 0: dKr, 1: dQr][side][item][D] fp32:
+// one row per workgroup of the dq (kind 0) and dkdv (kind 1) kernels, item =
+// batch row * tiles + tile, zeroed by the prep kernel and summed by the fold.
+// (Added to the accumulators with atomics instead, whose few addresses every
+// workgroup then meets at, they cost dkdv 56 us and DQ|TABLE 91 us at B=4,
+// L=2048, H=16.)
+DSA_DEV float* far_part(float* base, const FwdParams& p, int h, int kind, int side, int D) {
+  const int nt = (p.LqP > p.LkP ? p.LqP : p.LkP) / 128;
+  return base + (int64_t)((h * 2 + kind) * 2 + side) * p.B * nt * D;
 }
 
 template <typename T>
@@ -270,7 +377,7 @@ DSA_DEV void table_ks_block(const TableKs& t, int bx, int tb) {
   const char* src = (const char*)t.src[tb] + ((int64_t)h * t.hs[tb] + (int64_t)r * t.rs[tb] + s * ks + q * per16) * t.esize;
   *reinterpret_cast<uint4*>((char*)t.dst[tb] + c * 16) = *reinterpret_cast<const uint4*>(src);
 }
-__global__ __launch_bounds__(256) void dsa_table_ks_kernel(TableKs t) { table_ks_block(t, blockIdx.x, blockIdx.y); }
+static __global__ __launch_bounds__(256) void dsa_table_ks_kernel(TableKs t) { table_ks_block(t, blockIdx.x, blockIdx.y); }
 
 // Row tables of one tile: crow[x] / prow[x] are the element offsets (row *
 // row stride) of the c2p / p2c table rows of offset x (x = (i - i0) - (j -

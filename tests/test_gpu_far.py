@@ -1,0 +1,102 @@
+"""Far blocks: 128 x 128 blocks of (query, key) pairs whose relative position
+has saturated, run without bands (FarSpan, dsa_tiles.h).  The op against the
+CPU oracle where the rule or the span can go wrong: extents on both sides of
+the rule, a span on one side only, past the last query or key block or
+nowhere, every mask form that takes it, dropout and the p2p query rows; and
+the backward in separate stage calls against the one call.  The bounds are the
+parity suite's (fp32 1e-4 of scale, bf16 2e-2)."""
+
+from __future__ import annotations
+
+import ctypes
+import math
+
+import pytest
+import torch
+
+from tests._cases import Case
+from tests.test_gpu_parity import _check
+
+pytestmark = pytest.mark.gpu
+
+_CASES = [
+    Case(B=1, H=2, L=256, D=64, buckets=-1, max_pos=1, seed=1),  # saturated beside the diagonal, 2 blocks
+    Case(B=2, H=2, L=384, D=64, buckets=32, max_pos=64, seed=2),  # first length past the rule (129 >= 64)
+    Case(B=1, H=2, L=385, D=32, buckets=32, max_pos=64, seed=3),  # one row in the last block
+    Case(B=1, H=1, L=700, D=64, buckets=64, max_pos=512, seed=4),  # looked for, hardly any found
+    Case(B=1, H=1, L=450, D=64, buckets=64, max_pos=4096, seed=5),  # looked for, none found
+    Case(B=2, H=1, L=90, Lk=700, D=64, buckets=32, max_pos=64, seed=6),  # key side only, one query block
+    Case(B=2, H=1, L=700, Lk=90, D=32, buckets=32, max_pos=64, seed=7),  # query side only
+    Case(B=1, H=2, L=641, D=64, buckets=32, max_pos=64, types="c2p", seed=8),
+    Case(B=1, H=2, L=641, D=64, buckets=32, max_pos=64, types="p2c", seed=9),
+    Case(B=1, H=2, L=640, D=64, buckets=-1, max_pos=64, types="c2p|p2c|p2p", seed=10),
+    Case(B=3, H=2, L=600, D=64, buckets=32, max_pos=64, mask="key", seed=11),
+    Case(B=2, H=2, L=900, D=64, buckets=32, max_pos=64, mask="seg", seed=12),
+    Case(B=2, H=2, L=520, D=32, buckets=32, max_pos=64, mask="seg_mixed", seed=13),
+    Case(B=2, H=2, L=500, D=64, buckets=32, max_pos=64, mask="dead", seed=14),
+    Case(B=1, H=2, L=600, D=64, buckets=32, max_pos=64, dropout=0.1, seed=15),
+    Case(B=2, H=1, L=700, D=64, buckets=32, max_pos=64, mask="seg", dropout=0.1, seed=16),
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("c", _CASES, ids=[str(c.seed) for c in _CASES])
+def test_far_blocks(c, dtype, gpu):
+    # a saturated table row sums nearly all pairs of a head: its bf16
+    # gradient is held to its scale
+    _check(c, dtype, gpu, grads_to_scale=True)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("p2p", [False, True])
+@pytest.mark.parametrize("Lq,Lk", [(640, 640), (130, 900)])
+def test_far_stage_split(Lq, Lk, p2p, dtype, gpu):
+    """PREP, DKDV, DQ, TABLE and SUM in calls of their own (the table kernel
+    then sums the far blocks' dKr itself) and DQ|TABLE in one, against one
+    call for all."""
+    from deberta_amd import _lib, ops
+    from deberta_amd.attention import relative_operands
+    from deberta_amd.relpos import relative_offset_table
+
+    lib = _lib.load()
+    B, H, D, A = 2, 2, 64, 32
+    g = torch.Generator().manual_seed(5)
+    mk = lambda *s: torch.randn(*s, generator=g).to(gpu, dtype)
+    q, k, v, dout = mk(B, Lq, H, D), mk(B, Lk, H, D), mk(B, Lk, H, D), mk(B, Lq, H, D)
+    kr, qr = mk(H, 2 * A, D), mk(H, 2 * A, D)
+    table = relative_offset_table(Lq, Lk, bucket_size=A, max_position=64, device=gpu)
+    qc = relative_operands(["c2p", "p2c", "p2p"], q, kr, qr, A)[2].contiguous() if p2p else None
+    scale = 1 / math.sqrt(D * 3)
+    out, lse, bias, aux = torch.ops.deberta_amd.dsa_fwd(q, k, v, kr, qr, table, None, None, A, scale, True, qc)
+    stream = ctypes.c_void_p(torch.cuda.current_stream(gpu).cuda_stream)
+    bits = {n: getattr(_lib, f"DSA_STAGE_{n}") for n in ("PREP", "DQ", "DKDV", "TABLE", "SUM")}
+
+    def run(calls):
+        grads = [torch.full_like(t, float("nan")) for t in (q, k, v)]
+        dqc = torch.full_like(q, float("nan")) if p2p else None
+        tabs = [torch.zeros((H, 2 * A, D), dtype=torch.float32, device=gpu) for _ in range(2)]
+        a = ops.fill_bwd_args(dout, q, k, v, kr, qr, table, None, None, out, lse, bias, A, scale, *grads, *tabs,
+                              qc=qc, dqc=dqc, dropout_bits=aux)
+        ws = torch.empty((ops.bwd_workspace_bytes(a),), dtype=torch.uint8, device=gpu)
+        a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
+        for c in calls:
+            a.stages = sum(bits[s] for s in c.split("|") if s)
+            _lib.check(lib.dsa_bwd(ctypes.byref(a), stream), "dsa_bwd")
+        torch.cuda.synchronize(gpu)
+        return dict(zip(["dq", "dk", "dv", "dkr", "dqr", "dqc"], grads + tabs + [dqc]))
+
+    ref = run([""])
+    # the far rows are summed from float32 row sums of dS in one call and from
+    # its products in the other: fp32 sums in another order, and for bf16 the
+    # same products of bf16 dS
+    for calls in (["PREP", "DKDV", "DQ", "TABLE", "SUM"], ["PREP", "DKDV", "DQ|TABLE", "SUM"]):
+        got = run(calls)
+        for name, b in ref.items():
+            if b is None:
+                continue
+            assert torch.isfinite(got[name]).all(), name
+            if name in ("dkr", "dqr"):
+                err = float((got[name] - b).abs().max() / b.abs().max())
+                assert err <= 1e-5, (calls, name, err)
+            else:
+                assert torch.equal(got[name], b), (calls, name)
