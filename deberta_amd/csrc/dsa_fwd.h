@@ -240,6 +240,21 @@ __global__ __launch_bounds__(256, 2) void dsa_fwd_kernel(FwdParams p) {
   int relv = 0;  // this thread's relative position of the fetched tile (tid < XG)
   int ksn = 0;   // segment masks: this thread's key segment of the fetched tile (tid < BK)
   int kfetched = -1;
+  // The bands' carried operands (band_products_T, CARRY).  The new p2c rows of
+  // a tile (row block w) are requested with its K and V; the relative
+  // positions of their 16 offsets, requested a tile earlier still, are there
+  // by then.
+  // (Forward 137.9 -> 131.6 us at B=32, L=512, H=12, 82.4 -> 81.2 with padded
+  // rows, 246 -> 234 with documents at B=4, L=4096.  Not for the pair mask and
+  // the p2p query rows, whose kernels have no registers for the held rows, nor
+  // for fp32, whose rows are four loads each.)
+  constexpr bool CARRY = sizeof(T) == 2 && MASK != MASK_PAIR && !QC;
+  frag pheld[CARRY ? 3 : 1][NS], pnew[NS];
+#pragma unroll
+  for (int s = 0; s < NS; ++s) pnew[s] = M::zero();
+  int prel = 0;          // relative position of the lane's offset of row block w, of the tile to fetch next
+  int btile = -2;        // the tile whose bands the wave computed last
+  auto prel_at = [&](int kt) { return rel_of_tile(p.rel, i0, kt * BK, Lq, Lk, 16 * w + c16); };
   // dropout: this lane's keep word of the fetched tile (bit 16 ib + 4 jb + e)
   uint32_t dwn = 0;
   const uint32_t* dropw = nullptr;
@@ -252,6 +267,14 @@ __global__ __launch_bounds__(256, 2) void dsa_fwd_kernel(FwdParams p) {
     if constexpr (DROP) dwn = dropw[(int64_t)kt * 64];
     if (p.flags && tid < XG) relv = rel_of_tile(p.rel, i0, j0, Lq, Lk, tid);
     if (SEGM && tid < BK) ksn = j0 + tid < Lk ? sv(j0 + tid) : 0;
+    if constexpr (CARRY) {
+      if (p.flags & 2) {
+        const T* row = qrh + p2c_row(min(max(prel, -A), A), A) * (int)p.qrs[1];
+#pragma unroll
+        for (int s = 0; s < NS; ++s) pnew[s] = *reinterpret_cast<const frag*>(row + s * p.qrk + M::FRAG_ELEMS * g);
+        prel = prel_at(kt + 1);
+      }
+    }
 #pragma unroll
     for (int k = 0; k < KCH; ++k) {
       const int c = tid + 256 * k;
@@ -265,7 +288,13 @@ __global__ __launch_bounds__(256, 2) void dsa_fwd_kernel(FwdParams p) {
     }
     kfetched = kt;
   };
-  if (any_live && nlist > 0) fetch(SEGM ? __builtin_amdgcn_readfirstlane(klist[0]) : 0);
+  if (any_live && nlist > 0) {
+    const int k0 = SEGM ? __builtin_amdgcn_readfirstlane(klist[0]) : 0;
+    if constexpr (CARRY) {
+      if (p.flags & 2) prel = prel_at(k0);
+    }
+    fetch(k0);
+  }
   // The Q fragments and the first tile have landed before the loop (its
   // first iteration waits for the tile anyway).  Without this wait the
   // loads issued before the loop stay pending in the compiler's view of the
@@ -378,10 +407,19 @@ __global__ __launch_bounds__(256, 2) void dsa_fwd_kernel(FwdParams p) {
     // before the saved-term stores (with stores outstanding the compiler
     // cannot order the counts and waits for everything).  It has the gather,
     // the softmax and the PV product to land.
-    if (p.flags && !far)
-      band_products_T<T, D, MASK == MASK_PAIR ? 3 : 6>(kf, pick<QC>(qcf, qf), cb, pb, crow, prow, w, g, c16, krh, qrh,
-                                                       p.krk, p.qrk, p.flags);
-    if (n + 1 < nlist) fetch(SEGM ? __builtin_amdgcn_readfirstlane(klist[n + 1]) : n + 1);
+    if (p.flags && !far) {
+      band_products_T<T, D, CARRY ? 4 : MASK == MASK_PAIR ? 3 : 6, CARRY>(kf, pick<QC>(qcf, qf), cb, pb, crow, prow, w, g,
+                                                                          c16, krh, qrh, p.krk, p.qrk, p.flags,
+                                                                          btile == kt - 1, pheld, pnew);
+      btile = kt;
+    }
+    if (n + 1 < nlist) {
+      const int kn = SEGM ? __builtin_amdgcn_readfirstlane(klist[n + 1]) : n + 1;
+      if constexpr (CARRY && SEGM) {
+        if ((p.flags & 2) && kn != kt + 1) prel = prel_at(kn);
+      }
+      fetch(kn);
+    }
     if (p.flags && !far) band_gather_T<T, D>(st, cb, pb, w, g, c16, p.flags, biasl ? biasl + (int64_t)kt * 8192 : nullptr);
     __builtin_amdgcn_s_setprio(0);
 

@@ -461,12 +461,24 @@ DSA_DEV void store4_contig(B* p, const f32x4& v) {
 // waited for on return), band_gather_T (which begins with a __syncthreads:
 // the p2c band is shared) adds them to y and stores the saved term.  Call
 // both from every thread of the workgroup.
-template <typename T, int D, int GR>
+//   CARRY, for a caller that walks the key tiles in order: the offsets of row
+//   block b of a tile are those of block b + 4 of the next.  With adj (the
+//   wave's previous call was the tile before), the c2p rows [64, 96) are
+//   copied from that tile's rows [0, 32), which cb still holds, instead of
+//   loaded and multiplied again; and held carries the p2c operands (wave w
+//   takes the row blocks w, w + 4 and w + 8): on return those of this tile,
+//   whose first, pnew, the caller requested ahead.  The row loads are a
+//   fixed cost per instruction (64 lanes x 16 bytes gathered: about 1.4 us
+//   of the forward per load and tile at B=32, L=512, whether they hit or
+//   not); 18 a tile and wave become 10.
+template <typename T, int D, int GR, bool CARRY>
 DSA_DEV void band_products_T(const typename Mfma<T>::frag (&kf)[4][D / Mfma<T>::KSTEP],
                              const typename Mfma<T>::frag (&qf)[2][D / Mfma<T>::KSTEP],
                              typename BandType<T>::type* cb, typename BandType<T>::type* pb, const int* crow,
                              const int* prow, int w, int g, int c16, const T* krh, const T* qrh, int64_t krk,
-                             int64_t qrk, int flags) {
+                             int64_t qrk, int flags, bool adj,
+                             typename Mfma<T>::frag (&held)[CARRY ? 3 : 1][D / Mfma<T>::KSTEP],
+                             const typename Mfma<T>::frag (&pnew)[D / Mfma<T>::KSTEP]) {
   using M = Mfma<T>;
   typedef typename M::frag frag;
   typedef typename BandType<T>::type BT;
@@ -478,20 +490,19 @@ DSA_DEV void band_products_T(const typename Mfma<T>::frag (&kf)[4][D / Mfma<T>::
     return *reinterpret_cast<const frag*>(rowp + s * ks + FE * g);
   };
   if (flags & 1) {
-    // GR row blocks have their table rows requested together (one L2
-    // round trip per group)
-    static_assert((XW / 16) % GR == 0, "whole groups");
+    // n row blocks from rb0 on, whose table rows are requested together (one
+    // L2 round trip per group)
+    auto group = [&](auto n, int rb0) {
+      constexpr int N = decltype(n)::value;
+      frag af[N][NS];
 #pragma unroll
-    for (int rb0 = 0; rb0 < XW / 16; rb0 += GR) {
-      frag af[GR][NS];
-#pragma unroll
-      for (int u = 0; u < GR; ++u) {
+      for (int u = 0; u < N; ++u) {
         const T* rowp = krh + crow[WQ * w + 16 * (rb0 + u) + c16];
 #pragma unroll
         for (int s = 0; s < NS; ++s) af[u][s] = row_frag(rowp, krk, s);
       }
 #pragma unroll
-      for (int u = 0; u < GR; ++u)
+      for (int u = 0; u < N; ++u)
 #pragma unroll
         for (int ib = 0; ib < 2; ++ib) {
           f32x4 acc = zero4();
@@ -499,16 +510,64 @@ DSA_DEV void band_products_T(const typename Mfma<T>::frag (&kf)[4][D / Mfma<T>::
           for (int s = 0; s < NS; ++s) acc = M::mma(af[u][s], qf[ib][s], acc);
           store4_contig<BT>(cb + (16 * ib + c16) * CTS + 16 * (rb0 + u) + 4 * g, acc);
         }
+    };
+    if constexpr (CARRY) {
+      static_assert(XW == 96 && BK == 64, "four new row blocks and two carried ones");
+      if (adj) {
+        typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+        constexpr int CPR = 32 * (int)sizeof(BT) / 16;  // 16-byte chunks of a row's 32 carried columns
+        const int lane = 16 * g + c16;
+        u4 v[WQ * CPR / 64];
+#pragma unroll
+        for (int k = 0; k < WQ * CPR / 64; ++k) {
+          const int c = 64 * k + lane;
+          v[k] = *reinterpret_cast<const u4*>((const char*)(cb + (c / CPR) * CTS) + (c % CPR) * 16);
+        }
+        wave_lds_sync();
+#pragma unroll
+        for (int k = 0; k < WQ * CPR / 64; ++k) {
+          const int c = 64 * k + lane;
+          *reinterpret_cast<u4*>((char*)(cb + (c / CPR) * CTS + BK) + (c % CPR) * 16) = v[k];
+        }
+      } else {
+        group(std::integral_constant<int, 2>{}, 4);
+      }
+      group(std::integral_constant<int, GR>{}, 0);
+      if constexpr (GR < 4) group(std::integral_constant<int, 4 - GR>{}, GR);
+    } else {
+      static_assert((XW / 16) % GR == 0, "whole groups");
+#pragma unroll
+      for (int rb0 = 0; rb0 < XW / 16; rb0 += GR) group(std::integral_constant<int, GR>{}, rb0);
     }
   }
   if (flags & 2) {
+    if constexpr (CARRY) {
+      if (adj) {
+#pragma unroll
+        for (int s = 0; s < NS; ++s) held[2][s] = held[1][s], held[1][s] = held[0][s];
+      } else {
+#pragma unroll
+        for (int t = 1; t < 3; ++t) {
+          const T* rowp = qrh + prow[16 * (w + NW * t) + c16];
+#pragma unroll
+          for (int s = 0; s < NS; ++s) held[t][s] = row_frag(rowp, qrk, s);
+        }
+      }
+#pragma unroll
+      for (int s = 0; s < NS; ++s) held[0][s] = pnew[s];
+    }
 #pragma unroll
     for (int t = 0; t < XG / 16 / NW; ++t) {
       const int xb = w + NW * t;
-      const T* rowp = qrh + prow[16 * xb + c16];
       frag bf[NS];
+      if constexpr (CARRY) {
 #pragma unroll
-      for (int s = 0; s < NS; ++s) bf[s] = row_frag(rowp, qrk, s);
+        for (int s = 0; s < NS; ++s) bf[s] = held[t][s];
+      } else {
+        const T* rowp = qrh + prow[16 * xb + c16];
+#pragma unroll
+        for (int s = 0; s < NS; ++s) bf[s] = row_frag(rowp, qrk, s);
+      }
 #pragma unroll
       for (int jb = 0; jb < 4; ++jb) {
         f32x4 acc = zero4();
@@ -617,7 +676,8 @@ DSA_DEV void add_delta_bands_T(f32x4 (&y)[2][4], const typename Mfma<T>::frag (&
                                typename BandType<T>::type* cb, typename BandType<T>::type* pb, const int* crow,
                                const int* prow, int w, int g, int c16, const T* krh, const T* qrh, int64_t krk,
                                int64_t qrk, int flags, typename BandType<T>::type* bias = nullptr) {
-  band_products_T<T, D, GR>(kf, qf, cb, pb, crow, prow, w, g, c16, krh, qrh, krk, qrk, flags);
+  typename Mfma<T>::frag none[1][D / Mfma<T>::KSTEP] = {};
+  band_products_T<T, D, GR, false>(kf, qf, cb, pb, crow, prow, w, g, c16, krh, qrh, krk, qrk, flags, false, none, none[0]);
   band_gather_T<T, D>(y, cb, pb, w, g, c16, flags, bias);
 }
 
