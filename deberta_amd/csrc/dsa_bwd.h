@@ -196,14 +196,14 @@ DSA_DEV void prep_zero(const BwdParams& bp, int64_t gacc_floats, int blk) {
 }
 
 struct PrepBlocks {
-  int order, order_ny, gather, seg, chunk, zero, delta;
+  int order, order_ny, gather, seg, chunk, zero, pair, delta;
   int64_t gacc_floats;
 };
 // Blocks: the launch orders' cost blocks (dsa_order.h; batch row fastest,
 // then the tile group, then the job) first, then gather, segments, chunk
-// summaries, zeroing and rowinfo.
+// summaries, zeroing, a pair mask's bits and rowinfo.
 template <typename T, int D>
-__global__ __launch_bounds__(256) void dsa_bwd_prep_kernel(BwdParams bp, PrepBlocks nb, OrderParams2 op2) {
+__global__ __launch_bounds__(256) void dsa_bwd_prep_kernel(BwdParams bp, PrepBlocks nb, OrderParams2 op2, PairBits pb) {
   if ((int)blockIdx.x < nb.order) {
     const int k = blockIdx.x, B = op2.f.B;
     order_cost_block(op2, k % B, (k / B) % nb.order_ny, k / (B * nb.order_ny));
@@ -222,8 +222,10 @@ __global__ __launch_bounds__(256) void dsa_bwd_prep_kernel(BwdParams bp, PrepBlo
     prep_chunks(bp, blk - nb.gather - nb.seg);
   } else if (blk < nb.gather + nb.seg + nb.chunk + nb.zero) {
     prep_zero(bp, nb.gacc_floats, blk - nb.gather - nb.seg - nb.chunk);
+  } else if (blk < nb.gather + nb.seg + nb.chunk + nb.zero + nb.pair) {
+    pair_bits_block(pb, blk - nb.gather - nb.seg - nb.chunk - nb.zero);
   } else {
-    prep_delta<T, D>(bp, blk - nb.gather - nb.seg - nb.chunk - nb.zero);
+    prep_delta<T, D>(bp, blk - nb.gather - nb.seg - nb.chunk - nb.zero - nb.pair);
   }
 }
 

@@ -26,7 +26,8 @@
 //                qrgt window (160 offsets of the workgroup) is a ring of
 //                32-offset blocks, one new block per tile.
 // Every query tile of the padded extent is visited, so dS is fully written
-// (zeros for masked pairs, dead rows and padding).
+// (zeros for masked pairs, dead rows and padding), or, under a mask, the
+// listed tiles are and the others are neither written nor read.
 #pragma once
 
 #include "dsa_bwd.h"
@@ -84,17 +85,22 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
   __shared__ __align__(16) T Stg[NW * SW];        // each wave's dS^T tile
   // dropout: each wave's keep words of the tile (one per lane), double-buffered
   __shared__ __align__(16) uint32_t Dk0[DROP ? NW * 64 : 1], Dk1[DROP ? NW * 64 : 1];
+  static_assert(MASK != MASK_PAIR, "pair masks come as bits");
   constexpr bool SEGM = seg_mode(MASK);
+  constexpr bool BITS = MASK == MASK_BITS;
+  constexpr bool LIST = SEGM || BITS;  // the query tiles to visit are listed
   constexpr int MAXQT = 1024;  // query tiles (Lq <= 32768)
   // segment masks: the active query tiles in order (tile | 0x4000 if it
   // needs no masking), FAR: the far ones of either side, then the near ones;
   // query segments of MASK_SEG tiles
-  __shared__ short qlist[SEGM ? MAXQT : 1];
+  __shared__ short qlist[LIST ? MAXQT : 1];
   __shared__ int qlen[3];
   __shared__ __align__(16) int qsg[MASK == MASK_SEG ? 2 : 1][MASK == MASK_SEG ? BQ : 1];
-  // dense pair masks: the current tile's mask, one bit per (query, key),
-  // 16 keys a word (read once per tile with 16-byte loads)
-  __shared__ uint16_t pmask[MASK == MASK_PAIR ? BQ : 1][MASK == MASK_PAIR ? BKW / 16 : 1];
+  // pair bits: each wave's words of the tile, as dropout's keep words (with
+  // dropout, whose words fill the LDS of two workgroups a CU, each lane holds
+  // its four in registers)
+  constexpr bool PLDS = BITS && !DROP;
+  __shared__ __align__(16) uint32_t Pk0[PLDS ? NW * 64 : 1], Pk1[PLDS ? NW * 64 : 1];
 
   const int tid = threadIdx.x, lane = tid & 63;
   // SCAL: the wave index is known to the compiler as uniform, and the copies'
@@ -104,7 +110,7 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
   // kernels with per-element mask tests need, for more scalar ones, which
   // spill to vector lanes and cost the others up to 6% (dropout at B=12,
   // L=512: 85.7 against 80.8 us).
-  constexpr bool SCAL = FAR || MASK == MASK_SEG || MASK == MASK_PAIR;
+  constexpr bool SCAL = FAR || MASK == MASK_SEG || BITS;
   const int w = SCAL ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
   const int g = (tid & 63) >> 4, c16 = tid & 15;
   // one 16-byte LDS copy: byte offset off (lane part) from the uniform base
@@ -144,7 +150,8 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
   FarSpan fs{kNoFar, -kNoFar};
   if constexpr (FAR) fs = far_span_of(bp);
   auto is_far = [&](int qi) { return FAR && fs.far(qi / (128 / BQ) - kt); };
-  const uint8_t* pkb = (MASK == MASK_PAIR) ? p.pk + (int64_t)b * p.pkb + (int64_t)h * p.pkh : nullptr;
+  int64_t pmask = 0;  // pair bits: the mask of (b, h)
+  if constexpr (BITS) pmask = pair_index(p, b, h);
   const SegView<MASK> sv(p, b);
   T* dsw = (T*)bp.ds + (int64_t)(b * p.H + h) * p.LqP * p.LkP + jw;  // dS column jw, row 0
   const T* qrg = p2c ? (const T*)bp.qrgt + (int64_t)h * D * bp.TGP : nullptr;
@@ -162,7 +169,7 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
     if (SEGM && j < Lk) jseg[jb] = sv(j);
     jkeep[jb] = j < Lk && (!SEGM || jseg[jb] != 0);
   }
-  // Segment masks: the query tiles that meet this key tile (ChunkRange),
+  // Segment masks and pair bits: the query tiles that meet this key tile (ChunkRange; the tile flags),
   // listed by wave 0 (one chunk per lane); the others are neither computed
   // nor written.
   // FAR: the far tiles past neg (queries before the keys) come first, then
@@ -172,8 +179,9 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
   // nothing of the others.
   bool any_key;
   int nlist = nqt, n1 = 0, n2 = 0, qhi = 0;
-  if constexpr (SEGM) {
-    const ChunkRange kr = key_tile_range(bp.cinfo + (int64_t)b * nqt, kt, nqt);
+  if constexpr (LIST) {
+    ChunkRange kr{0, 0, 0};
+    if constexpr (SEGM) kr = key_tile_range(bp.cinfo + (int64_t)b * nqt, kt, nqt);
     if (w == 0) {
       int n = 0;
 #pragma unroll 1
@@ -182,9 +190,15 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
           const int c = c0 + lane;
           bool act = false, full = false;
           if (c < nqt) {
-            const ChunkRange x = chunk_range(bp.cinfo + (int64_t)b * nqt, c);
-            act = x.meets(kr);
-            full = act && x.all && kr.all && x.lo == x.hi && kr.lo == kr.hi && x.lo == kr.lo;
+            if constexpr (SEGM) {
+              const ChunkRange x = chunk_range(bp.cinfo + (int64_t)b * nqt, c);
+              act = x.meets(kr);
+              full = act && x.all && kr.all && x.lo == x.hi && kr.lo == kr.hi && x.lo == kr.lo;
+            } else {
+              const unsigned f = *reinterpret_cast<const uint16_t*>(pair_flags(p, pmask, c) + 2 * kt);
+              act = (f & 0x0101u) != 0;
+              full = (f & 0x0202u) == 0x0202u;
+            }
             if (FAR) act = act && part == (!is_far(c) ? 2 : c / (128 / BQ) < kt ? 0 : 1);
           }
           n = wave_append(act, (short)(c | (full ? 0x4000 : 0)), qlist, n);
@@ -233,18 +247,20 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
   // jw + 16 jb + c16) is bit 16 ib + 4 (2 (w % 2) + jb) + c16 % 4 of the word
   // of forward lane 16 (c16 / 4) + 4 g + e: a lane's four words are 16
   // contiguous bytes.
-  const uint32_t* dropw = nullptr;
+  const uint32_t *dropw = nullptr, *pairw = nullptr;
   const int NKT64 = p.LkP / 64;
+  if constexpr (BITS) pairw = p.pbits + (pmask * nqt * NKT64 + jw / 64) * 64;
   if constexpr (DROP) dropw = p.drop + drop_word0(b, h, p.H, p.LqP / 32, NKT64, 0, jw / 64);
   // Issues the LDS copies of query tile qi into the given buffers (lane
   // order = physical chunk order; Q and dO rows are clamped to Lq - 1, where
   // probabilities are zero anyway), and, with ring set, its qrgt block
   // (whose ring slot was last read two tiles earlier); with dropout, the
   // wave's keep words.
+  uint4 pnext = {0, 0, 0, 0};  // pair bits in registers: the lane's words of the next tile
   int qseg_next = 0;  // MASK_SEG: query segment of lane (w = 1, lane < 32) in the next tile
   // nring: the last blocks of the tile's qrgt window to copy; side: the far
   // side of a far tile, or -1.
-  auto issue = [&](int qi, int nring, int side, T* Qd, T* dOd, BT* Bd, float* Rd, uint32_t* Dd) {
+  auto issue = [&](int qi, int nring, int side, T* Qd, T* dOd, BT* Bd, float* Rd, uint32_t* Dd, uint32_t* Pd) {
     const int i0 = qi * BQ;
     if (MASK == MASK_SEG && w == 1 && lane < BQ) qseg_next = (i0 + lane < Lq) ? sv(i0 + lane) : 0;
 #pragma unroll
@@ -278,6 +294,8 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
         if (nring) issue_ring(tw0 / 32 + qi + 4);
       }
     }
+    if (BITS && !PLDS) pnext = *reinterpret_cast<const uint4*>(pairw + (int64_t)qi * NKT64 * 64 + 16 * (c16 >> 2) + 4 * g);
+    if (PLDS && lane < 16) copy16(pairw + (int64_t)qi * NKT64 * 64, lane * 16, (char*)(Pd + w * 64));
     if (DROP && lane < 16) copy16(dropw + (int64_t)qi * NKT64 * 64, lane * 16, (char*)(Dd + w * 64));
   };
 
@@ -293,7 +311,7 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
     *reinterpret_cast<vec8*>(dsw + (int64_t)(i0 + 16 * mi + c16) * p.LkP + 8 * g) = v;
   };
   if (!any_key) {
-    if (!SEGM)
+    if (!LIST)
       for (int qi = 0; qi < nqt; ++qi)
 #pragma unroll
         for (int mi = 0; mi < BQ / 16; ++mi) store_ds(qi * BQ, mi, vec8{});
@@ -336,7 +354,7 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
     // tw0 / 32) while tile qi is computed; block qi + 5 lands in the sixth
     // slot meanwhile when the next tile is qi + 1.  The first window:
     auto entry = [&](int n) {
-      if constexpr (SEGM) return __builtin_amdgcn_readfirstlane(qlist[n]);
+      if constexpr (LIST) return __builtin_amdgcn_readfirstlane(qlist[n]);
       if constexpr (!FAR) return n;
       return n < n1 ? n : n < n2 ? qhi + n - n1 : n1 + n - n2;
     };
@@ -344,19 +362,19 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
     if (!FAR || n2 == 0) {
       if (p2c)
         for (int r = 0; r < 4; ++r) issue_ring(tw0 / 32 + qfirst + r);
-      issue(qfirst, 1, -1, Qs0, dOs0, Bs0, Rs0, Dk0);
+      issue(qfirst, 1, -1, Qs0, dOs0, Bs0, Rs0, Dk0, Pk0);
     } else {
       // the near part's first tile is to find its buffers first
-      if (n2 & 1) issue(qfirst, 0, n1 > 0 ? 1 : 0, Qs1, dOs1, Bs1, Rs1, Dk1);
-      else issue(qfirst, 0, n1 > 0 ? 1 : 0, Qs0, dOs0, Bs0, Rs0, Dk0);
+      if (n2 & 1) issue(qfirst, 0, n1 > 0 ? 1 : 0, Qs1, dOs1, Bs1, Rs1, Dk1, Pk1);
+      else issue(qfirst, 0, n1 > 0 ? 1 : 0, Qs0, dOs0, Bs0, Rs0, Dk0, Pk0);
     }
     lds_dma_wait();
     // Far tiles, one side at a time: the p2c term of the lane's keys and the
     // column sums of dS (every row of the A operand is ones).
     float fb[2] = {0.f, 0.f};
     f32x4 fcs[2] = {zero4(), zero4()};
-    auto tile = [&](auto farkind, int n, const T* Q, const T* dO, const BT* Bt, const float* R, const uint32_t* Dw, T* nQ, T* ndO,
-                    BT* nBt, float* nR, uint32_t* nDw) {
+    auto tile = [&](auto farkind, int n, const T* Q, const T* dO, const BT* Bt, const float* R, const uint32_t* Dw,
+                    const uint32_t* Pw, T* nQ, T* ndO, BT* nBt, float* nR, uint32_t* nDw, uint32_t* nPw) {
       constexpr bool far = decltype(farkind)::value;
       const int ent = entry(n);
       const int qi = ent & 0x3ff, i0 = qi * BQ;
@@ -366,7 +384,7 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
       vm_wait<NST>();
       if (MASK == MASK_SEG && w == 1 && lane < BQ) qsg[n & 1][lane] = qseg_next;
       __syncthreads();  // ... every wave's, and the previous tile is no longer read
-      if (SEGM && !far && p2c && n > n2) {
+      if (LIST && !far && p2c && n > n2) {
         // after skipped tiles: the blocks of this tile's window not in the
         // ring yet (their slots hold blocks no longer needed)
         const int pv = __builtin_amdgcn_readfirstlane(qlist[n - 1]) & 0x3ff;
@@ -376,37 +394,17 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
           __syncthreads();
         }
       }
+      const uint4 pcur = pnext;
       if (n + 1 < nlist) {
         const int qn = entry(n + 1) & 0x3ff;
-        if constexpr (far) issue(qn, n + 1 == n2 ? 5 : 0, n + 1 < n1 ? 1 : n + 1 < n2 ? 0 : -1, nQ, ndO, nBt, nR, nDw);
-        else issue(qn, qn == qi + 1, -1, nQ, ndO, nBt, nR, nDw);
+        if constexpr (far) issue(qn, n + 1 == n2 ? 5 : 0, n + 1 < n1 ? 1 : n + 1 < n2 ? 0 : -1, nQ, ndO, nBt, nR, nDw, nPw);
+        else issue(qn, qn == qi + 1, -1, nQ, ndO, nBt, nR, nDw, nPw);
       }
       // With segments, a tile whose queries all share the workgroup's single
       // key segment needs no masking beyond the dead-row test.  Other modes:
       // tiles without a kept (query, key) pair store zeros.
-      const bool full = SEGM && (ent & 0x4000);
-      bool skip = !SEGM && i0 >= Lq;
-      if (!skip && MASK == MASK_PAIR) {
-        int keep = 0;
-        const int r = tid >> 3, part = tid & 7;
-        const int i = i0 + r;
-        uint32_t bits = 0;
-        if (i < Lq && pkb[(int64_t)i * p.pkq + i]) {
-          // one 16-byte read of the mask row (rows 16-byte aligned,
-          // host-checked; a 16-key chunk that starts below Lk lies in the
-          // row's allocation), kept as 16 bits in LDS for the tile
-          const int jb0 = j0 + part * (BKW / 8);
-          if (jb0 < Lk) {
-            const uint4 v = *reinterpret_cast<const uint4*>(pkb + (int64_t)i * p.pkq + jb0);
-            const uint32_t wv[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-            for (int q = 0; q < 16; ++q) bits |= ((wv[q >> 2] >> (8 * (q & 3))) & 0xffu) ? (1u << q) : 0u;
-          }
-        }
-        pmask[r][part] = (uint16_t)bits;
-        keep = bits != 0;
-        skip = !__syncthreads_or(keep);
-      }
+      const bool full = LIST && (ent & 0x4000);
+      const bool skip = !LIST && i0 >= Lq;
       if (skip) {
 #pragma unroll
           for (int mi = 0; mi < BQ / 16; ++mi) store_ds(i0, mi, vec8{});
@@ -460,21 +458,27 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
       __builtin_amdgcn_s_setprio(0);
       // ---- P, dP, dS -----------------------------------------------------------------------------
       f32x4 pp[2][BQ / 16], dsh[2][BQ / 16];
-      // dropout: this lane's 16 keep bits, bit 8 ib + 4 jb + e
-      uint32_t dm = 0;
-      if constexpr (DROP) {
-        const uint4 f4 = *reinterpret_cast<const uint4*>(Dw + w * 64 + 16 * (c16 >> 2) + 4 * g);
+      // this lane's 16 bits of a tile's words, bit 8 ib + 4 jb + e: word e,
+      // shifted by 8 (w % 2) + c16 % 4, holds the pair (ib, jb) at bit 16 ib +
+      // 4 jb: bits 0 and 4 stay, bits 16 and 20 move to 8 and 12, then the
+      // word's four bits go to 8 ib + 4 jb + e
+      auto lane_words = [&](const uint32_t* W) {
+        return *reinterpret_cast<const uint4*>(W + w * 64 + 16 * (c16 >> 2) + 4 * g);
+      };
+      auto lane_bits = [&](const uint4& f4) {
         const uint32_t f[4] = {f4.x, f4.y, f4.z, f4.w};
-        // word e, shifted by 8 (w % 2) + c16 % 4, holds the pair (ib, jb) at
-        // bit 16 ib + 4 jb: bits 0 and 4 stay, bits 16 and 20 move to 8
-        // and 12, then the word's four bits go to 8 ib + 4 jb + e
         const int sh = 8 * (w & 1) + (c16 & 3);
+        uint32_t m = 0;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const uint32_t t = f[e] >> sh;
-          dm |= ((t & 0x11u) | ((t >> 8) & 0x1100u)) << e;
+          m |= ((t & 0x11u) | ((t >> 8) & 0x1100u)) << e;
         }
-      }
+        return m;
+      };
+      uint32_t dm = 0, pm = 0;  // dropout's keep bits, the pair mask's
+      if constexpr (DROP) dm = lane_bits(lane_words(Dw));
+      if constexpr (BITS) pm = lane_bits(PLDS ? lane_words(Pw) : pcur);
       auto probs = [&](auto plain) {
         // segment masks: the lane's query segments, four consecutive rows
         // of each 16-row block in one 16-byte LDS read (read per element,
@@ -508,7 +512,7 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
                 bool keep = jkeep[jb] && lr != INFINITY;
                 if (MASK == MASK_SEG && !full)
                   keep = keep && (e == 0 ? qv[ib].x : e == 1 ? qv[ib].y : e == 2 ? qv[ib].z : qv[ib].w) == jseg[jb];
-                if (MASK == MASK_PAIR) keep = keep && ((pmask[il][2 * w + jb] >> c16) & 1u);
+                if constexpr (BITS) keep = keep && (full || ((pm >> (8 * ib + 4 * jb + e)) & 1u));
                 pe = keep ? __builtin_amdgcn_exp2f(__builtin_fmaf(sc[jb][ib][e], sl2, -lr)) : 0.f;
               }
               if constexpr (DROP) {
@@ -526,7 +530,7 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
       // without masking: unmasked tiles inside the sequence, and segment
       // tiles listed as full (every query and key of the tile active and in
       // one segment, so every pair is kept and every row has probabilities)
-      if (!DROP && ((keys_in && i0 + BQ <= Lq) || (MASK == MASK_SEG && full)))
+      if (!DROP && ((keys_in && i0 + BQ <= Lq) || ((MASK == MASK_SEG || BITS) && full)))
         probs(std::true_type{});
       else
         probs(std::false_type{});
@@ -624,8 +628,8 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
           // the parity picks the buffers at run time (the copies are issued
           // from assembly, so the compiler waits for none of them)
           const bool o = (n ^ n2) & 1;
-          tile(std::true_type{}, n, o ? Qs1 : Qs0, o ? dOs1 : dOs0, o ? Bs1 : Bs0, o ? Rs1 : Rs0, o ? Dk1 : Dk0,
-               o ? Qs0 : Qs1, o ? dOs0 : dOs1, o ? Bs0 : Bs1, o ? Rs0 : Rs1, o ? Dk0 : Dk1);
+          tile(std::true_type{}, n, o ? Qs1 : Qs0, o ? dOs1 : dOs0, o ? Bs1 : Bs0, o ? Rs1 : Rs0, o ? Dk1 : Dk0, o ? Pk1 : Pk0,
+               o ? Qs0 : Qs1, o ? dOs0 : dOs1, o ? Bs0 : Bs1, o ? Rs0 : Rs1, o ? Dk0 : Dk1, o ? Pk0 : Pk1);
         }
         if (p2c) {
           cs[side][0] = fcs[0][0], cs[side][1] = fcs[1][0];
@@ -663,8 +667,8 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
     }
     using near_t = std::false_type;
     for (int n = n2; n < nlist; n += 2) {
-      tile(near_t{}, n, Qs0, dOs0, Bs0, Rs0, Dk0, Qs1, dOs1, Bs1, Rs1, Dk1);
-      if (n + 1 < nlist) tile(near_t{}, n + 1, Qs1, dOs1, Bs1, Rs1, Dk1, Qs0, dOs0, Bs0, Rs0, Dk0);
+      tile(near_t{}, n, Qs0, dOs0, Bs0, Rs0, Dk0, Pk0, Qs1, dOs1, Bs1, Rs1, Dk1, Pk1);
+      if (n + 1 < nlist) tile(near_t{}, n + 1, Qs1, dOs1, Bs1, Rs1, Dk1, Pk1, Qs0, dOs0, Bs0, Rs0, Dk0, Pk0);
     }
   }
 

@@ -159,24 +159,30 @@ DSA_DEV void dq_body(const BwdParams& bp, int blk, int nblk, DqLds<T, D>& L) {
     }
   };
 
-  // With a key-padding or segment mask, dS was computed only for the tiles
-  // of 32 queries x 128 keys whose segments can meet (ChunkRange): a key
+  // With a mask, dS was computed only for the tiles of 32 queries x 128 keys
+  // whose segments can meet (ChunkRange) or that hold a kept pair (pair_active): a key
   // tile is visited if one of its 4 query chunks is active, and the rows of
   // inactive chunks are read as zeros.  klist holds kt | (chunk mask << 10).
   int nkt = bp.f.LkP / BK;
-  if (bp.cinfo) {
+  if (bp.cinfo || p.pflag) {
     // listed by wave 0, one key tile per lane
     if (tid < 64) {
       const int nch = bp.f.LqP / 32;
       const int4* ci = bp.cinfo + (int64_t)b * nch;
+      const int64_t pm = p.pflag ? pair_index(p, b, h) : 0;
       int n = 0;
       for (int k0 = 0; k0 < nkt; k0 += 64) {
         const int kt = k0 + tid;
         int mask = 0;
         if (kt < nkt) {
-          const ChunkRange kr = key_tile_range(ci, kt / 2, nch);
+          if (p.pflag) {
 #pragma unroll
-          for (int u = 0; u < BQ / 32; ++u) mask |= chunk_range(ci, i0 / 32 + u).meets(kr) ? (1 << u) : 0;
+            for (int u = 0; u < BQ / 32; ++u) mask |= pair_active(p, pm, i0 / 32 + u, kt / 2) ? (1 << u) : 0;
+          } else {
+            const ChunkRange kr = key_tile_range(ci, kt / 2, nch);
+#pragma unroll
+            for (int u = 0; u < BQ / 32; ++u) mask |= chunk_range(ci, i0 / 32 + u).meets(kr) ? (1 << u) : 0;
+          }
         }
         n = wave_append(mask != 0, (short)(kt | (mask << 10)), klist, n);
       }

@@ -111,8 +111,8 @@ struct TabLds {
 };
 
 // Workgroup blk of nblk (the logical index, whose remainder mod 8 is the
-// XCD it runs on).  LISTED: a key-padding or segment mask is given
-// (bp.cinfo): items without an active part are skipped and partials carry
+// XCD it runs on).  LISTED: a mask is given (bp.cinfo, or the pair mask's
+// flags): items without an active part are skipped and partials carry
 // flags.
 template <typename T, int D, bool LISTED, bool FAR>
 DSA_DEV void table_body(const BwdParams& bp, int blk, int nblk, TabLds<T, D>& L) {
@@ -243,26 +243,28 @@ DSA_DEV void table_body(const BwdParams& bp, int blk, int nblk, TabLds<T, D>& L)
     auto item_mask = [&](int b, int r0) -> int {
       if (!LISTED && !FAR) return 0xff;
       const int4* ci = LISTED ? bp.cinfo + (int64_t)b * nqc : nullptr;
+      const bool pf = LISTED && p.pflag != nullptr;  // pair bits: their flags
+      const int64_t pm = pf ? pair_index(p, b, h) : 0;
       int m = 0;
       if constexpr (!P) {
         const int jc0 = r0 - d0 - DBW, kA = (jc0 >= 0 ? jc0 : jc0 - 127) / 128;
         ChunkRange qc{0, 0, 0};
-        if constexpr (LISTED) qc = chunk_range(ci, r0 / 32);
+        if (LISTED && !pf) qc = chunk_range(ci, r0 / 32);
 #pragma unroll
         for (int u = 0; u < 3; ++u) {
           const int k = kA + u;
           if (k < 0 || k >= nkt128 || 128 * k >= jc0 + DBW + CH || (exf && fs.far(r0 / 128 - k))) continue;
-          if (!LISTED || qc.meets(key_tile_range(ci, k, nqc))) m |= 1 << u;
+          if (!LISTED || (pf ? pair_active(p, pm, r0 / 32, k) : qc.meets(key_tile_range(ci, k, nqc)))) m |= 1 << u;
         }
       } else {
         ChunkRange kr{0, 0, 0};
-        if constexpr (LISTED) kr = key_tile_range(ci, r0 / 128, nqc);
+        if (LISTED && !pf) kr = key_tile_range(ci, r0 / 128, nqc);
         const int cA = (r0 + d0) / 32;  // r0 + d0 is a multiple of 32 (may be negative)
 #pragma unroll
         for (int u = 0; u < PR / 32; ++u) {
           const int c = cA + u;
           if (c < 0 || c >= nqc || (exf && fs.far(c / 4 - r0 / 128))) continue;
-          if (!LISTED || chunk_range(ci, c).meets(kr)) m |= 1 << u;
+          if (!LISTED || (pf ? pair_active(p, pm, c, r0 / 128) : chunk_range(ci, c).meets(kr))) m |= 1 << u;
         }
       }
       return m;

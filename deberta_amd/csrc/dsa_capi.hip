@@ -182,9 +182,17 @@ size_t tables_ks_bytes(const dsa_fwd_args* a) {
 // tables `tab_buf` (NULL: the bands read the caller's tables) and, with
 // dropout, the scratch for its keep bits `drop_buf`.  Arguments already
 // checked.
-int run_fwd(const dsa_fwd_args* a, int* order_buf, void* tab_buf, uint32_t* drop_buf, hipStream_t st) {
+int run_fwd(const dsa_fwd_args* a, int* order_buf, void* tab_buf, uint32_t* drop_buf, void* pair_buf, hipStream_t st) {
   dsa::FwdParams p = to_params(a);
   const int mode = mask_mode(a);
+  dsa::PairBits pairs{};
+  int npair = 0;
+  if (pair_buf) {
+    pairs = fill_pair(a, pair_buf, p);
+    npair = pair_blocks(pairs);
+  } else if (mode == dsa::MASK_PAIR) {
+    p.far = 0;  // the kernels on the mask's bytes look for no far blocks
+  }
   if (drop_buf && launch_dropout_bits(a, drop_buf, p, st)) return 1;
   if (tab_buf && a->flags) {
     dsa::TableKs t;
@@ -211,12 +219,19 @@ int run_fwd(const dsa_fwd_args* a, int* order_buf, void* tab_buf, uint32_t* drop
       dsa::OrderParams2 op;
       int ny = 0;
       const int ncost = fill_orders(p, 1, bufs, nts, kinds, op, ny);
-      hipLaunchKernelGGL(dsa::dsa_fwd_pre_kernel, dim3((unsigned)(ncost + 2 * ncopy)), dim3(256), 0, st, t, op, ncost,
-                         ncopy);
+      hipLaunchKernelGGL(dsa::dsa_fwd_pre_kernel, dim3((unsigned)(ncost + 2 * ncopy)), dim3(256), 0, st, t, op, pairs,
+                         ncost, 0, ncopy);
       if (launch_check("dsa_fwd_pre_kernel")) return 1;
       if (launch_order_sort(op, st)) return 1;
       p.order = order_buf + (int64_t)a->B * fwd_tiles(a);
       order_buf = nullptr;  // done
+    } else if (npair) {
+      // a pair mask's bits in the same launch as the copies
+      dsa::OrderParams2 op{};
+      hipLaunchKernelGGL(dsa::dsa_fwd_pre_kernel, dim3((unsigned)(npair + 2 * ncopy)), dim3(256), 0, st, t, op, pairs, 0,
+                         npair, ncopy);
+      if (launch_check("dsa_fwd_pre_kernel")) return 1;
+      npair = 0;  // done
     } else {
       hipLaunchKernelGGL(dsa::dsa_table_ks_kernel, dim3((unsigned)ncopy, 2), dim3(256), 0, st, t);
       if (launch_check("dsa_table_ks_kernel")) return 1;
@@ -226,6 +241,12 @@ int run_fwd(const dsa_fwd_args* a, int* order_buf, void* tab_buf, uint32_t* drop
     const int64_t hs = (int64_t)(a->D / ks) * R * ks;
     if (has[0]) p.kr = t.dst[0], p.krs[0] = hs, p.krs[1] = ks, p.krk = (int64_t)R * ks;
     if (has[1]) p.qr = t.dst[1], p.qrs[0] = hs, p.qrs[1] = ks, p.qrk = (int64_t)R * ks;
+  }
+  if (npair) {
+    dsa::OrderParams2 op{};
+    hipLaunchKernelGGL(dsa::dsa_fwd_pre_kernel, dim3((unsigned)npair), dim3(256), 0, st, dsa::TableKs{}, op, pairs, 0,
+                       npair, 1);
+    if (launch_check("dsa_fwd_pre_kernel")) return 1;
   }
   if (order_buf) {
     int* bufs[1] = {order_buf};
@@ -440,7 +461,13 @@ int dsa_fwd(const dsa_fwd_args* a, void* stream) {
     if (db) dbits = reinterpret_cast<uint32_t*>(static_cast<char*>(a->workspace) + ob + tb);
   }
   if (a->dropout_threshold && a->dropout_bits) dbits = static_cast<uint32_t*>(a->dropout_bits);
-  return run_fwd(a, buf, tabs, dbits, st);
+  // a pair mask's bits, in the workspace's last part (a workspace without it,
+  // or none: the kernels read the mask's bytes)
+  void* pairs = nullptr;
+  const size_t pb = fwd_pair_bytes(a);
+  if (pb && a->workspace && aligned16(a->workspace) && a->workspace_bytes >= ob + tb + db + pb)
+    pairs = static_cast<char*>(a->workspace) + ob + tb + db;
+  return run_fwd(a, buf, tabs, dbits, pairs, st);
 }
 
 int dsa_fwd_static(const dsa_fwd_args* a, void* stream) {
@@ -450,7 +477,7 @@ int dsa_fwd_static(const dsa_fwd_args* a, void* stream) {
   if (refuse_capture(st, "dsa_fwd_static")) return 1;
   if (a->dropout_threshold)
     return fail("dsa_fwd_static: attention dropout needs dsa_fwd and its workspace (the keep bits)");
-  if (!(a->key_keep || a->seg)) return run_fwd(a, nullptr, nullptr, nullptr, st);  // no scratch used
+  if (!(a->key_keep || a->seg)) return run_fwd(a, nullptr, nullptr, nullptr, nullptr, st);  // no scratch used
   const int64_t n = (int64_t)a->B * fwd_tiles(a);
   if (n > kMaxOrderItems)
     return fail("dsa_fwd_static: B * ceil(Lq / 128) = %lld launch-order items exceed the static scratch's "
@@ -467,7 +494,7 @@ int dsa_fwd_static(const dsa_fwd_args* a, void* stream) {
   int* buf = static_cast<int*>(static_scratch_locked(s));
   if (!buf) return fail("dsa_fwd_static: no address for the static scratch (or its event) on device %d", dev);
   if (hipStreamWaitEvent(st, s.done, 0) != hipSuccess) return fail("dsa_fwd_static: hipStreamWaitEvent failed");
-  const int rc = run_fwd(a, buf, nullptr, nullptr, st);
+  const int rc = run_fwd(a, buf, nullptr, nullptr, nullptr, st);
   if (hipEventRecord(s.done, st) != hipSuccess) {
     (void)hipGetLastError();
     return rc ? rc : fail("dsa_fwd_static: hipEventRecord failed");
@@ -549,7 +576,7 @@ size_t dsa_fwd_dropout_bytes(const dsa_fwd_args* a) {
 size_t dsa_fwd_workspace_bytes(const dsa_fwd_args* a) {
   if (!a || a->B < 1 || a->Lq < 1 || a->H < 1 || a->D < 1) return 0;
   if (a->flags && (a->att_span < 1 || a->att_span > 16383)) return 0;
-  return order_bytes(a, fwd_tiles(a)) + tables_ks_bytes(a) + drop_bytes(a);
+  return order_bytes(a, fwd_tiles(a)) + tables_ks_bytes(a) + drop_bytes(a) + fwd_pair_bytes(a);
 }
 
 size_t dsa_bwd_workspace_bytes(const dsa_bwd_args* a) {

@@ -398,6 +398,8 @@ DSA_DEV const X& pick(const X& a, const X& b) {
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
 
-enum MaskMode { MASK_NONE = 0, MASK_KEY = 1, MASK_PAIR = 2, MASK_SEG = 3 };
+// MASK_PAIR: a dense pair mask read as bytes (the forward without a
+// workspace); MASK_BITS: the same mask as bits and tile flags (dsa_pair.h).
+enum MaskMode { MASK_NONE = 0, MASK_KEY = 1, MASK_PAIR = 2, MASK_SEG = 3, MASK_BITS = 4 };
 
 }  // namespace dsa

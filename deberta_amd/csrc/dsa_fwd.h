@@ -51,13 +51,15 @@ __global__ __launch_bounds__(256, 2) void dsa_fwd_kernel(FwdParams p) {
   __shared__ __align__(16) BT cb_all[NW * CB_ELEMS];
   __shared__ __align__(16) BT pb[PB_ELEMS];
   constexpr bool SEGM = seg_mode(MASK);
+  constexpr bool BITS = MASK == MASK_BITS;
+  constexpr bool LIST = SEGM || BITS;  // the key tiles to visit are listed
   constexpr int MAXKT = 512;  // key tiles (Lk <= 32768)
   __shared__ int segred[SEGM ? 3 * NW : 1];
   __shared__ __align__(16) int ksg[SEGM ? BK : 1];  // key segments of the current tile
-  // segment masks: per key tile, bit 0 = some pair of one segment, bit 1 =
-  // no masking needed; the list of the active tiles in order
-  __shared__ unsigned char kflag[SEGM ? MAXKT : 1];
-  __shared__ short klist[SEGM ? MAXKT : 1];
+  // segment masks and pair bits: per key tile, bit 0 = some pair kept, bit 1
+  // = no masking needed; the list of the active tiles in order
+  __shared__ unsigned char kflag[LIST ? MAXKT : 1];
+  __shared__ short klist[LIST ? MAXKT : 1];
   __shared__ int klen;
   // far blocks (FarSpan), per side: the p2c row, and each query's c2p term
   __shared__ __align__(16) T farq[2][FAR ? D : VEC];
@@ -94,7 +96,7 @@ __global__ __launch_bounds__(256, 2) void dsa_fwd_kernel(FwdParams p) {
   const T* vbase = (const T*)p.v + (int64_t)b * p.vs[0] + (int64_t)h * p.vs[2];
   const T* krh = (p.flags & 1) ? (const T*)p.kr + (int64_t)h * p.krs[0] : nullptr;
   const T* qrh = (p.flags & 2) ? (const T*)p.qr + (int64_t)h * p.qrs[0] : nullptr;
-  const uint8_t* pkb = (MASK == MASK_PAIR) ? p.pk + (int64_t)b * p.pkb + (int64_t)h * p.pkh : nullptr;
+  const uint8_t* pkb = (MASK == MASK_PAIR || BITS) ? p.pk + (int64_t)b * p.pkb + (int64_t)h * p.pkh : nullptr;
   const SegView<MASK> sv(p, b);
 
   // Per-lane query columns (two 16-wide tiles per wave) and their segments.
@@ -109,7 +111,7 @@ __global__ __launch_bounds__(256, 2) void dsa_fwd_kernel(FwdParams p) {
       sq[ib] = sv(irow[ib]);
       live = sq[ib] != 0;
     }
-    if (MASK == MASK_PAIR && valid) live = pkb[(int64_t)irow[ib] * p.pkq + irow[ib]] != 0;
+    if ((MASK == MASK_PAIR || BITS) && valid) live = pkb[(int64_t)irow[ib] * p.pkq + irow[ib]] != 0;
     ilive[ib] = live;
   }
 
@@ -233,6 +235,33 @@ __global__ __launch_bounds__(256, 2) void dsa_fwd_kernel(FwdParams p) {
     __syncthreads();
     nlist = __builtin_amdgcn_readfirstlane(klen);
   }
+  // Pair bits: the same list from the tile flags, wave 0's lanes over the key
+  // tiles.
+  int64_t pmask = 0;
+  if constexpr (BITS) {
+    pmask = pair_index(p, b, h);
+    if (w == 0) {
+      const uint8_t* fl = pair_flags(p, pmask, i0 / 32);
+      int n = 0;
+      for (int c0 = 0; any_live && c0 < nkt; c0 += 64) {
+        const int c = c0 + tid;
+        int any = 0, all = 2;
+        if (c < nkt) {
+#pragma unroll
+          for (int u = 0; u < BQ / 32; ++u) {
+            const int f = fl[u * (p.LkP / 64) + c];
+            any |= f;
+            all &= f;
+          }
+          kflag[c] = (any & 1) | all;
+        }
+        n = wave_append(c < nkt && (any & 1), (short)c, klist, n);
+      }
+      if (tid == 0) klen = n;
+    }
+    __syncthreads();
+    nlist = __builtin_amdgcn_readfirstlane(klen);
+  }
 
   // The next key tile (K and V rows) is fetched into registers while the
   // current one's softmax and PV product run.
@@ -258,6 +287,10 @@ __global__ __launch_bounds__(256, 2) void dsa_fwd_kernel(FwdParams p) {
   // dropout: this lane's keep word of the fetched tile (bit 16 ib + 4 jb + e)
   uint32_t dwn = 0;
   const uint32_t* dropw = nullptr;
+  // pair bits: this lane's word of the fetched tile, laid out alike
+  uint32_t pwn = 0;
+  const uint32_t* pairw = nullptr;
+  if constexpr (BITS) pairw = p.pbits + (pmask * (p.LqP / 32) + iw / 32) * (p.LkP / 64) * 64 + (tid & 63);
   if constexpr (DROP) {
     static_assert(BK == 64 && WQ == 32, "one keep word per lane, 32-query block and 64-key tile");
     dropw = p.drop + drop_word0(b, h, p.H, p.LqP / 32, p.LkP / 64, iw / 32, 0) + (tid & 63);
@@ -265,6 +298,7 @@ __global__ __launch_bounds__(256, 2) void dsa_fwd_kernel(FwdParams p) {
   auto fetch = [&](int kt) {
     const int j0 = kt * BK;
     if constexpr (DROP) dwn = dropw[(int64_t)kt * 64];
+    if constexpr (BITS) pwn = pairw[(int64_t)kt * 64];
     if (p.flags && tid < XG) relv = rel_of_tile(p.rel, i0, j0, Lq, Lk, tid);
     if (SEGM && tid < BK) ksn = j0 + tid < Lk ? sv(j0 + tid) : 0;
     if constexpr (CARRY) {
@@ -289,7 +323,7 @@ __global__ __launch_bounds__(256, 2) void dsa_fwd_kernel(FwdParams p) {
     kfetched = kt;
   };
   if (any_live && nlist > 0) {
-    const int k0 = SEGM ? __builtin_amdgcn_readfirstlane(klist[0]) : 0;
+    const int k0 = LIST ? __builtin_amdgcn_readfirstlane(klist[0]) : 0;
     if constexpr (CARRY) {
       if (p.flags & 2) prel = prel_at(k0);
     }
@@ -303,14 +337,14 @@ __global__ __launch_bounds__(256, 2) void dsa_fwd_kernel(FwdParams p) {
   vm_wait<0>();
 
   for (int n = 0; any_live && n < nlist; ++n) {
-    const int kt = SEGM ? __builtin_amdgcn_readfirstlane(klist[n]) : n;
+    const int kt = LIST ? __builtin_amdgcn_readfirstlane(klist[n]) : n;
     const int j0 = kt * BK;
     // Skip key tiles that every query row of the workgroup masks out: their
     // probabilities are exactly zero (segment masks: the list holds the
     // others).  With segments, a tile whose keys all share the workgroup's
     // single query segment needs no masking at all.
     bool full = false;
-    if constexpr (SEGM) {
+    if constexpr (LIST) {
       full = (kflag[kt] & 2) != 0;
     } else if (MASK == MASK_PAIR) {
       // 16-byte reads of the mask rows (rows 16-byte aligned, host-checked;
@@ -341,8 +375,9 @@ __global__ __launch_bounds__(256, 2) void dsa_fwd_kernel(FwdParams p) {
     // first reuse of a register that an earlier load wrote.
     vm_wait<0>();
     if (kt != kfetched) fetch(kt);  // a tile after skipped ones was not prefetched
-    uint32_t dw = 0;
+    uint32_t dw = 0, pw = 0;
     if constexpr (DROP) dw = dwn;  // the next fetch overwrites dwn
+    if constexpr (BITS) pw = pwn;
 #pragma unroll
     for (int k = 0; k < KCH; ++k) {
       const int c = tid + 256 * k;
@@ -414,8 +449,8 @@ __global__ __launch_bounds__(256, 2) void dsa_fwd_kernel(FwdParams p) {
       btile = kt;
     }
     if (n + 1 < nlist) {
-      const int kn = SEGM ? __builtin_amdgcn_readfirstlane(klist[n + 1]) : n + 1;
-      if constexpr (CARRY && SEGM) {
+      const int kn = LIST ? __builtin_amdgcn_readfirstlane(klist[n + 1]) : n + 1;
+      if constexpr (CARRY && LIST) {
         if ((p.flags & 2) && kn != kt + 1) prel = prel_at(kn);
       }
       fetch(kn);
@@ -424,7 +459,17 @@ __global__ __launch_bounds__(256, 2) void dsa_fwd_kernel(FwdParams p) {
     __builtin_amdgcn_s_setprio(0);
 
     // ---- mask: only where a key or query of the tile can be masked out ------
-    if (MASK == MASK_PAIR || (SEGM && !full) || j0 + BK > Lk) {
+    if constexpr (BITS) {
+      if (!full) {  // the bits hold the rows' liveness and the sequence's ends too
+#pragma unroll
+        for (int ib = 0; ib < 2; ++ib)
+#pragma unroll
+          for (int jb = 0; jb < 4; ++jb)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (!((pw >> (16 * ib + 4 * jb + e)) & 1u)) st[ib][jb][e] = -INFINITY;
+      }
+    } else if (MASK == MASK_PAIR || (SEGM && !full) || j0 + BK > Lk) {
 #pragma unroll
       for (int ib = 0; ib < 2; ++ib) {
         const int i = irow[ib];

@@ -53,10 +53,9 @@ static int round_up(int x, int a) { return (x + a - 1) / a * a; }
 
 static int elem_bytes(int dtype) { return dtype == DSA_BF16 ? 2 : 4; }
 
-// Whether the call's kernels look for far blocks (FarSpan): by its extents,
-// and not under a dense pair mask, whose kernels have no registers left.
+// Whether the call's kernels look for far blocks (FarSpan).
 static bool far_call(const dsa_fwd_args* a) {
-  return !a->pair_keep && dsa::far_wanted(a->flags, round_up(a->Lq, 128), round_up(a->Lk, 128), a->att_span);
+  return dsa::far_wanted(a->flags, round_up(a->Lq, 128), round_up(a->Lk, 128), a->att_span);
 }
 
 static dsa::FwdParams to_params(const dsa_fwd_args* a) {
@@ -105,8 +104,39 @@ static dsa::FwdParams to_params(const dsa_fwd_args* a) {
   p.drop_scale = 1.f;
   p.olo = a->dtype == DSA_BF16 ? a->out_lo : nullptr;
   p.far = far_call(a);
+  p.pbits = nullptr;  // set where the pair mask's bits are made
+  p.pflag = nullptr;
   return p;
 }
+
+// ---- pair masks as bits (dsa_pair.h) ----
+// Bytes of a pair mask's bits and of its tile flags (0 without one).
+static size_t pair_words_bytes(const dsa_fwd_args* a) {
+  if (!a->pair_keep) return 0;
+  const int64_t m = dsa::pair_masks(a->B, a->H, a->pair_keep_strides[0], a->pair_keep_stride_h);
+  return (size_t)m * (round_up(a->Lq, 128) / 32) * (round_up(a->Lk, 128) / 64) * 64 * sizeof(uint32_t);
+}
+static size_t pair_bytes(const dsa_fwd_args* a) {
+  return align_up(pair_words_bytes(a), 256) + align_up(pair_words_bytes(a) / 256, 256);
+}
+// Bytes of them in the forward's workspace: none past the length of its tile
+// lists in LDS (the kernels then read the mask's bytes; the backward's
+// extents end below it).
+constexpr int kMaxPairL = 32768;
+static size_t fwd_pair_bytes(const dsa_fwd_args* a) { return a->Lk <= kMaxPairL ? pair_bytes(a) : 0; }
+// Points the kernels' parameters at the bits in buf and sets up their block.
+static dsa::PairBits fill_pair(const dsa_fwd_args* a, void* buf, dsa::FwdParams& p) {
+  dsa::PairBits t{};
+  t.pk = a->pair_keep;
+  t.pkb = p.pkb, t.pkq = p.pkq, t.pkh = p.pkh;
+  t.bits = static_cast<uint32_t*>(buf);
+  t.flags = static_cast<uint8_t*>(buf) + align_up(pair_words_bytes(a), 256);
+  t.B = p.B, t.H = p.H, t.Lq = p.Lq, t.Lk = p.Lk, t.LqP = p.LqP, t.LkP = p.LkP;
+  p.pbits = t.bits;
+  p.pflag = t.flags;
+  return t;
+}
+static int pair_blocks(const dsa::PairBits& t) { return (int)((dsa::pair_tiles(t) + 3) / 4); }
 
 static int mask_mode(const dsa_fwd_args* a) {
   return a->pair_keep ? dsa::MASK_PAIR : a->key_keep ? dsa::MASK_KEY : a->seg ? dsa::MASK_SEG : dsa::MASK_NONE;
@@ -226,7 +256,9 @@ template <typename T, int D>
 int fwd_mask(const dsa::FwdParams& p, int mode, hipStream_t st) {
   switch (mode) {
     case dsa::MASK_KEY: return launch_fwd<T, D, dsa::MASK_KEY>(p, st);
-    case dsa::MASK_PAIR: return launch_fwd<T, D, dsa::MASK_PAIR>(p, st);
+    case dsa::MASK_PAIR:  // the bits wherever there is room for them (dsa_pair.h has both sides' times)
+      if (p.pflag) return launch_fwd<T, D, dsa::MASK_BITS>(p, st);
+      return launch_fwd<T, D, dsa::MASK_PAIR>(p, st);
     case dsa::MASK_SEG: return launch_fwd<T, D, dsa::MASK_SEG>(p, st);
     default: return launch_fwd<T, D, dsa::MASK_NONE>(p, st);
   }
@@ -247,7 +279,7 @@ static int device_cus() {
 // extents the kernels share.
 struct WsLayout {
   int LqP, LkP, TGP, OFF, NDB, NPG;
-  size_t rowinfo, krgt, qrgt, ds, gpart, farpart, farspan, seg, cinfo, korder, qorder, drop, total;
+  size_t rowinfo, krgt, qrgt, ds, gpart, farpart, farspan, seg, cinfo, pair, korder, qorder, drop, total;
 };
 
 // fp32 elements of the far blocks' table gradient partials (far_part),
@@ -278,7 +310,7 @@ static WsLayout ws_layout(const dsa_bwd_args* a) {
   const int per = f.H * w.NDB;
   const int64_t items = (int64_t)f.B * ((w.LqP > w.LkP ? w.LqP : w.LkP) / 32);
   int64_t groups = (3 * device_cus() / 2 + per - 1) / per;
-  if (w.NDB > 16 || f.key_keep || f.seg) groups = std::max<int64_t>(groups, (items + 63) / 64);
+  if (w.NDB > 16 || f.key_keep || f.seg || f.pair_keep) groups = std::max<int64_t>(groups, (items + 63) / 64);
   w.NPG = (int)std::min<int64_t>(std::max<int64_t>(groups, 1), items);
   size_t off = 0;
   w.rowinfo = off;
@@ -301,6 +333,8 @@ static WsLayout ws_layout(const dsa_bwd_args* a) {
   if (f.flags) off = align_up(off + (size_t)2 * 2 * (2 * f.att_span) * sizeof(int), 256);
   w.cinfo = off;
   if (f.key_keep || f.seg) off = align_up(off + (size_t)f.B * (w.LqP / 32) * 4 * sizeof(int), 256);
+  w.pair = off;
+  off += pair_bytes(&f);
   w.korder = off;  // dkdv launch order (cost, order), under key_keep / seg
   off += order_bytes(&f, w.LkP / dsa::kvcfg::BKW);
   w.qorder = off;  // dq launch order
@@ -319,8 +353,8 @@ int launch_dkdv(const dsa::BwdParams& bp, const WsLayout& ws, int mode, hipStrea
     case dsa::MASK_KEY:
       hipLaunchKernelGGL((dsa::dsa_bwd_dkdv_kernel<T, D, dsa::MASK_KEY, DROP, FAR>), grid, dim3(256), 0, st, bp);
       break;
-    case dsa::MASK_PAIR:  // no far blocks (far_call)
-      hipLaunchKernelGGL((dsa::dsa_bwd_dkdv_kernel<T, D, dsa::MASK_PAIR, DROP, false>), grid, dim3(256), 0, st, bp);
+    case dsa::MASK_PAIR:
+      hipLaunchKernelGGL((dsa::dsa_bwd_dkdv_kernel<T, D, dsa::MASK_BITS, DROP, FAR>), grid, dim3(256), 0, st, bp);
       break;
     case dsa::MASK_SEG:
       hipLaunchKernelGGL((dsa::dsa_bwd_dkdv_kernel<T, D, dsa::MASK_SEG, DROP, FAR>), grid, dim3(256), 0, st, bp);
@@ -342,7 +376,7 @@ int launch_dkdv(const dsa::BwdParams& bp, const WsLayout& ws, int mode, hipStrea
 template <typename T, int D, bool FAR>
 int launch_dq_fold(const dsa::BwdParams& bp, const dsa::BwdParams& tp, int ntab, int ndq, bool dq, bool fold,
                    hipStream_t st) {
-  const bool listed = bp.cinfo != nullptr, qc = bp.f.qc != nullptr;
+  const bool listed = bp.cinfo != nullptr || bp.f.pflag != nullptr, qc = bp.f.qc != nullptr;
   if (fold && dq) {
     const int nt8 = (ntab + 7) / 8 * 8;
     const dim3 grid((unsigned)(nt8 + ndq));
@@ -404,6 +438,8 @@ int launch_bwd(const dsa_bwd_args* a, const WsLayout& ws, int mode, hipStream_t 
   bp.farspan = reinterpret_cast<int*>(base + ws.farspan);
   bp.rowseg = reinterpret_cast<int*>(base + ws.seg);
   bp.cinfo = (f.key_keep || f.seg) ? reinterpret_cast<int4*>(base + ws.cinfo) : nullptr;
+  dsa::PairBits pairs{};
+  if (f.pair_keep) pairs = fill_pair(&f, base + ws.pair, bp.f);
   const int nkt = ws.LkP / dsa::kvcfg::BKW;
   int* kbuf = order_bytes(&f, nkt) ? reinterpret_cast<int*>(base + ws.korder) : nullptr;
   bp.korder = kbuf ? kbuf + (int64_t)f.B * nkt : nullptr;
@@ -455,6 +491,7 @@ int launch_bwd(const dsa_bwd_args* a, const WsLayout& ws, int mode, hipStream_t 
     const int64_t n = (int64_t)f.B * f.H * ws.LqP * (D / (16 / (int)sizeof(T)));
     nb.delta = (int)((n + 255) / 256);
     nb.gather = nb.seg = nb.chunk = nb.zero = 0;
+    nb.pair = f.pair_keep ? pair_blocks(pairs) : 0;
     nb.gacc_floats = 0;
     if (f.key_keep || f.seg) nb.chunk = (int)(((int64_t)f.B * (ws.LqP / 32) + 255) / 256);
     if (f.flags) {
@@ -467,8 +504,8 @@ int launch_bwd(const dsa_bwd_args* a, const WsLayout& ws, int mode, hipStream_t 
       nb.zero = (int)((nb.gacc_floats / 4 + 255) / 256);
     }
     hipLaunchKernelGGL((dsa::dsa_bwd_prep_kernel<T, D>),
-                       dim3((unsigned)(nb.order + nb.gather + nb.seg + nb.chunk + nb.zero + nb.delta)), dim3(256), 0, st,
-                       bp, nb, op);
+                       dim3((unsigned)(nb.order + nb.gather + nb.seg + nb.chunk + nb.zero + nb.pair + nb.delta)),
+                       dim3(256), 0, st, bp, nb, op, pairs);
     if (launch_check("dsa_bwd_prep_kernel")) return 1;
     if (nj && launch_order_sort(op, st)) return 1;
   }

@@ -32,7 +32,7 @@
 // workgroup writes only its own outputs, so the results do not.
 #pragma once
 
-#include "dsa_tiles.h"
+#include "dsa_pair.h"
 
 namespace dsa {
 
@@ -174,15 +174,19 @@ static __global__ __launch_bounds__(256) void dsa_order_cost_kernel(OrderParams2
 }
 
 // The forward's preparation in one launch: its launch-order cost blocks
-// (ncost of them, batch row fastest; none without an order) first, then the
-// k-step copies of the relative tables (ncopy blocks per table; none
-// without the copies).  The sort runs after it (dsa_order_sort_kernel).
-static __global__ __launch_bounds__(256) void dsa_fwd_pre_kernel(TableKs t, OrderParams2 op2, int ncost, int ncopy) {
+// (ncost of them, batch row fastest; none without an order) first, then a
+// pair mask's bits (npair blocks), then the k-step copies of the relative
+// tables (ncopy blocks per table; none without the copies).  The sort runs
+// after it (dsa_order_sort_kernel).
+static __global__ __launch_bounds__(256) void dsa_fwd_pre_kernel(TableKs t, OrderParams2 op2, PairBits pb, int ncost,
+                                                                 int npair, int ncopy) {
   const int blk = blockIdx.x;
   if (blk < ncost) {
     order_cost_block(op2, blk % op2.f.B, blk / op2.f.B, 0);
+  } else if (blk < ncost + npair) {
+    pair_bits_block(pb, blk - ncost);
   } else {
-    const int k = blk - ncost;
+    const int k = blk - ncost - npair;
     table_ks_block(t, k % ncopy, k / ncopy);
   }
 }

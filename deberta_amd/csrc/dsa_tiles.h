@@ -39,6 +39,10 @@ struct FwdParams {
   float drop_scale;
   void* olo;        // bf16 only: O's rounding residual, with out's strides, or null
   int far;          // far blocks are looked for (FarSpan)
+  // a dense pair mask as bits and tile flags (dsa_pair.h), or null:
+  // [masks][LqP / 32][LkP / 64] tiles of 64 words and of one byte
+  const uint32_t* pbits;
+  const uint8_t* pflag;
 };
 
 struct BwdParams {

@@ -102,7 +102,11 @@ typedef struct dsa_fwd_args {
   void* bias;             /* optional [B, H, round_up(Lq, 128), round_up(Lk, 128)]
                              contiguous: the relative score term c2p + p2c
                              (unscaled; fp16 for bf16 inputs, fp32 for fp32),
-                             written for dsa_bwd.  NULL: not written. */
+                             written for dsa_bwd, which reads what a call of
+                             the same extents and masks wrote: tiles a mask
+                             skips and blocks past the tables' saturation on
+                             both sides are left as they are.  NULL: not
+                             written. */
   int64_t q_strides[3];   /* element strides of b, l, h */
   int64_t k_strides[3];
   int64_t v_strides[3];
@@ -122,13 +126,15 @@ typedef struct dsa_fwd_args {
   const int32_t* seg;     /* [B, L] segment ids or NULL (see Masks above) */
   int64_t seg_stride_b;
   /* Optional scratch of dsa_fwd_workspace_bytes(args) bytes (16-byte
-     aligned), for two things: under key_keep or seg, the forward launches
+     aligned), for three things: under key_keep or seg, the forward launches
      its workgroups heaviest first (a small cost and sort pass before the
      kernel); with c2p / p2c, it reads a copy of kr / qr laid out by 64-byte
      k-steps (one small copy kernel), whose row gathers touch half as many
-     cache lines.  NULL (or a scratch of only the launch order's bytes): the
-     default order and the caller's tables, same results.  Ignored by
-     dsa_bwd, which has its own workspace. */
+     cache lines; under pair_keep, the mask as bits and tile flags (one pass
+     over its bytes), so that tiles without a kept pair are skipped.  NULL,
+     or a scratch that ends before one of these parts (in this order): the
+     default order, the caller's tables, the mask's bytes, same results.
+     Ignored by dsa_bwd, which has its own workspace. */
   void* workspace;
   size_t workspace_bytes;
   /* Optional [B, Lq, H, D] (element strides qc_strides, D contiguous): the
@@ -264,8 +270,8 @@ size_t dsa_fwd_bias_bytes(const dsa_fwd_args* args);
  * mask in autograd's saved tensors. */
 size_t dsa_fwd_dropout_bytes(const dsa_fwd_args* args);
 /* Bytes of dsa_fwd_args.workspace for these arguments: the heaviest-first
- * launch order under key_keep or seg, then the k-step copies of kr / qr with
- * c2p / p2c (0 without either).  No counterpart in the reference, whose
+ * launch order under key_keep or seg, the k-step copies of kr / qr with
+ * c2p / p2c, dropout's keep bits, the bits of a pair mask (0 without any).  No counterpart in the reference, whose
  * eager path has no launch order to choose and reads its tables through
  * torch's gathers. */
 size_t dsa_fwd_workspace_bytes(const dsa_fwd_args* args);
