@@ -24,7 +24,7 @@ DSA_STAGE_FOLD = 8
 DSA_STAGE_TABLE = 16  # the first half of FOLD: per-offset sums (workspace)
 DSA_STAGE_SUM = 32  # the second half: their fold onto dkr / dqr
 
-EXPECTED_VERSION = 11
+EXPECTED_VERSION = 12
 
 _i64x3 = ctypes.c_int64 * 3
 _i64x2 = ctypes.c_int64 * 2
@@ -94,6 +94,7 @@ class DsaBwdArgs(ctypes.Structure):
         ("dtab_overwrite", ctypes.c_int32),
         ("dqc", ctypes.c_void_p),
         ("dqc_strides", _i64x3),
+        ("dtab_rows_first", ctypes.c_int32),
     ]
 
 

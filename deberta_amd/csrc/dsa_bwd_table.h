@@ -468,7 +468,7 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_table_kernel(BwdParams bp) {
   table_body<T, D, LISTED, FAR>(bp, blockIdx.x, gridDim.x, L);
 }
 
-// tab[h][r][:] (+)= s * sum over offsets d with row(d) = r of the block
+// tab[h][r][:] (or [r][h][:], dtab_rows) (+)= s * sum over offsets d with row(d) = r of the block
 // accumulators (accumulated into fp32, or written in fp32 or bf16).  WPR
 // waves per (table, h, r), 256 / (64 WPR) rows per workgroup: the WPR * 64
 // / (D/4) parts of a row split the units of its offset range [begin, end)
@@ -550,7 +550,9 @@ __global__ __launch_bounds__(256) void dsa_bwd_fold_kernel(BwdParams bp) {
     for (int k = 1; k < NWV; ++k) acc += wsum[k][c4];
   }
   if (part != 0) return;
-  const int64_t o = ((int64_t)h * R + r) * D + 4 * c4;
+  // dtab_rows: in the order of the projections, which saves the caller a copy
+  // launch of 5 us per table
+  const int64_t o = (bp.dtab_rows ? (int64_t)r * p.H + h : (int64_t)h * R + r) * D + 4 * c4;
   void* tab = q ? bp.dqr : bp.dkr;
   const f32x4 v = acc * p.scale;
   if (bp.dtab_bf16) {

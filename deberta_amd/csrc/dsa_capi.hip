@@ -435,7 +435,7 @@ dsa::rows::RtdParams rtd_params(const dsa_rtd_args* a) {
 
 extern "C" {
 
-int dsa_version(void) { return 11; }
+int dsa_version(void) { return 12; }
 
 const char* dsa_last_error(void) { return g_err.c_str(); }
 

@@ -428,6 +428,7 @@ int launch_bwd(const dsa_bwd_args* a, const WsLayout& ws, int mode, hipStream_t 
   bp.dqr = a->dqr;
   bp.dtab_bf16 = a->dtab_dtype == DSA_BF16;
   bp.dtab_overwrite = a->dtab_overwrite != 0;
+  bp.dtab_rows = a->dtab_rows_first != 0;
   char* base = static_cast<char*>(a->workspace);
   bp.rowinfo = reinterpret_cast<float*>(base + ws.rowinfo);
   bp.krgt = base + ws.krgt;

@@ -57,7 +57,7 @@ struct BwdParams {
   int64_t dqcs[3];
   void* dkr;        // table gradients: fp32 accumulated, or fp32 / bf16 overwritten
   void* dqr;
-  int dtab_bf16, dtab_overwrite;
+  int dtab_bf16, dtab_overwrite, dtab_rows;  // dtab_rows: order [R, H, D] in place of [H, R, D]
   // workspace
   float* rowinfo;   // [B, H, LqP, 2]: lse*log2e (inf: dead or padding row), dO . O; three planes with far blocks
   void* ds;         // dS [B, H, f.LqP, f.LkP] (rows = queries), zero outside [0, Lq) x [0, Lk)

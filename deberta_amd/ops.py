@@ -390,9 +390,11 @@ def fill_bwd_args(
     dropout_t: int = 0,
     dropout_seed: Optional[Tensor] = None,
     dropout_bits: Optional[Tensor] = None,
+    dtab_rows_first: bool = False,
 ) -> _lib.DsaBwdArgs:
     """Backward arguments.  dkr / dqr are fp32 and accumulated into, or, with
-    ``dtab_overwrite``, written (fp32 or bf16, their dtype).  With ``qc``,
+    ``dtab_overwrite``, written (fp32 or bf16, their dtype); their memory is
+    [H, 2A, D] or, with ``dtab_rows_first``, [2A, H, D].  With ``qc``,
     ``dqc`` receives its gradient (the c2p part of dq).  The dropout
     arguments are the forward's (with its keep bits, none are generated;
     without, they are regenerated from the seed)."""
@@ -415,7 +417,23 @@ def fill_bwd_args(
     tab = dkr if dkr is not None else dqr
     a.dtab_dtype = _DTYPES[tab.dtype] if tab is not None else _lib.DSA_F32
     a.dtab_overwrite = int(dtab_overwrite)
+    a.dtab_rows_first = int(dtab_rows_first)
     return a
+
+
+def _rows_first(kr: Optional[Tensor], qr: Optional[Tensor]) -> bool:
+    """Whether the given tables are [2A, H, D] projections seen as
+    [H, 2A, D]: their gradients then take that memory order too, and reach
+    the projection without a copy."""
+    return all(t.stride(0) < t.stride(1) for t in (kr, qr) if t is not None)
+
+
+def _table_grad(like: Tensor, shape: tuple, rows_first: bool) -> Tensor:
+    """An empty [H, 2A, D] gradient in ``like``'s dtype, in either order."""
+    H, R, D = shape
+    if rows_first:
+        return like.new_empty((R, H, D)).permute(1, 0, 2)
+    return like.new_empty((H, R, D))
 
 
 def _alert_nondeterministic_tables() -> None:
@@ -461,7 +479,7 @@ def _dsa_bwd_impl(
     """Gradients (dq, dk, dv, dkr, dqr, dqc).  With ``dqkv`` (a contiguous
     ``[B, L, 3, H, D]`` buffer), dq, dk and dv are written into its three
     slices and returned as views of it.  dkr/dqr are [H, 2A, D] in the
-    tables' dtype (empty when the matching table is None).  ``bias`` is the
+    tables' dtype, their memory in the tables' order (empty when the matching table is None).  ``bias`` is the
     relative term dsa_fwd saved (required with c2p/p2c).  With ``qc`` (the
     c2p term's query rows), dqc is its gradient and dq the content part;
     else dqc is empty.  ``dropout_t`` / ``dropout_seed`` / ``drop_bits``:
@@ -470,6 +488,7 @@ def _dsa_bwd_impl(
     if kr is not None or qr is not None:
         _alert_nondeterministic_tables()
     q, k, v = _kernel_ready(q), _kernel_ready(k), _kernel_ready(v)
+    rows_first = _rows_first(kr, qr)
     kr = None if kr is None else _kernel_ready(kr)
     qr = None if qr is None else _kernel_ready(qr)
     qc = None if qc is None else _kernel_ready(qc)
@@ -487,14 +506,14 @@ def _dsa_bwd_impl(
         dv = torch.empty_like(v, memory_format=torch.contiguous_format)
     # the table gradients are written in the tables' dtype (no zeroing, no cast)
     tab = dict(dtype=q.dtype, device=q.device)
-    dkr = torch.empty((H, R, D), **tab) if kr is not None else torch.empty((0,), **tab)
-    dqr = torch.empty((H, R, D), **tab) if qr is not None else torch.empty((0,), **tab)
+    dkr = _table_grad(q, (H, R, D), rows_first) if kr is not None else torch.empty((0,), **tab)
+    dqr = _table_grad(q, (H, R, D), rows_first) if qr is not None else torch.empty((0,), **tab)
     dqc = torch.empty_like(q, memory_format=torch.contiguous_format) if qc is not None else torch.empty((0,), **tab)
     args = fill_bwd_args(
         dout, q, k, v, kr, qr, rel_table, key_keep, pair_keep, out, lse, bias, att_span, scale,
         dq, dk, dv, dkr if kr is not None else None, dqr if qr is not None else None, dtab_overwrite=True,
         qc=qc, dqc=dqc if qc is not None else None, dropout_t=dropout_t, dropout_seed=dropout_seed,
-        dropout_bits=drop_bits,
+        dropout_bits=drop_bits, dtab_rows_first=rows_first,
     )
     ws = torch.empty((max(bwd_workspace_bytes(args), 16),), dtype=torch.uint8, device=q.device)
     args.workspace = ws.data_ptr()
@@ -516,8 +535,9 @@ def _dsa_bwd_fake(
 ):
     H, D = q.shape[2], q.shape[3]
     R = 2 * int(att_span)
-    dkr = q.new_empty((H, R, D)) if kr is not None else q.new_empty((0,))
-    dqr = q.new_empty((H, R, D)) if qr is not None else q.new_empty((0,))
+    rows_first = _rows_first(kr, qr)
+    dkr = _table_grad(q, (H, R, D), rows_first) if kr is not None else q.new_empty((0,))
+    dqr = _table_grad(q, (H, R, D), rows_first) if qr is not None else q.new_empty((0,))
     dqc = q.new_empty(q.shape) if qc is not None else q.new_empty((0,))
     return (
         q.new_empty(q.shape),

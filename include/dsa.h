@@ -196,8 +196,8 @@ typedef struct dsa_bwd_args {
   int64_t dq_strides[3];
   int64_t dk_strides[3];
   int64_t dv_strides[3];
-  void* dkr;              /* [H, R, D] contiguous; NULL if !C2P */
-  void* dqr;              /* [H, R, D] contiguous; NULL if !P2C */
+  void* dkr;              /* [H, R, D] contiguous (or see dtab_rows_first); NULL if !C2P */
+  void* dqr;              /* likewise; NULL if !P2C */
   /* workspace: dsa_bwd_workspace_bytes() bytes, caller-allocated, in
      ordinary (coarse-grained) device memory such as hipMalloc returns: the
      table-gradient accumulators in it take fp32 atomic adds, which
@@ -213,6 +213,11 @@ typedef struct dsa_bwd_args {
      s sum_j dS_ij k_j.  Unused without fwd.qc. */
   void* dqc;
   int64_t dqc_strides[3];
+  /* Order of dkr / dqr: 0: [H, R, D]; 1: [R, H, D], the gradient of tables
+     that are [R, H, D] projections seen through a permuted view (one store of
+     the fold either way, where the caller's copy into that order takes a
+     launch per table).  (Version 12.) */
+  int32_t dtab_rows_first;
 } dsa_bwd_args;
 
 /* Forward: out = softmax(mask((QK^T + c2p + p2c) * scale)) V and its
