@@ -268,6 +268,10 @@ DSA_DEV void lds_dma16_nt(const void* src, void* lds_wave) {
 }
 // The same copies from a wave-uniform base and a 32-bit byte offset per lane
 // (global_load_lds_dwordx4 with a scalar base: no 64-bit address per lane).
+// The base may come straight from a readfirstlane: a vector memory instruction
+// reads a scalar register that a vector instruction wrote only 5 wait states
+// later (CDNA ISA, manually inserted wait states), and the compiler does not
+// look for that hazard inside inline asm: s_mov_b32 and s_nop 3 are those 5.
 template <typename P>
 DSA_DEV P* uniform_ptr(P* p) {
   const uintptr_t a = (uintptr_t)p;
@@ -279,14 +283,14 @@ DSA_DEV void lds_dma16_s(const void* base, unsigned off, void* lds_wave) {
   base = uniform_ptr(base);
   const unsigned lds =
       __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(__attribute__((address_space(3))) void*)lds_wave);
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds)
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds)
                : "memory", "m0");
 }
 DSA_DEV void lds_dma16_s_nt(const void* base, unsigned off, void* lds_wave) {
   base = uniform_ptr(base);
   const unsigned lds =
       __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(__attribute__((address_space(3))) void*)lds_wave);
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(off), "s"(base), "s"(lds)
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(off), "s"(base), "s"(lds)
                : "memory", "m0");
 }
 // Waits until at most N of this wave's vector-memory instructions are
