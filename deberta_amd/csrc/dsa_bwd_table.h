@@ -475,9 +475,11 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_table_kernel(BwdParams bp) {
 // (from prep_segments), each part with four independent sums so that four
 // loads are in flight; lanes of a part hold 4 columns each.  The parts are
 // summed with lane shuffles and, across waves, through LDS in a fixed
-// order.  Long sequences use WPR = 4: the rows where the relative position
-// saturates then hold thousands of offsets; short ones one wave a row, four
-// rows a workgroup (a quarter of the workgroups to launch).
+// order.  Bound by the launch of its workgroups, most of whose rows hold a few
+// offsets.  Long sequences use WPR = 2, for the rows where the relative
+// position saturates (hundreds of units to sum): 22.2 us with four waves a
+// row, 17.7 with two (B=4, L=2048, H=16); short ones one wave a row, four rows
+// a workgroup.
 template <int D, int WPR>
 __global__ __launch_bounds__(256) void dsa_bwd_fold_kernel(BwdParams bp) {
   using namespace tbcfg;
@@ -540,14 +542,13 @@ __global__ __launch_bounds__(256) void dsa_bwd_fold_kernel(BwdParams bp) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) acc[e] += __shfl_xor(acc[e], m);
   if constexpr (NWV > 1) {
-    __shared__ f32x4 wsum[NWV][Q4];
+    __shared__ f32x4 wsum[4][Q4];
     const int w = threadIdx.x / 64, lane = threadIdx.x % 64;
     if (lane < Q4) wsum[w][lane] = acc;
     __syncthreads();
-    if (w != 0) return;
-    acc = wsum[0][c4];
+    if (w % NWV != 0) return;
 #pragma unroll
-    for (int k = 1; k < NWV; ++k) acc += wsum[k][c4];
+    for (int k = 1; k < NWV; ++k) acc += wsum[w + k][c4];
   }
   if (part != 0) return;
   // dtab_rows: in the order of the projections, which saves the caller a copy

@@ -538,8 +538,8 @@ int launch_bwd(const dsa_bwd_args* a, const WsLayout& ws, int mode, hipStream_t 
   }
   if (sum) {
     const int rows = 2 * f.H * (2 * f.att_span);
-    if (f.Lq + f.Lk > 2048)  // long rows of saturated relative positions: four waves a row
-      hipLaunchKernelGGL((dsa::dsa_bwd_fold_kernel<D, 4>), dim3((unsigned)rows), dim3(256), 0, st, bp);
+    if (f.Lq + f.Lk > 2048)  // long rows of saturated relative positions: two waves a row
+      hipLaunchKernelGGL((dsa::dsa_bwd_fold_kernel<D, 2>), dim3((unsigned)((rows + 1) / 2)), dim3(256), 0, st, bp);
     else  // one wave a row, four rows a workgroup
       hipLaunchKernelGGL((dsa::dsa_bwd_fold_kernel<D, 1>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, st, bp);
     if (launch_check("dsa_bwd_fold_kernel")) return 1;
