@@ -196,12 +196,13 @@ DSA_DEV void prep_zero(const BwdParams& bp, int64_t gacc_floats, int blk) {
 }
 
 struct PrepBlocks {
-  int order, order_ny, gather, seg, chunk, zero, pair, delta;
+  int order, order_ny, span, gather, seg, chunk, zero, pair, delta;
   int64_t gacc_floats;
 };
 // Blocks: the launch orders' cost blocks (dsa_order.h; batch row fastest,
-// then the tile group, then the job) first, then gather, segments, chunk
-// summaries, zeroing, a pair mask's bits and rowinfo.
+// then the tile group, then the job) first, then the far blocks' span (one
+// block with them), gather, segments, chunk summaries, zeroing, a pair mask's
+// bits and rowinfo.
 template <typename T, int D>
 __global__ __launch_bounds__(256) void dsa_bwd_prep_kernel(BwdParams bp, PrepBlocks nb, OrderParams2 op2, PairBits pb) {
   if ((int)blockIdx.x < nb.order) {
@@ -209,14 +210,16 @@ __global__ __launch_bounds__(256) void dsa_bwd_prep_kernel(BwdParams bp, PrepBlo
     order_cost_block(op2, k % B, (k / B) % nb.order_ny, k / (B * nb.order_ny));
     return;
   }
-  const int blk = blockIdx.x - nb.order;
+  if ((int)blockIdx.x < nb.order + nb.span) {
+    __shared__ __align__(16) int red[8];
+    const FarSpan fs = far_span(bp.f, red);
+    if (threadIdx.x == 0) bp.farspan[0] = fs.pos, bp.farspan[1] = fs.neg;
+    return;
+  }
+  const int blk = blockIdx.x - nb.order - nb.span;
   if (blk < nb.gather) {
     prep_gather<T, D>(bp, blk);
   } else if (blk < nb.gather + nb.seg) {
-    if (bp.f.far && blk == nb.gather && threadIdx.x < 64) {
-      const FarSpan fs = far_span(bp.f);
-      if (threadIdx.x == 0) bp.farspan[0] = fs.pos, bp.farspan[1] = fs.neg;
-    }
     prep_segments(bp, blk - nb.gather);
   } else if (blk < nb.gather + nb.seg + nb.chunk) {
     prep_chunks(bp, blk - nb.gather - nb.seg);

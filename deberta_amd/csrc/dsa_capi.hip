@@ -179,10 +179,12 @@ size_t tables_ks_bytes(const dsa_fwd_args* a) {
 
 // The forward with the launch-order scratch `order_buf` (NULL: no
 // heaviest-first order), the scratch for the k-step copies of the relative
-// tables `tab_buf` (NULL: the bands read the caller's tables) and, with
-// dropout, the scratch for its keep bits `drop_buf`.  Arguments already
-// checked.
-int run_fwd(const dsa_fwd_args* a, int* order_buf, void* tab_buf, uint32_t* drop_buf, void* pair_buf, hipStream_t st) {
+// tables `tab_buf` (NULL: the bands read the caller's tables), with dropout
+// the scratch for its keep bits `drop_buf`, under a pair mask the one for its
+// bits `pair_buf` (NULL: its bytes) and the one for the far blocks' span
+// `span_buf` (NULL: each workgroup finds it).  Arguments already checked.
+int run_fwd(const dsa_fwd_args* a, int* order_buf, void* tab_buf, uint32_t* drop_buf, void* pair_buf, int* span_buf,
+            hipStream_t st) {
   dsa::FwdParams p = to_params(a);
   const int mode = mask_mode(a);
   dsa::PairBits pairs{};
@@ -193,6 +195,8 @@ int run_fwd(const dsa_fwd_args* a, int* order_buf, void* tab_buf, uint32_t* drop
   } else if (mode == dsa::MASK_PAIR) {
     p.far = 0;  // the kernels on the mask's bytes look for no far blocks
   }
+  if (!p.far) span_buf = nullptr;
+  const int nspan = span_buf ? 1 : 0;
   if (drop_buf && launch_dropout_bits(a, drop_buf, p, st)) return 1;
   if (tab_buf && a->flags) {
     dsa::TableKs t;
@@ -219,17 +223,18 @@ int run_fwd(const dsa_fwd_args* a, int* order_buf, void* tab_buf, uint32_t* drop
       dsa::OrderParams2 op;
       int ny = 0;
       const int ncost = fill_orders(p, 1, bufs, nts, kinds, op, ny);
-      hipLaunchKernelGGL(dsa::dsa_fwd_pre_kernel, dim3((unsigned)(ncost + 2 * ncopy)), dim3(256), 0, st, t, op, pairs,
-                         ncost, 0, ncopy);
+      hipLaunchKernelGGL(dsa::dsa_fwd_pre_kernel, dim3((unsigned)(nspan + ncost + 2 * ncopy)), dim3(256), 0, st, t, op,
+                         pairs, ncost, 0, ncopy, span_buf);
       if (launch_check("dsa_fwd_pre_kernel")) return 1;
       if (launch_order_sort(op, st)) return 1;
       p.order = order_buf + (int64_t)a->B * fwd_tiles(a);
       order_buf = nullptr;  // done
-    } else if (npair) {
-      // a pair mask's bits in the same launch as the copies
+    } else if (npair || span_buf) {
+      // a pair mask's bits and the far blocks' span in the same launch as the copies
       dsa::OrderParams2 op{};
-      hipLaunchKernelGGL(dsa::dsa_fwd_pre_kernel, dim3((unsigned)(npair + 2 * ncopy)), dim3(256), 0, st, t, op, pairs, 0,
-                         npair, ncopy);
+      op.f = p;
+      hipLaunchKernelGGL(dsa::dsa_fwd_pre_kernel, dim3((unsigned)(nspan + npair + 2 * ncopy)), dim3(256), 0, st, t, op,
+                         pairs, 0, npair, ncopy, span_buf);
       if (launch_check("dsa_fwd_pre_kernel")) return 1;
       npair = 0;  // done
     } else {
@@ -239,13 +244,14 @@ int run_fwd(const dsa_fwd_args* a, int* order_buf, void* tab_buf, uint32_t* drop
     // the bands read the copies: head stride NS * R * KS, row stride KS,
     // k-step stride R * KS
     const int64_t hs = (int64_t)(a->D / ks) * R * ks;
+    p.span = span_buf;
     if (has[0]) p.kr = t.dst[0], p.krs[0] = hs, p.krs[1] = ks, p.krk = (int64_t)R * ks;
     if (has[1]) p.qr = t.dst[1], p.qrs[0] = hs, p.qrs[1] = ks, p.qrk = (int64_t)R * ks;
   }
   if (npair) {
     dsa::OrderParams2 op{};
     hipLaunchKernelGGL(dsa::dsa_fwd_pre_kernel, dim3((unsigned)npair), dim3(256), 0, st, dsa::TableKs{}, op, pairs, 0,
-                       npair, 1);
+                       npair, 1, (int*)nullptr);
     if (launch_check("dsa_fwd_pre_kernel")) return 1;
   }
   if (order_buf) {
@@ -467,7 +473,12 @@ int dsa_fwd(const dsa_fwd_args* a, void* stream) {
   const size_t pb = fwd_pair_bytes(a);
   if (pb && a->workspace && aligned16(a->workspace) && a->workspace_bytes >= ob + tb + db + pb)
     pairs = static_cast<char*>(a->workspace) + ob + tb + db;
-  return run_fwd(a, buf, tabs, dbits, pairs, st);
+  // and the far blocks' span after it
+  int* span = nullptr;
+  const size_t sb = fwd_span_bytes(a);
+  if (sb && a->workspace && aligned16(a->workspace) && a->workspace_bytes >= ob + tb + db + pb + sb)
+    span = reinterpret_cast<int*>(static_cast<char*>(a->workspace) + ob + tb + db + pb);
+  return run_fwd(a, buf, tabs, dbits, pairs, span, st);
 }
 
 int dsa_fwd_static(const dsa_fwd_args* a, void* stream) {
@@ -477,7 +488,7 @@ int dsa_fwd_static(const dsa_fwd_args* a, void* stream) {
   if (refuse_capture(st, "dsa_fwd_static")) return 1;
   if (a->dropout_threshold)
     return fail("dsa_fwd_static: attention dropout needs dsa_fwd and its workspace (the keep bits)");
-  if (!(a->key_keep || a->seg)) return run_fwd(a, nullptr, nullptr, nullptr, nullptr, st);  // no scratch used
+  if (!(a->key_keep || a->seg)) return run_fwd(a, nullptr, nullptr, nullptr, nullptr, nullptr, st);  // no scratch used
   const int64_t n = (int64_t)a->B * fwd_tiles(a);
   if (n > kMaxOrderItems)
     return fail("dsa_fwd_static: B * ceil(Lq / 128) = %lld launch-order items exceed the static scratch's "
@@ -494,7 +505,7 @@ int dsa_fwd_static(const dsa_fwd_args* a, void* stream) {
   int* buf = static_cast<int*>(static_scratch_locked(s));
   if (!buf) return fail("dsa_fwd_static: no address for the static scratch (or its event) on device %d", dev);
   if (hipStreamWaitEvent(st, s.done, 0) != hipSuccess) return fail("dsa_fwd_static: hipStreamWaitEvent failed");
-  const int rc = run_fwd(a, buf, nullptr, nullptr, nullptr, st);
+  const int rc = run_fwd(a, buf, nullptr, nullptr, nullptr, nullptr, st);
   if (hipEventRecord(s.done, st) != hipSuccess) {
     (void)hipGetLastError();
     return rc ? rc : fail("dsa_fwd_static: hipEventRecord failed");
@@ -576,7 +587,8 @@ size_t dsa_fwd_dropout_bytes(const dsa_fwd_args* a) {
 size_t dsa_fwd_workspace_bytes(const dsa_fwd_args* a) {
   if (!a || a->B < 1 || a->Lq < 1 || a->H < 1 || a->D < 1) return 0;
   if (a->flags && (a->att_span < 1 || a->att_span > 16383)) return 0;
-  return order_bytes(a, fwd_tiles(a)) + tables_ks_bytes(a) + drop_bytes(a) + fwd_pair_bytes(a);
+  return order_bytes(a, fwd_tiles(a)) + tables_ks_bytes(a) + drop_bytes(a) + fwd_pair_bytes(a) +
+         fwd_span_bytes(a);
 }
 
 size_t dsa_bwd_workspace_bytes(const dsa_bwd_args* a) {

@@ -64,6 +64,7 @@ __global__ __launch_bounds__(256, 2) void dsa_fwd_kernel(FwdParams p) {
   // far blocks (FarSpan), per side: the p2c row, and each query's c2p term
   __shared__ __align__(16) T farq[2][FAR ? D : VEC];
   __shared__ float fara[2][FAR ? BQ : 1];
+  __shared__ __align__(16) int farred[FAR ? 8 : 1];
 
   const int tid = threadIdx.x;
   const int w = tid >> 6, g = (tid & 63) >> 4, c16 = tid & 15;
@@ -135,7 +136,8 @@ __global__ __launch_bounds__(256, 2) void dsa_fwd_kernel(FwdParams p) {
 
   FarSpan fs{kNoFar, -kNoFar};
   if constexpr (FAR) {
-    fs = far_span(p);
+    if (p.span) fs = FarSpan{__builtin_amdgcn_readfirstlane(p.span[0]), __builtin_amdgcn_readfirstlane(p.span[1])};
+    else fs = far_span(p, farred);
 #pragma unroll
     for (int side = 0; side < 2; ++side) {
       const int e = far_offset(p, side);

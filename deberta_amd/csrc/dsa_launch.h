@@ -104,6 +104,7 @@ static dsa::FwdParams to_params(const dsa_fwd_args* a) {
   p.drop_scale = 1.f;
   p.olo = a->dtype == DSA_BF16 ? a->out_lo : nullptr;
   p.far = far_call(a);
+  p.span = nullptr;  // set where the span is found before the kernel
   p.pbits = nullptr;  // set where the pair mask's bits are made
   p.pflag = nullptr;
   return p;
@@ -124,6 +125,8 @@ static size_t pair_bytes(const dsa_fwd_args* a) {
 // extents end below it).
 constexpr int kMaxPairL = 32768;
 static size_t fwd_pair_bytes(const dsa_fwd_args* a) { return a->Lk <= kMaxPairL ? pair_bytes(a) : 0; }
+// Bytes of the far blocks' span in the forward's workspace.
+static size_t fwd_span_bytes(const dsa_fwd_args* a) { return far_call(a) ? 256 : 0; }
 // Points the kernels' parameters at the bits in buf and sets up their block.
 static dsa::PairBits fill_pair(const dsa_fwd_args* a, void* buf, dsa::FwdParams& p) {
   dsa::PairBits t{};
@@ -486,6 +489,7 @@ int launch_bwd(const dsa_bwd_args* a, const WsLayout& ws, int mode, hipStream_t 
     op.f = bp.f;
     op.njobs = 0;
     dsa::PrepBlocks nb;
+    nb.span = bp.f.far ? 1 : 0;
     nb.order = 0;
     nb.order_ny = 1;
     if (nj) nb.order = fill_orders(bp.f, nj, bufs, nts, kinds, op, nb.order_ny);
@@ -505,7 +509,7 @@ int launch_bwd(const dsa_bwd_args* a, const WsLayout& ws, int mode, hipStream_t 
       nb.zero = (int)((nb.gacc_floats / 4 + 255) / 256);
     }
     hipLaunchKernelGGL((dsa::dsa_bwd_prep_kernel<T, D>),
-                       dim3((unsigned)(nb.order + nb.gather + nb.seg + nb.chunk + nb.zero + nb.pair + nb.delta)),
+                       dim3((unsigned)(nb.order + nb.span + nb.gather + nb.seg + nb.chunk + nb.zero + nb.pair + nb.delta)),
                        dim3(256), 0, st, bp, nb, op, pairs);
     if (launch_check("dsa_bwd_prep_kernel")) return 1;
     if (nj && launch_order_sort(op, st)) return 1;

@@ -176,12 +176,18 @@ static __global__ __launch_bounds__(256) void dsa_order_cost_kernel(OrderParams2
 // The forward's preparation in one launch: its launch-order cost blocks
 // (ncost of them, batch row fastest; none without an order) first, then a
 // pair mask's bits (npair blocks), then the k-step copies of the relative
-// tables (ncopy blocks per table; none without the copies).  The sort runs
-// after it (dsa_order_sort_kernel).
+// tables (ncopy blocks per table; none without the copies) and, with span,
+// the far blocks' span (FarSpan, from op2.f's table).  The sort runs after it
+// (dsa_order_sort_kernel).
 static __global__ __launch_bounds__(256) void dsa_fwd_pre_kernel(TableKs t, OrderParams2 op2, PairBits pb, int ncost,
-                                                                 int npair, int ncopy) {
-  const int blk = blockIdx.x;
-  if (blk < ncost) {
+                                                                 int npair, int ncopy, int* span) {
+  // (span first: its block takes the longest)
+  const int blk = (int)blockIdx.x - (span ? 1 : 0);
+  if (blk < 0) {
+    __shared__ __align__(16) int red[8];
+    const FarSpan fs = far_span(op2.f, red);
+    if (threadIdx.x == 0) span[0] = fs.pos, span[1] = fs.neg;
+  } else if (blk < ncost) {
     order_cost_block(op2, blk % op2.f.B, blk / op2.f.B, 0);
   } else if (blk < ncost + npair) {
     pair_bits_block(pb, blk - ncost);

@@ -39,6 +39,7 @@ struct FwdParams {
   float drop_scale;
   void* olo;        // bf16 only: O's rounding residual, with out's strides, or null
   int far;          // far blocks are looked for (FarSpan)
+  const int* span;  // far: the call's FarSpan, found before the kernel, or null (the kernel finds it)
   // a dense pair mask as bits and tile flags (dsa_pair.h), or null:
   // [masks][LqP / 32][LkP / 64] tiles of 64 words and of one byte
   const uint32_t* pbits;
@@ -174,12 +175,13 @@ DSA_DEV SegRange wg_seg_range(int s, bool has, int* red) {
 
 // Far blocks: the 128-query x 128-key blocks (query block qt, key block kt)
 // whose offsets all read one c2p row and one p2c row, because the relative
-// position saturates there.  The rows are monotone in the offset, so block
-// diagonal delta = qt - kt >= 1 is far iff its smallest offset, 128 delta -
-// 127, has the rows of the largest offset of the call, Lq - 1; then every
-// larger delta is far too, and likewise for delta <= -1 with -(Lk - 1).  In
-// a far block the relative term of pair (i, j) is a_i + b_j with a_i = q_i .
-// Kr[c] and b_j = k_j . Qr[p] of the one row pair, so no band is computed,
+// position saturates there: block diagonal delta = qt - kt >= 1 is far iff
+// every offset from its smallest, 128 delta - 127, to the largest of the
+// call, Lq - 1, has the same rows (so every larger delta is far too), and
+// likewise delta <= -1 with -(Lk - 1).  Every offset is looked at, so a table
+// that is not monotone has no far block that is none.  In a far block the
+// relative term of pair (i, j) is a_i + b_j with a_i = q_i . Kr[c] and b_j =
+// k_j . Qr[p] of the one row pair, so no band is computed,
 // gathered, saved or read back: the products of a tile fall to those of
 // plain attention, its gradients to one row and one column sum of dS (s_i,
 // t_j):
@@ -187,8 +189,10 @@ DSA_DEV SegRange wg_seg_range(int s, bool has, int* red) {
 // At position buckets 256 / max_position 512 delta >= 5 is far: 52% of the
 // blocks at L = 2048, 74% at L = 4096.  Whether blocks can be far is decided
 // on the host from the extents (far_wanted), so shorter calls search nothing.
-// The forward finds the span itself, the backward's prep kernel finds the
-// same one from the same table for the kernels after it.
+// One workgroup of the preparation before the forward, and one of the
+// backward's prep kernel, find the span for the kernels after them (2 us at
+// L = 4096, beside the preparation's other blocks); a forward without a
+// workspace finds it in each of its workgroups.
 constexpr int kNoFar = 1 << 26;  // a block diagonal past every call's (and 4x it, the 32-query tiles, in range)
 struct FarSpan {
   int pos, neg;  // far iff delta >= pos or delta <= neg
@@ -212,31 +216,35 @@ DSA_DEV int offset_row(const int32_t* rel, int d, int Lq, int Lk, int A, bool p2
   return p2c ? p2c_row(t, A) : c2p_row(t, A);
 }
 
-// Every lane of the wave calls it (one block diagonal a lane); the result is
-// uniform.
-DSA_DEV FarSpan far_span(const FwdParams& p) {
+// The span, searched by a workgroup of 256 threads, all of which call it (red:
+// 8 ints of LDS); the result is uniform.
+DSA_DEV FarSpan far_span(const FwdParams& p, int* red) {
   FarSpan s{kNoFar, -kNoFar};
   if (!p.far) return s;
-  const int lane = threadIdx.x & 63;
+  int last[2];  // the furthest offset of a side whose rows differ from the end's
 #pragma unroll
   for (int side = 0; side < 2; ++side) {
-    const int n = (side == 0 ? p.LqP : p.LkP) / 128;
-    const int e = far_offset(p, side);
+    const int e = far_offset(p, side), n = side == 0 ? e : -e;
     const int ce = offset_row(p.rel, e, p.Lq, p.Lk, p.A, false), pe = offset_row(p.rel, e, p.Lq, p.Lk, p.A, true);
-    for (int d0 = 1; d0 < n; d0 += 64) {
-      const int d = d0 + lane;
-      const int o = side == 0 ? 128 * d - 127 : -(128 * d - 127);
-      const bool ok = d < n && (!(p.flags & 1) || offset_row(p.rel, o, p.Lq, p.Lk, p.A, false) == ce) &&
-                      (!(p.flags & 2) || offset_row(p.rel, o, p.Lq, p.Lk, p.A, true) == pe);
-      const unsigned long long m = __ballot(ok);
-      if (m) {
-        const int f = d0 + __builtin_ctzll(m);
-        if (side == 0) s.pos = f;
-        else s.neg = -f;
-        break;
-      }
+    int m = 0;
+#pragma unroll 8
+    for (int o = 1 + (int)threadIdx.x; o < n; o += 256) {
+      const int t = min(max(p.rel[(side == 0 ? o : -o) + p.Lk - 1], -p.A), p.A);
+      if (((p.flags & 1) && c2p_row(t, p.A) != ce) || ((p.flags & 2) && p2c_row(t, p.A) != pe)) m = o;
     }
+#pragma unroll
+    for (int k = 32; k >= 1; k >>= 1) m = max(m, __shfl_xor(m, k));
+    last[side] = m;
   }
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = last[0], red[4 + (threadIdx.x >> 6)] = last[1];
+  __syncthreads();
+  const int4 a = *reinterpret_cast<const int4*>(red), b = *reinterpret_cast<const int4*>(red + 4);
+  __syncthreads();
+  // the first diagonal whose smallest offset is past it
+  const int dp = (max(max(a.x, a.y), max(a.z, a.w)) + 127) / 128 + 1;
+  const int dn = (max(max(b.x, b.y), max(b.z, b.w)) + 127) / 128 + 1;
+  if (dp < p.LqP / 128) s.pos = __builtin_amdgcn_readfirstlane(dp);
+  if (dn < p.LkP / 128) s.neg = -__builtin_amdgcn_readfirstlane(dn);
   return s;
 }
 

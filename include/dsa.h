@@ -33,6 +33,9 @@
  *     column and row.  The kernels derive the c2p row clamp(clamp(t,-A,A)+A,
  *     0, 2A-1) and the p2c row clamp(-clamp(t,-A,A)+A, 0, 2A-1) in registers
  *     (deberta_v2_native.py:377, 395, 407).
+ *     The table may hold any values; dkr and dqr need it non-decreasing in
+ *     i - j (a table row's offsets are then one range), as every table of
+ *     the reference is.
  *   - Masks: key_keep is a [B, Lk] byte mask (nonzero = keep) for the
  *     reference's broadcast (B,1,1,S) keep mask; pair_keep is a [B, Lq, Lk]
  *     byte mask for the pairwise (B,1,S,S) form, or [B, H, Lq, Lk] for a
@@ -126,14 +129,16 @@ typedef struct dsa_fwd_args {
   const int32_t* seg;     /* [B, L] segment ids or NULL (see Masks above) */
   int64_t seg_stride_b;
   /* Optional scratch of dsa_fwd_workspace_bytes(args) bytes (16-byte
-     aligned), for three things: under key_keep or seg, the forward launches
+     aligned), for four things: under key_keep or seg, the forward launches
      its workgroups heaviest first (a small cost and sort pass before the
      kernel); with c2p / p2c, it reads a copy of kr / qr laid out by 64-byte
      k-steps (one small copy kernel), whose row gathers touch half as many
      cache lines; under pair_keep, the mask as bits and tile flags (one pass
-     over its bytes), so that tiles without a kept pair are skipped.  NULL,
-     or a scratch that ends before one of these parts (in this order): the
-     default order, the caller's tables, the mask's bytes, same results.
+     over its bytes), so that tiles without a kept pair are skipped; in long
+     calls, where the tables' saturation on either side begins (one pass over
+     rel_table).  NULL, or a scratch that ends before one of these parts (in
+     this order): the default order, the caller's tables, the mask's bytes,
+     the search in each workgroup, same results.
      Ignored by dsa_bwd, which has its own workspace. */
   void* workspace;
   size_t workspace_bytes;

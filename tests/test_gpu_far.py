@@ -14,7 +14,7 @@ import math
 import pytest
 import torch
 
-from tests._cases import Case
+from tests._cases import Case, make_inputs
 from tests.test_gpu_parity import _check
 
 pytestmark = pytest.mark.gpu
@@ -100,3 +100,46 @@ def test_far_stage_split(Lq, Lk, p2p, dtype, gpu):
                 assert err <= 1e-5, (calls, name, err)
             else:
                 assert torch.equal(got[name], b), (calls, name)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("mask", ["none", "key"])
+def test_far_table_not_monotone(mask, dtype, gpu):
+    """A table that comes back to its end's rows on every block diagonal but
+    not on the offsets between them has no far block: out, dq, dk and dv are
+    those of any Toeplitz table (dkr and dqr need a monotone one).  The forward
+    without a workspace searches in its workgroups: equal to the last bit."""
+    from deberta_amd import _lib, ops
+    from deberta_amd.masks import kernel_masks
+    from oracle import eager
+
+    c = Case(B=2, H=2, L=514, D=64, buckets=32, max_pos=64, mask=mask, seed=21)
+    x = make_inputs(c)
+    d = torch.arange(-(c.L - 1), c.L)
+    table = (d + 32) % 64 - 32
+    i = torch.arange(c.L)
+    leaf = lambda t: t.to(dtype).float().requires_grad_()
+    hm = lambda t: t.permute(0, 2, 1, 3)
+    rq, rk, rv, rkr, rqr = (leaf(x[n]) for n in ("q", "k", "v", "kr", "qr"))
+    ctx, _ = eager.attend(
+        hm(rq), hm(rk), hm(rv), rkr, rqr, table[i[:, None] - i[None] + c.L - 1], x["mask"], types=c.type_list,
+        att_span=c.A, use_relative=True,
+    )
+    ref = [ctx, *torch.autograd.grad(ctx, [rq, rk, rv], hm(x["dout"].to(dtype).float()))]
+
+    q, k, v, kr, qr = (x[n].to(gpu, dtype).requires_grad_() for n in ("q", "k", "v", "kr", "qr"))
+    rel = table.to(gpu, torch.int32)
+    kk, _ = kernel_masks(None if x["mask"] is None else x["mask"].to(gpu), c.B, c.L, c.L, gpu)
+    scale = 1 / math.sqrt(3 * c.D)
+    out, lse, _, _ = torch.ops.deberta_amd.dsa_fwd(q, k, v, kr, qr, rel, kk, None, c.A, scale, True)
+    got = [hm(out), *torch.autograd.grad(out, [q, k, v], x["dout"].to(gpu, dtype))]
+    for name, a, b in zip(("out", "dq", "dk", "dv"), got, ref):
+        err = float((a.detach().float().cpu() - b).abs().max())
+        tol = 2e-2 if dtype == torch.bfloat16 else 1e-4 * float(b.abs().max())
+        assert err <= tol, (name, err)
+
+    out2, lse2 = torch.full_like(out, float("nan")), torch.full_like(lse, float("nan"))
+    a = ops._fill_fwd_args(q, k, v, kr, qr, rel, kk, None, out2, lse2, c.A, scale)
+    _lib.check(_lib.load().dsa_fwd(ctypes.byref(a), ctypes.c_void_p(torch.cuda.current_stream(gpu).cuda_stream)), "dsa_fwd")
+    torch.cuda.synchronize(gpu)
+    assert torch.equal(out2, out) and torch.equal(lse2, lse)
