@@ -94,8 +94,10 @@ DSA_DEV void prep_delta(const BwdParams& bp, int blk) {
     *reinterpret_cast<float2*>(bp.rowinfo + 2 * row) = make_float2(lse2, acc);
     if (p.far) {
       const float sl2 = p.scale * kLog2e;
-      *reinterpret_cast<float2*>(bp.rowinfo + 2 * (n + row)) = make_float2(lse2 - fa[0] * sl2, acc);
-      *reinterpret_cast<float2*>(bp.rowinfo + 2 * (2 * n + row)) = make_float2(lse2 - fa[1] * sl2, acc);
+#pragma unroll
+      for (int s = 0; s < 2; ++s)  // (rows without probabilities stay marked, whatever their q . Kr)
+        *reinterpret_cast<float2*>(bp.rowinfo + 2 * ((1 + s) * n + row)) =
+            make_float2(lse2 == INFINITY ? INFINITY : lse2 - fa[s] * sl2, acc);
     }
   }
 }

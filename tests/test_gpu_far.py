@@ -143,3 +143,54 @@ def test_far_table_not_monotone(mask, dtype, gpu):
     _lib.check(_lib.load().dsa_fwd(ctypes.byref(a), ctypes.c_void_p(torch.cuda.current_stream(gpu).cuda_stream)), "dsa_fwd")
     torch.cuda.synchronize(gpu)
     assert torch.equal(out2, out) and torch.equal(lse2, lse)
+
+
+def _grads(c: Case, x: dict, dtype, gpu):
+    """(out, dq, dk, dv, dkr, dqr) of the op on the case's inputs."""
+    from deberta_amd import ops  # noqa: F401
+    from deberta_amd.masks import SegmentMask, kernel_masks
+    from deberta_amd.relpos import relative_offset_table
+
+    q, k, v, kr, qr = (x[n].to(gpu, dtype).requires_grad_() for n in ("q", "k", "v", "kr", "qr"))
+    table = relative_offset_table(c.L, c.L, bucket_size=c.buckets, max_position=c.max_pos, device=gpu)
+    mask = SegmentMask(x["seg"]) if x["seg"] is not None else x["mask"].to(gpu)
+    kk, pk = kernel_masks(mask, c.B, c.L, c.L, gpu, segments_from_dense=False)
+    out = torch.ops.deberta_amd.dsa_fwd(q, k, v, kr, qr, table, kk, pk, c.A, 1 / math.sqrt(3 * c.D), True)[0]
+    return [out.detach(), *torch.autograd.grad(out, [q, k, v, kr, qr], x["dout"].to(gpu, dtype))]
+
+
+def _padded(c: Case, live: int, kind: str) -> dict:
+    """The case's inputs with queries and keys past ``live`` padded, as a key
+    mask, segment ids or a pair mask."""
+    x = make_inputs(c)
+    keep = (torch.arange(c.L) < live)[None].repeat(c.B, 1)
+    if kind == "key":
+        x["mask"] = keep[:, None, None, :]
+    elif kind == "seg":
+        x["seg"] = keep.long()
+    else:
+        x["mask"] = (keep[:, :, None] & keep[:, None, :])[:, None]
+    return x
+
+
+def _same(got, want):
+    for name, a, b in zip(("out", "dq", "dk", "dv", "dkr", "dqr"), got, want):
+        assert torch.isfinite(a).all(), name
+        if name in ("dkr", "dqr"):  # sums of atomic additions: one step of the dtype, 2^-20 of scale in fp32
+            tol = (2.0**-20 if a.dtype == torch.float32 else 2.0**-7) * float(b.float().abs().max())
+            assert float((a.float() - b.float()).abs().max()) <= tol, name
+        else:
+            assert torch.equal(a, b), name
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("kind", ["key", "seg", "pair"])
+def test_far_dead_rows_overflow(kind, dtype, gpu):
+    """Padded query rows whose products with the tables overflow, beside live
+    ones of the same 32 rows, change nothing: as with zeros there."""
+    c = Case(B=2, H=2, L=640, D=64, buckets=32, max_pos=64, seed=22)
+    x = _padded(c, 530, kind)
+    x["q"][:, 530:] = 0
+    want = _grads(c, x, dtype, gpu)
+    x["q"][:, 530:] = 3e38
+    _same(_grads(c, x, dtype, gpu), want)
