@@ -198,7 +198,7 @@ DSA_DEV void dq_body(const BwdParams& bp, int blk, int nblk, DqLds<T, D>& L) {
   // lane holds its queries' sums), one side at a time (tiles come in key
   // order: the far side past pos, the near tiles, the far side past neg).
   f32x4 frs[2] = {zero4(), zero4()};
-  int fside = -1;
+  int fside = -1, fsides = 0;  // the last tile's side, the sides visited
   frag ones;
 #pragma unroll
   for (int e = 0; e < FE; ++e) ones[e] = (T)1.0f;
@@ -235,6 +235,7 @@ DSA_DEV void dq_body(const BwdParams& bp, int blk, int nblk, DqLds<T, D>& L) {
           frs[0] = frs[1] = zero4();
         }
         fside = side;
+        fsides |= 1 << side;
       }
     }
     // ---- dQ^T += K^T dS^T: B = dS row i, keys KSTEP*s + FE*g + [0, FE) -----------------------
@@ -313,17 +314,19 @@ DSA_DEV void dq_body(const BwdParams& bp, int blk, int nblk, DqLds<T, D>& L) {
     for (int side = 0; side < 2; ++side) {
       const T* row = (const T*)p.kr + (int64_t)h * p.krs[0] +
                      (int64_t)offset_row(p.rel, far_offset(p, side), p.Lq, p.Lk, p.A, false) * p.krs[1];
+      if ((fsides >> side) & 1) {
 #pragma unroll
-      for (int db = 0; db < ND; ++db)
+        for (int db = 0; db < ND; ++db)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float x = (float)row[16 * db + 4 * g + e];
+          for (int e = 0; e < 4; ++e) {
+            const float x = (float)row[16 * db + 4 * g + e];
 #pragma unroll
-          for (int ib = 0; ib < 2; ++ib) {
-            f32x4& a = QC ? dqca[QC ? db : 0][ib] : dqa[db][ib];
-            a[e] = __builtin_fmaf(x, rs[side][ib], a[e]);
+            for (int ib = 0; ib < 2; ++ib) {
+              f32x4& a = QC ? dqca[QC ? db : 0][ib] : dqa[db][ib];
+              a[e] = __builtin_fmaf(x, rs[side][ib], a[e]);
+            }
           }
-        }
+      }
       far_row_sum<T, NSD>(red + (w * 2 + side) * D, rs[side], qv, g, c16);
     }
     __syncthreads();

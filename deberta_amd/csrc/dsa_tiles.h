@@ -257,7 +257,8 @@ DSA_DEV FarSpan far_span_of(const BwdParams& bp) {
 // LDS, this wave's) = sum over the wave's 32 columns (two 16-wide tiles,
 // column c16 of tile t in the lanes c16 of every group g) of coef[t] *
 // rows[t][..][k], rows the columns' operand fragments (CONTIG k-set), coef the
-// same in the four lane groups.
+// same in the four lane groups.  A column whose coefficient is zero (masked
+// throughout, or of tiles not visited) adds nothing, whatever its row holds.
 template <typename T, int NS>
 DSA_DEV void far_row_sum(float* out, const float (&coef)[2], const typename Mfma<T>::frag (&rows)[2][NS], int g,
                          int c16) {
@@ -266,7 +267,8 @@ DSA_DEV void far_row_sum(float* out, const float (&coef)[2], const typename Mfma
   for (int s = 0; s < NS; ++s)
 #pragma unroll
     for (int e = 0; e < M::FRAG_ELEMS; ++e) {
-      float v = coef[0] * (float)rows[0][s][e] + coef[1] * (float)rows[1][s][e];
+      float v = (coef[0] != 0.f ? coef[0] * (float)rows[0][s][e] : 0.f) +
+                (coef[1] != 0.f ? coef[1] * (float)rows[1][s][e] : 0.f);
 #pragma unroll
       for (int o = 1; o < 16; o <<= 1) v += __shfl_xor(v, o);
       if (c16 == 0) out[M::KSTEP * s + M::FRAG_ELEMS * g + e] = v;

@@ -194,3 +194,32 @@ def test_far_dead_rows_overflow(kind, dtype, gpu):
     want = _grads(c, x, dtype, gpu)
     x["q"][:, 530:] = 3e38
     _same(_grads(c, x, dtype, gpu), want)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("kind", ["key", "seg", "pair"])
+def test_far_dead_chunks(kind, dtype, gpu):
+    """What the padded queries of 32-row chunks without a live one hold (NaN)
+    reaches nothing, the far rows of dKr included."""
+    c = Case(B=2, H=2, L=640, D=64, buckets=32, max_pos=64, seed=23)
+    x = _padded(c, 544, kind)
+    for n in ("q", "dout"):
+        x[n][:, 544:] = 0
+    want = _grads(c, x, dtype, gpu)
+    for n in ("q", "dout"):
+        x[n][:, 544:] = float("nan")
+    _same(_grads(c, x, dtype, gpu), want)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+def test_far_side_without_pairs(dtype, gpu):
+    """Far keys on one side only: the other side's table rows reach nothing."""
+    c = Case(B=1, H=2, L=800, D=64, buckets=64, max_pos=256, seed=24)
+    x = make_inputs(c)
+    x["mask"] = torch.ones(c.L, c.L, dtype=torch.bool).triu()[None, None]
+    x["kr"][:, 2 * c.A - 1] = 0
+    x["qr"][:, 0] = 0
+    want = _grads(c, x, dtype, gpu)
+    x["kr"][:, 2 * c.A - 1] = float("nan")
+    x["qr"][:, 0] = float("nan")
+    _same(_grads(c, x, dtype, gpu), want)
