@@ -427,6 +427,19 @@ __global__ __launch_bounds__(256, 2) void dsa_fwd_kernel(FwdParams p) {
           st[ib][jb] = acc;
         }
       }
+      // a term that is not finite joins here, before the masks, so that it
+      // stays with the kept pairs (at the softmax it would meet the masked
+      // ones' -inf)
+      if (__any(!(fabsf(fa[0]) < INFINITY && fabsf(fa[1]) < INFINITY))) {
+#pragma unroll
+        for (int ib = 0; ib < 2; ++ib) {
+#pragma unroll
+          for (int jb = 0; jb < 4; ++jb)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) st[ib][jb][e] += fa[ib];
+          fa[ib] = 0.f;
+        }
+      }
     } else {
 #pragma unroll
       for (int jb = 0; jb < 4; ++jb)

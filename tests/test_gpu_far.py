@@ -218,8 +218,41 @@ def test_far_side_without_pairs(dtype, gpu):
     x = make_inputs(c)
     x["mask"] = torch.ones(c.L, c.L, dtype=torch.bool).triu()[None, None]
     x["kr"][:, 2 * c.A - 1] = 0
-    x["qr"][:, 0] = 0
+    x["qr"][:, 1] = 0  # (bucket A - 1)
     want = _grads(c, x, dtype, gpu)
     x["kr"][:, 2 * c.A - 1] = float("nan")
-    x["qr"][:, 0] = float("nan")
+    x["qr"][:, 1] = float("nan")
     _same(_grads(c, x, dtype, gpu), want)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), float("-inf")])
+def test_far_term_not_finite(value, dtype, gpu):
+    """A far c2p term that is not finite stays with the pairs it belongs to:
+    the rows of the same tiles whose far pairs are all masked are as without
+    it."""
+    from deberta_amd import ops  # noqa: F401
+    from deberta_amd.masks import kernel_masks
+    from deberta_amd.relpos import relative_offset_table
+
+    c = Case(B=1, H=2, L=700, D=64, buckets=32, max_pos=64, types="c2p", seed=25)
+    x = make_inputs(c)
+    i = torch.arange(c.L)
+    keep = (i[:, None] - i[None]).abs() <= 20  # none of these reads a saturated row
+    keep[::128] = True  # one row of every tile keeps all keys
+    kk, pk = kernel_masks(keep[None, None].to(gpu), c.B, c.L, c.L, gpu, segments_from_dense=False)
+    table = relative_offset_table(c.L, c.L, bucket_size=c.buckets, max_position=c.max_pos, device=gpu)
+    q, k, v = (x[n].to(gpu, dtype) for n in ("q", "k", "v"))
+    local = torch.arange(c.L) % 128 != 0
+    got = []
+    for far in (0.0, value):
+        kr = x["kr"].clone()
+        kr[:, 1] = 0.0  # the row of the keys far after the queries (bucket 1 - A)
+        kr[:, 1, 0] = far
+        out, lse, _, _ = torch.ops.deberta_amd.dsa_fwd(
+            q, k, v, kr.to(gpu, dtype), None, table, kk, pk, c.A, 1 / math.sqrt(2 * c.D), False
+        )
+        got.append((out[:, local], lse[:, :, local]))
+    assert torch.isfinite(got[0][0]).all()
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
