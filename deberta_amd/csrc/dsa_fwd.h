@@ -433,11 +433,13 @@ __global__ __launch_bounds__(256, 2) void dsa_fwd_kernel(FwdParams p) {
       if (__any(!(fabsf(fa[0]) < INFINITY && fabsf(fa[1]) < INFINITY))) {
 #pragma unroll
         for (int ib = 0; ib < 2; ++ib) {
+          const bool fine = fabsf(fa[ib]) < INFINITY;  // the lane's other queries stay as they are
+          const float a = fine ? 0.f : fa[ib];
 #pragma unroll
           for (int jb = 0; jb < 4; ++jb)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) st[ib][jb][e] += fa[ib];
-          fa[ib] = 0.f;
+            for (int e = 0; e < 4; ++e) st[ib][jb][e] += a;
+          fa[ib] = fine ? fa[ib] : 0.f;
         }
       }
     } else {
