@@ -358,7 +358,10 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
       if constexpr (!FAR) return n;
       return n < n1 ? n : n < n2 ? qhi + n - n1 : n1 + n - n2;
     };
-    const int qfirst = entry(0) & 0x3ff;
+    // the tile of an entry (a list entry has its flag above 10 bits; a call
+    // without a list may have more tiles)
+    auto tile_of = [&](int ent) { return LIST ? ent & 0x3ff : ent; };
+    const int qfirst = tile_of(entry(0));
     if (!FAR || n2 == 0) {
       if (p2c)
         for (int r = 0; r < 4; ++r) issue_ring(tw0 / 32 + qfirst + r);
@@ -377,7 +380,7 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
                     const uint32_t* Pw, T* nQ, T* ndO, BT* nBt, float* nR, uint32_t* nDw, uint32_t* nPw) {
       constexpr bool far = decltype(farkind)::value;
       const int ent = entry(n);
-      const int qi = ent & 0x3ff, i0 = qi * BQ;
+      const int qi = tile_of(ent), i0 = qi * BQ;
       // This wave's copies of tile qi have landed: they were issued before
       // the previous tile's NST dS stores, its last vector-memory
       // instructions (tile 0 was waited for before the loop).
@@ -396,7 +399,7 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
       }
       const uint4 pcur = pnext;
       if (n + 1 < nlist) {
-        const int qn = entry(n + 1) & 0x3ff;
+        const int qn = tile_of(entry(n + 1));
         if constexpr (far) issue(qn, n + 1 == n2 ? 5 : 0, n + 1 < n1 ? 1 : n + 1 < n2 ? 0 : -1, nQ, ndO, nBt, nR, nDw, nPw);
         else issue(qn, qn == qi + 1, -1, nQ, ndO, nBt, nR, nDw, nPw);
       }

@@ -24,7 +24,7 @@ namespace dsa {
 
 namespace dqcfg {
 constexpr int NW = 4, WQ = 32, BQ = 128, BK = 64;
-constexpr int MAX_KT = 1024;  // key tiles (Lk <= 65536)
+constexpr int MAX_KT = 1024;  // key tiles of a list (masks: Lk <= 32768)
 constexpr int XW = 96;   // offset rows per wave (95 used)
 constexpr int ZC = 32;   // zero columns before each staged dS row
 }  // namespace dqcfg
@@ -125,7 +125,7 @@ DSA_DEV void dq_body(const BwdParams& bp, int blk, int nblk, DqLds<T, D>& L) {
     vecT(&sr)[SCH] = r.s;
     vecT(&kr)[KCH] = r.k;
     vecT(&gr)[GCH] = r.g;
-    const int kt = entry & 1023, cmask = entry >> 10;
+    const int kt = entry & 0xfffff, cmask = entry >> 20;
     const int j0 = kt * BK;
 #pragma unroll
     for (int k = 0; k < SCH; ++k) {
@@ -162,9 +162,11 @@ DSA_DEV void dq_body(const BwdParams& bp, int blk, int nblk, DqLds<T, D>& L) {
   // With a mask, dS was computed only for the tiles of 32 queries x 128 keys
   // whose segments can meet (ChunkRange) or that hold a kept pair (pair_active): a key
   // tile is visited if one of its 4 query chunks is active, and the rows of
-  // inactive chunks are read as zeros.  klist holds kt | (chunk mask << 10).
+  // inactive chunks are read as zeros.  klist holds kt | (chunk mask << 10);
+  // entry gives kt | (chunk mask << 20), without a mask every tile's.
   int nkt = bp.f.LkP / BK;
-  if (bp.cinfo || p.pflag) {
+  const bool listed = bp.cinfo || p.pflag;
+  if (listed) {
     // listed by wave 0, one key tile per lane
     if (tid < 64) {
       const int nch = bp.f.LqP / 32;
@@ -190,10 +192,12 @@ DSA_DEV void dq_body(const BwdParams& bp, int blk, int nblk, DqLds<T, D>& L) {
     }
     __syncthreads();
     nkt = __builtin_amdgcn_readfirstlane(segred[0]);
-  } else {
-    for (int t = tid; t < nkt; t += 256) klist[t] = (short)(t | (0xf << 10));
-    __syncthreads();
   }
+  auto entry = [&](int n) {
+    if (!listed) return n | (0xf << 20);
+    const int e = klist[n];
+    return (e & 1023) | ((e >> 10) << 20);
+  };
   // Far tiles: row sums of dS (every row of the A operand is ones, so each
   // lane holds its queries' sums), one side at a time (tiles come in key
   // order: the far side past pos, the near tiles, the far side past neg).
@@ -204,7 +208,7 @@ DSA_DEV void dq_body(const BwdParams& bp, int blk, int nblk, DqLds<T, D>& L) {
   for (int e = 0; e < FE; ++e) ones[e] = (T)1.0f;
   float rs[2][2] = {{0.f, 0.f}, {0.f, 0.f}};  // per side
   auto tile = [&](int n, Regs& r) {
-    const int kt = klist[n] & 1023;
+    const int kt = entry(n) & 0xfffff;
     const bool far = is_far(kt);
     __syncthreads();  // previous tile's readers are done
 #pragma unroll
@@ -225,7 +229,7 @@ DSA_DEV void dq_body(const BwdParams& bp, int blk, int nblk, DqLds<T, D>& L) {
       }
     }
     __syncthreads();
-    if (n + 2 < nkt) fetch(klist[n + 2], r);
+    if (n + 2 < nkt) fetch(entry(n + 2), r);
 
     if (FAR && far && c2p) {
       const int side = fs.side(qt - kt / (128 / BK));
@@ -284,8 +288,8 @@ DSA_DEV void dq_body(const BwdParams& bp, int blk, int nblk, DqLds<T, D>& L) {
       }
     }
   };
-  if (nkt > 0) fetch(klist[0], ra);
-  if (nkt > 1) fetch(klist[1], rb);
+  if (nkt > 0) fetch(entry(0), ra);
+  if (nkt > 1) fetch(entry(1), rb);
   for (int n = 0; n < nkt; n += 2) {
     tile(n, ra);
     if (n + 1 < nkt) tile(n + 1, rb);
