@@ -358,9 +358,11 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
       if constexpr (!FAR) return n;
       return n < n1 ? n : n < n2 ? qhi + n - n1 : n1 + n - n2;
     };
-    // the tile of an entry (a list entry has its flag above 10 bits; a call
-    // without a list may have more tiles)
-    auto tile_of = [&](int ent) { return LIST ? ent & 0x3ff : ent; };
+    // the tile of an entry: a list entry has its flag above 10 bits; a call
+    // without a list may have more tiles, below 2^18 (the padded dS slice, at
+    // least 128 keys wide, is below 2 GiB; the compiler is told, since without
+    // a bound the unmasked kernel spills 13 registers)
+    auto tile_of = [&](int ent) { return ent & (LIST ? 0x3ff : 0x3ffff); };
     const int qfirst = tile_of(entry(0));
     if (!FAR || n2 == 0) {
       if (p2c)

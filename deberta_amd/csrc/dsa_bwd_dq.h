@@ -46,8 +46,10 @@ struct DqLds {
 // Workgroup blk of nblk (the logical index, whose remainder mod 8 is the
 // XCD it runs on).  QC: the c2p part (the gradient of the c2p term's query
 // rows qc) is accumulated apart and written to dqc; dq then holds the
-// content part.  FAR: calls that can have far blocks (FarSpan).
-template <typename T, int D, bool QC, bool FAR>
+// content part.  FAR: calls that can have far blocks (FarSpan).  LISTED: a
+// mask is given (bp.cinfo, or the pair mask's flags), whose key tiles are
+// listed.
+template <typename T, int D, bool LISTED, bool QC, bool FAR>
 DSA_DEV void dq_body(const BwdParams& bp, int blk, int nblk, DqLds<T, D>& L) {
   using namespace dqcfg;
   using M = Mfma<T>;
@@ -165,8 +167,7 @@ DSA_DEV void dq_body(const BwdParams& bp, int blk, int nblk, DqLds<T, D>& L) {
   // inactive chunks are read as zeros.  klist holds kt | (chunk mask << 10);
   // entry gives kt | (chunk mask << 20), without a mask every tile's.
   int nkt = bp.f.LkP / BK;
-  const bool listed = bp.cinfo || p.pflag;
-  if (listed) {
+  if constexpr (LISTED) {
     // listed by wave 0, one key tile per lane
     if (tid < 64) {
       const int nch = bp.f.LqP / 32;
@@ -194,7 +195,7 @@ DSA_DEV void dq_body(const BwdParams& bp, int blk, int nblk, DqLds<T, D>& L) {
     nkt = __builtin_amdgcn_readfirstlane(segred[0]);
   }
   auto entry = [&](int n) {
-    if (!listed) return n | (0xf << 20);
+    if constexpr (!LISTED) return n | (0xf << 20);
     const int e = klist[n];
     return (e & 1023) | ((e >> 10) << 20);
   };
@@ -373,10 +374,10 @@ DSA_DEV void dq_body(const BwdParams& bp, int blk, int nblk, DqLds<T, D>& L) {
   }
 }
 
-template <typename T, int D, bool QC, bool FAR>
+template <typename T, int D, bool LISTED, bool QC, bool FAR>
 __global__ __launch_bounds__(256, 2) void dsa_bwd_dq_kernel(BwdParams bp) {
   __shared__ DqLds<T, D> L;
-  dq_body<T, D, QC, FAR>(bp, blockIdx.x, gridDim.x, L);
+  dq_body<T, D, LISTED, QC, FAR>(bp, blockIdx.x, gridDim.x, L);
 }
 
 }  // namespace dsa

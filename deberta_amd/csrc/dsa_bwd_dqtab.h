@@ -34,7 +34,7 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dqtab_kernel(BwdParams bp, Bwd
   if (n < nt8) {
     if (n < ntab) table_body<T, D, LISTED, FAR>(tp, n, ntab, L.tab);
   } else {
-    dq_body<T, D, QC, FAR>(bp, n - nt8, ndq, L.dq);
+    dq_body<T, D, LISTED, QC, FAR>(bp, n - nt8, ndq, L.dq);
   }
 }
 

@@ -401,10 +401,14 @@ int launch_dq_fold(const dsa::BwdParams& bp, const dsa::BwdParams& tp, int ntab,
     return launch_check("dsa_bwd_table_kernel");
   }
   if (dq) {
-    if (qc)
-      hipLaunchKernelGGL((dsa::dsa_bwd_dq_kernel<T, D, true, FAR>), dim3(ndq), dim3(256), 0, st, bp);
+    if (listed && qc)
+      hipLaunchKernelGGL((dsa::dsa_bwd_dq_kernel<T, D, true, true, FAR>), dim3(ndq), dim3(256), 0, st, bp);
+    else if (listed)
+      hipLaunchKernelGGL((dsa::dsa_bwd_dq_kernel<T, D, true, false, FAR>), dim3(ndq), dim3(256), 0, st, bp);
+    else if (qc)
+      hipLaunchKernelGGL((dsa::dsa_bwd_dq_kernel<T, D, false, true, FAR>), dim3(ndq), dim3(256), 0, st, bp);
     else
-      hipLaunchKernelGGL((dsa::dsa_bwd_dq_kernel<T, D, false, FAR>), dim3(ndq), dim3(256), 0, st, bp);
+      hipLaunchKernelGGL((dsa::dsa_bwd_dq_kernel<T, D, false, false, FAR>), dim3(ndq), dim3(256), 0, st, bp);
     return launch_check("dsa_bwd_dq_kernel");
   }
   return 0;
