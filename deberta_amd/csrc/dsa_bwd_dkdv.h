@@ -149,7 +149,6 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
   const int64_t riplane = (int64_t)p.B * p.H * p.LqP * 2;  // far blocks: the planes of the two sides follow
   FarSpan fs{kNoFar, -kNoFar};
   if constexpr (FAR) fs = far_span_of(bp);
-  auto is_far = [&](int qi) { return FAR && fs.far(qi / (128 / BQ) - kt); };
   int64_t pmask = 0;  // pair bits: the mask of (b, h)
   if constexpr (BITS) pmask = pair_index(p, b, h);
   const SegView<MASK> sv(p, b);
@@ -179,6 +178,12 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
   // nothing of the others.
   bool any_key;
   int nlist = nqt, n1 = 0, n2 = 0, qhi = 0;
+  if constexpr (FAR) {
+    // far: the tiles below n1 and from qhi on
+    n1 = min(max((128 / BQ) * (kt + fs.neg + 1), 0), nqt);
+    qhi = min(max((128 / BQ) * (kt + fs.pos), 0), nqt);
+    n2 = n1 + nqt - qhi;
+  }
   if constexpr (LIST) {
     ChunkRange kr{0, 0, 0};
     if constexpr (SEGM) kr = key_tile_range(bp.cinfo + (int64_t)b * nqt, kt, nqt);
@@ -186,10 +191,12 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
       int n = 0;
 #pragma unroll 1
       for (int part = 0; part < (FAR ? 3 : 1); ++part) {
-        for (int c0 = 0; c0 < nqt; c0 += 64) {
+        const int from = part == 0 ? 0 : part == 1 ? qhi : n1;
+        const int to = !FAR || part == 1 ? nqt : part == 0 ? n1 : qhi;
+        for (int c0 = from; c0 < to; c0 += 64) {
           const int c = c0 + lane;
           bool act = false, full = false;
-          if (c < nqt) {
+          if (c < to) {
             if constexpr (SEGM) {
               const ChunkRange x = chunk_range(bp.cinfo + (int64_t)b * nqt, c);
               act = x.meets(kr);
@@ -199,7 +206,6 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
               act = (f & 0x0101u) != 0;
               full = (f & 0x0202u) == 0x0202u;
             }
-            if (FAR) act = act && part == (!is_far(c) ? 2 : c / (128 / BQ) < kt ? 0 : 1);
           }
           n = wave_append(act, (short)(c | (full ? 0x4000 : 0)), qlist, n);
         }
@@ -214,11 +220,6 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
     nlist = __builtin_amdgcn_readfirstlane(qlen[FAR ? 2 : 0]);
     any_key = nlist > 0;
   } else {
-    if constexpr (FAR) {
-      n1 = min(max((128 / BQ) * (kt + fs.neg + 1), 0), nqt);
-      qhi = min(max((128 / BQ) * (kt + fs.pos), 0), nqt);
-      n2 = n1 + nqt - qhi;
-    }
     any_key = __syncthreads_or(tid < BKW && j0 + tid < Lk);
   }
 

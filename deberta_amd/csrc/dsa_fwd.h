@@ -134,38 +134,6 @@ __global__ __launch_bounds__(256, 2) void dsa_fwd_kernel(FwdParams p) {
         qcf[ib][s] = (irow[ib] < Lq) ? M::load_contig(qcbase + (int64_t)irow[ib] * p.qcs[1], s, g) : M::zero();
   }
 
-  FarSpan fs{kNoFar, -kNoFar};
-  if constexpr (FAR) {
-    if (p.span) fs = FarSpan{__builtin_amdgcn_readfirstlane(p.span[0]), __builtin_amdgcn_readfirstlane(p.span[1])};
-    else fs = far_span(p, farred);
-#pragma unroll
-    for (int side = 0; side < 2; ++side) {
-      const int e = far_offset(p, side);
-      if (tid < D / VEC) {
-        vecT x;
-#pragma unroll
-        for (int u = 0; u < VEC; ++u) x[u] = (T)0.0f;  // without p2c
-        if (p.flags & 2)
-          x = *reinterpret_cast<const vecT*>(qrh + (int64_t)offset_row(p.rel, e, Lq, Lk, A, true) * p.qrs[1] +
-                                             (tid * VEC / M::KSTEP) * p.qrk + tid * VEC % M::KSTEP);
-        *reinterpret_cast<vecT*>(&farq[side][tid * VEC]) = x;
-      }
-      f32x4 a2[2] = {zero4(), zero4()};
-      if (p.flags & 1) {
-        // every row of the A operand is the far row: the result's rows all
-        // hold the queries' terms
-        const T* row = krh + (int64_t)offset_row(p.rel, e, Lq, Lk, A, false) * p.krs[1];
-#pragma unroll
-        for (int s = 0; s < NS; ++s) {
-          const frag af = *reinterpret_cast<const frag*>(row + s * p.krk + M::FRAG_ELEMS * g);
-#pragma unroll
-          for (int ib = 0; ib < 2; ++ib) a2[ib] = M::mma(af, pick<QC>(qcf, qf)[ib][s], a2[ib]);
-        }
-      }
-      if (g == 0) fara[side][w * WQ + c16] = a2[0][0], fara[side][w * WQ + 16 + c16] = a2[1][0];
-    }
-  }
-
   float mref[2] = {-INFINITY, -INFINITY};  // reference max of the unscaled scores
   float lrow[2] = {0.f, 0.f};
   f32x4 o[ND][2];
@@ -263,6 +231,48 @@ __global__ __launch_bounds__(256, 2) void dsa_fwd_kernel(FwdParams p) {
     }
     __syncthreads();
     nlist = __builtin_amdgcn_readfirstlane(klen);
+  }
+
+  // Far blocks: the p2c row and the queries' c2p terms of either side, for the
+  // workgroups that visit one (the tiles lie in key order: a far one comes
+  // first or last).
+  FarSpan fs{kNoFar, -kNoFar};
+  bool any_far = false;
+  if constexpr (FAR) {
+    if (p.span) fs = FarSpan{__builtin_amdgcn_readfirstlane(p.span[0]), __builtin_amdgcn_readfirstlane(p.span[1])};
+    else fs = far_span(p, farred);
+    if (any_live && nlist > 0) {
+      const int ka = LIST ? klist[0] : 0, kb = LIST ? klist[nlist - 1] : nkt - 1;
+      any_far = __builtin_amdgcn_readfirstlane(fs.far(qt - ka / 2) || fs.far(qt - kb / 2));
+    }
+  }
+  if (FAR && any_far) {
+#pragma unroll
+    for (int side = 0; side < 2; ++side) {
+      const int e = far_offset(p, side);
+      if (tid < D / VEC) {
+        vecT x;
+#pragma unroll
+        for (int u = 0; u < VEC; ++u) x[u] = (T)0.0f;  // without p2c
+        if (p.flags & 2)
+          x = *reinterpret_cast<const vecT*>(qrh + (int64_t)offset_row(p.rel, e, Lq, Lk, A, true) * p.qrs[1] +
+                                             (tid * VEC / M::KSTEP) * p.qrk + tid * VEC % M::KSTEP);
+        *reinterpret_cast<vecT*>(&farq[side][tid * VEC]) = x;
+      }
+      f32x4 a2[2] = {zero4(), zero4()};
+      if (p.flags & 1) {
+        // every row of the A operand is the far row: the result's rows all
+        // hold the queries' terms
+        const T* row = krh + (int64_t)offset_row(p.rel, e, Lq, Lk, A, false) * p.krs[1];
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+          const frag af = *reinterpret_cast<const frag*>(row + s * p.krk + M::FRAG_ELEMS * g);
+#pragma unroll
+          for (int ib = 0; ib < 2; ++ib) a2[ib] = M::mma(af, pick<QC>(qcf, qf)[ib][s], a2[ib]);
+        }
+      }
+      if (g == 0) fara[side][w * WQ + c16] = a2[0][0], fara[side][w * WQ + 16 + c16] = a2[1][0];
+    }
   }
 
   // The next key tile (K and V rows) is fetched into registers while the
