@@ -286,10 +286,13 @@ __global__ __launch_bounds__(256, 2) void dsa_fwd_kernel(FwdParams p) {
   // positions of their 16 offsets, requested a tile earlier still, are there
   // by then.
   // (Forward 137.9 -> 131.6 us at B=32, L=512, H=12, 82.4 -> 81.2 with padded
-  // rows, 246 -> 234 with documents at B=4, L=4096.  Not for the pair mask and
-  // the p2p query rows, whose kernels have no registers for the held rows, nor
-  // for fp32, whose rows are four loads each.)
-  constexpr bool CARRY = sizeof(T) == 2 && MASK != MASK_PAIR && !QC;
+  // rows, 246 -> 234 with documents at B=4, L=4096.  Not for the pair mask's
+  // bytes, the p2p query rows and masks with dropout, whose kernels have no
+  // registers for the held rows (with them, masks with dropout spill 4, 8
+  // beside far blocks: 58.8 -> 60.4 us with documents, 90.1 -> 91.8 with padded
+  // rows at B=32, L=512, 152 -> 160 at B=2, L=3072), nor for fp32, whose rows
+  // are four loads each.)
+  constexpr bool CARRY = sizeof(T) == 2 && MASK != MASK_PAIR && !QC && (MASK == MASK_NONE || !DROP);
   frag pheld[CARRY ? 3 : 1][NS], pnew[NS];
 #pragma unroll
   for (int s = 0; s < NS; ++s) pnew[s] = M::zero();
