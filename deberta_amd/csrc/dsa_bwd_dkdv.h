@@ -109,18 +109,15 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
   // spilled in the near loop: 339 against 276 us at B=4, L=2048, H=16) and the
   // kernels with per-element mask tests need, for more scalar ones, which
   // spill to vector lanes and cost the others up to 6% (dropout at B=12,
-  // L=512: 85.7 against 80.8 us).
-  constexpr bool SCAL = FAR || MASK == MASK_SEG || BITS;
+  // L=512: 85.7 against 80.8 us; documents with dropout at B=32, whose kernel
+  // fits without: 71.1 against 69.0).
+  constexpr bool SCAL = FAR || (MASK == MASK_SEG && !DROP) || BITS;
   const int w = SCAL ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
   const int g = (tid & 63) >> 4, c16 = tid & 15;
   // one 16-byte LDS copy: byte offset off (lane part) from the uniform base
   auto copy16 = [&](const void* base, unsigned off, void* lds_wave) {
     if constexpr (SCAL) lds_dma16_s(base, off, lds_wave);
     else lds_dma16((const char*)base + off, lds_wave);
-  };
-  auto copy16_nt = [&](const void* base, unsigned off, void* lds_wave) {
-    if constexpr (SCAL) lds_dma16_s_nt(base, off, lds_wave);
-    else lds_dma16_nt((const char*)base + off, lds_wave);
   };
   const int Lq = p.Lq, Lk = p.Lk;
   const int NKT = p.LkP / BKW;
@@ -235,9 +232,14 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
 #pragma unroll
     for (int k = 0; k < (RCPB + 255) / 256; ++k) {
       if (256 * k + w * 64 < RCPB) {
-        const int c = (256 * k + w * 64) / D + lane / D, d = lane % D;  // D divides 64
-        copy16(qrg + 32 * rb, (unsigned)((d * bp.TGP + c * VEC) * (int)sizeof(T)),
-                    (char*)(slot + (256 * k + w * 64) * VEC));
+        char* dst = (char*)(slot + (256 * k + w * 64) * VEC);
+        if constexpr (SCAL) {
+          const int c = (256 * k + w * 64) / D + lane / D, d = lane % D;  // D divides 64
+          lds_dma16_s(qrg + 32 * rb, (unsigned)((d * bp.TGP + c * VEC) * (int)sizeof(T)), dst);
+        } else {
+          const int pc = 256 * k + w * 64 + lane;
+          lds_dma16(qrg + (int64_t)(pc % D) * bp.TGP + 32 * rb + (pc / D) * VEC, dst);
+        }
       }
     }
   };
@@ -280,10 +282,13 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
       constexpr int CPB = 2048 * (int)sizeof(BT) / 16;
 #pragma unroll
       for (int k = 0; k < BCW / 64; ++k) {
-        const int pc = w * BCW + 64 * k;  // of lane 0; a wave's 64 chunks lie in one block
+        // of lane 0 (SCAL; a wave's 64 chunks lie in one block) or the lane
+        const int pc = w * BCW + 64 * k + (SCAL ? 0 : lane);
         const BT* src = biasb + bias_tile_offset(b, h, p.H, i0 / 128, j0 / 64 + pc / CPB, p.LqP, p.LkP) +
                         ((i0 % 128) / 32) * 2048 + (pc % CPB) * (16 / (int)sizeof(BT));
-        copy16_nt(src, lane * 16, (char*)Bd + pc * 16);  // read once: non-temporal
+        char* dst = (char*)Bd + (w * BCW + 64 * k) * 16;
+        if constexpr (SCAL) lds_dma16_s_nt(src, lane * 16, dst);  // read once: non-temporal
+        else lds_dma16_nt(src, dst);
       }
     }
     if (w == 0 && lane < 2 * BQ * 4 / 16)
