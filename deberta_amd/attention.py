@@ -31,6 +31,7 @@ from deberta_amd.relpos import (
     is_toeplitz,
     normalize_relative_pos,
     relative_offset_table,
+    saturation_distance,
     table_from_matrix,
 )
 
@@ -209,6 +210,7 @@ def fused_attention(
     qc: Optional[torch.Tensor] = None,
     qkv: Optional[torch.Tensor] = None,
     dropout_p: float = 0.0,
+    rel_saturated: int = 0,
 ) -> torch.Tensor:
     """Core call on ``[B, L, H, D]`` layers; returns ``[B, Lq, H, D]``.
     ``kr`` / ``qr`` are the c2p / p2c tables (None: term off); ``qc`` the
@@ -216,7 +218,8 @@ def fused_attention(
     ``[B, L, 3, H, D]`` tensor (q, k, v are then None); the op takes it
     whole and its gradient comes back as one tensor.  ``dropout_p``:
     attention dropout in the kernels, with a fresh seed from torch's CPU
-    generator (``ops.dropout_threshold(dropout_p)`` must lie in [1, 65535])."""
+    generator (``ops.dropout_threshold(dropout_p)`` must lie in [1, 65535]).
+    ``rel_saturated``: the ops' hint of where ``table`` saturates."""
     ref = qkv if qkv is not None else q  # shapes, dtype and device
     _require_gpu(ref)
     B, Lq, H = ref.shape[0], ref.shape[1], ref.shape[-2]
@@ -242,11 +245,13 @@ def fused_attention(
         seed = ops.draw_dropout_seed()
     if qkv is not None:
         out, _, _, _ = ops.attention_packed(
-            qkv, kr, qr, table, key_keep, pair_keep, int(att_span), float(scale), save_bias, qc, drop_t, seed
+            qkv, kr, qr, table, key_keep, pair_keep, int(att_span), float(scale), save_bias, qc, drop_t, seed,
+            rel_saturated,
         )
     else:
         out, _, _, _ = ops.attention(
-            q, k, v, kr, qr, table, key_keep, pair_keep, int(att_span), float(scale), save_bias, qc, drop_t, seed
+            q, k, v, kr, qr, table, key_keep, pair_keep, int(att_span), float(scale), save_bias, qc, drop_t, seed,
+            rel_saturated,
         )
     return out
 
@@ -320,7 +325,10 @@ def disentangled_attention(
     if kr is not None or qr is not None:
         table = table_for(relative_pos, q.shape[1], k.shape[1], position_buckets, max_relative_positions, q.device)
     _check_mask_rank(attention_mask)
-    out = fused_attention(q, k, v, kr, qr, table, attention_mask, att_span, scale, qc, dropout_p=dropout_p)
+    sat = saturation_distance(position_buckets, max_relative_positions, att_span)
+    out = fused_attention(
+        q, k, v, kr, qr, table, attention_mask, att_span, scale, qc, dropout_p=dropout_p, rel_saturated=sat
+    )
     return out.transpose(1, 2) if layout == "bhld" else out
 
 
@@ -576,7 +584,10 @@ class DisentangledSelfAttention(nn.Module):
 
         # the op takes the packed projection whole (its gradient comes back
         # as one tensor)
-        ctx = fused_attention(q, k, v, kr, qr, table, attention_mask, att_span, scale, qc, qkv=qkv, dropout_p=drop_p)
+        sat = saturation_distance(self.position_buckets, self.max_relative_positions, att_span)
+        ctx = fused_attention(
+            q, k, v, kr, qr, table, attention_mask, att_span, scale, qc, qkv=qkv, dropout_p=drop_p, rel_saturated=sat
+        )
         bsz, seq_len = ctx.shape[0], ctx.shape[1]
         context_layer = ctx.reshape(bsz, seq_len, self.all_head_size).to(dtype=model_dtype)
         return context_layer, None

@@ -441,7 +441,7 @@ dsa::rows::RtdParams rtd_params(const dsa_rtd_args* a) {
 
 extern "C" {
 
-int dsa_version(void) { return 12; }
+int dsa_version(void) { return 13; }
 
 const char* dsa_last_error(void) { return g_err.c_str(); }
 

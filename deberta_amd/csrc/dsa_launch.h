@@ -53,9 +53,31 @@ static int round_up(int x, int a) { return (x + a - 1) / a * a; }
 
 static int elem_bytes(int dtype) { return dtype == DSA_BF16 ? 2 : 4; }
 
-// Whether the call's kernels look for far blocks (FarSpan).
+// Whether the call's kernels look for far blocks (FarSpan): where at least
+// `need` percent of its blocks lie past the saturation.  A far block saves its
+// bands, but the FAR kernels' near tiles are the slower ones (in bf16 dkdv's
+// scalar registers spill, and its query rows are read once more for the far
+// planes), so that calls with few far blocks lose.  Training step at 12 heads,
+// buckets 256 / max_position 512, 8192 tokens, plain -> FAR in us:
+//   L (share)     1024 (19%)  1152 (25%)  1408 (35%)  1536 (39%)  2048 (52%)
+//   no mask       493 -> 514  579 -> 559  620 -> 600  718 -> 655  952 -> 806
+//   ... p2p       491 -> 512  546 -> 545  599 -> 587  680 -> 644  933 -> 775
+//   ... and drop  550 -> 579  615 -> 627  675 -> 683  778 -> 745  1018 -> 903
+//   padded rows   397 -> 400  311 -> 309  358 -> 344  471 -> 405  485 -> 424
+//   causal, bits  390 -> 381  400 -> 391  431 -> 401  531 -> 478  687 -> 574
+// Documents know no share: those of 2/3 of a row gain from 39% on (441 -> 437,
+// 654 -> 606 at 52%, 644 -> 560 at L = 3072), those of 250 tokens hold no far
+// pair and lose 5 to 7% at any length (290 -> 303, 262 -> 282), more with
+// dropout (dkdv's registers again): they take long rows.  In float32 (4096
+// tokens) the registers fit: 6% 1006 -> 1023, 12% 1149 -> 1121, 30% 1604 ->
+// 1477; documents 30% 1242 -> 1189 and 605 -> 622.
 static bool far_call(const dsa_fwd_args* a) {
-  return dsa::far_wanted(a->flags, round_up(a->Lq, 128), round_up(a->Lk, 128), a->att_span);
+  if (!a->flags) return false;
+  const int nq = round_up(a->Lq, 128) / 128, nk = round_up(a->Lk, 128) / 128;
+  const int64_t far = dsa::far_blocks(nq, nk, a->rel_saturated > 0 ? a->rel_saturated : 2 * a->att_span);
+  const bool bf = a->dtype == DSA_BF16, drop = a->dropout_threshold != 0;
+  const int need = a->seg ? (!bf ? 30 : drop ? 60 : 50) : !bf ? 10 : a->qc ? 38 : 25;
+  return far > 0 && far * 100 >= (int64_t)nq * nk * need;
 }
 
 static dsa::FwdParams to_params(const dsa_fwd_args* a) {

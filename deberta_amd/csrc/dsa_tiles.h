@@ -188,7 +188,7 @@ DSA_DEV SegRange wg_seg_range(int s, bool has, int* red) {
 //   dQ_i += s_i Kr[c],  dKr[c] += sum_i s_i q_i,  and so for K and Qr.
 // At position buckets 256 / max_position 512 delta >= 5 is far: 52% of the
 // blocks at L = 2048, 74% at L = 4096.  Whether blocks can be far is decided
-// on the host from the extents (far_wanted), so shorter calls search nothing.
+// on the host from the extents (far_call), so shorter calls search nothing.
 // One workgroup of the preparation before the forward, and one of the
 // backward's prep kernel, find the span for the kernels after them (2 us at
 // L = 4096, beside the preparation's other blocks); a forward without a
@@ -199,12 +199,15 @@ struct FarSpan {
   DSA_DEV bool far(int delta) const { return delta >= pos || delta <= neg; }
   DSA_DEV int side(int delta) const { return delta > 0 ? 0 : 1; }  // of a far delta: 0 past pos, 1 past neg
 };
-// The host's rule: the furthest block diagonal's smallest offset is at least
-// the 2 att_span rows of a table.  An unbucketed table saturates att_span
-// offsets out, the log-bucketed ones of max_position = 2 att_span about 2
-// att_span out; nearer searches would find nothing or a corner block.
-inline bool far_wanted(int flags, int LqP, int LkP, int A) {
-  return flags != 0 && (LqP > LkP ? LqP : LkP) - 128 - 127 >= 2 * A;
+// Blocks past a saturation at distance sat, of the nq x nk blocks of a call.
+inline int64_t far_blocks(int nq, int nk, int sat) {
+  const int d = sat > 1 ? (sat + 254) / 128 : 1;  // the first diagonal with 128 d - 127 >= sat
+  int64_t n = 0;
+  for (int side = 0; side < 2; ++side) {
+    const int64_t m = (side ? nk : nq) - d, k = m < (side ? nq : nk) ? m : (side ? nq : nk);
+    if (k > 0) n += k * m - k * (k - 1) / 2;  // m + (m - 1) + ..., k terms
+  }
+  return n;
 }
 // Offset whose table rows a far block of this side reads.
 DSA_DEV int far_offset(const FwdParams& p, int side) { return side == 0 ? p.Lq - 1 : -(p.Lk - 1); }

@@ -35,6 +35,10 @@ Tensor layouts (see include/dsa.h):
                     2 att_span, O's rounding residual (dsa_fwd_args.out_lo,
                     bfloat16 [B, Lq, H, D] at a 256-byte aligned offset);
                     empty when there is neither
+  rel_saturated     a hint: the offset distance from which on rel_table holds
+                    its end values (0: taken as 2 att_span); it decides which
+                    kernels run, not what they compute, and is the same in the
+                    forward and its backward
 """
 
 from __future__ import annotations
@@ -165,6 +169,7 @@ def _fill_fwd_args(
     dropout_t: int = 0,
     dropout_seed: Optional[Tensor] = None,
     dropout_bits: Optional[Tensor] = None,
+    rel_saturated: int = 0,
 ) -> _lib.DsaFwdArgs:
     B, Lq, H, D = q.shape
     Lk = k.shape[1]
@@ -199,6 +204,7 @@ def _fill_fwd_args(
     a.dtype = _DTYPES[q.dtype]
     a.flags = _flags(kr, qr)
     a.scale = float(scale)
+    a.rel_saturated = int(rel_saturated)
     if qc is not None:
         a.qc = qc.data_ptr()
         a.qc_strides[:] = _strides3(qc)
@@ -294,6 +300,7 @@ def _dsa_fwd_impl(
     qc: Optional[Tensor] = None,
     dropout_t: int = 0,
     dropout_seed: Optional[Tensor] = None,
+    rel_saturated: int = 0,
 ) -> tuple[Tensor, Tensor, Tensor, Tensor]:
     """(out, lse, bias, drop_bits).  With c2p/p2c and ``save_bias`` the
     relative score term is written to ``bias`` for the backward (which
@@ -319,7 +326,7 @@ def _dsa_fwd_impl(
     drop_bits = torch.empty((aux_layout(q, k, dropout_t, residual)[2],), dtype=torch.uint8, device=q.device)
     args = _fill_fwd_args(
         q, k, v, kr, qr, rel_table, key_keep, pair_keep, out, lse, att_span, scale, bias, qc, dropout_t, dropout_seed,
-        drop_bits,
+        drop_bits, rel_saturated,
     )
     lib = _lib.load()
     # scratch for the heaviest-first launch order under key / segment masks,
@@ -347,7 +354,7 @@ dsa_fwd = torch.library.custom_op(
 @dsa_fwd.register_fake
 def _dsa_fwd_fake(
     q, k, v, kr, qr, rel_table, key_keep, pair_keep, att_span, scale, save_bias=True, qc=None, dropout_t=0,
-    dropout_seed=None,
+    dropout_seed=None, rel_saturated=0,
 ):
     B, Lq, H, D = q.shape
     out = q.new_empty((B, Lq, H, D))
@@ -391,6 +398,7 @@ def fill_bwd_args(
     dropout_seed: Optional[Tensor] = None,
     dropout_bits: Optional[Tensor] = None,
     dtab_rows_first: bool = False,
+    rel_saturated: int = 0,
 ) -> _lib.DsaBwdArgs:
     """Backward arguments.  dkr / dqr are fp32 and accumulated into, or, with
     ``dtab_overwrite``, written (fp32 or bf16, their dtype); their memory is
@@ -401,7 +409,7 @@ def fill_bwd_args(
     a = _lib.DsaBwdArgs()
     a.fwd = _fill_fwd_args(
         q, k, v, kr, qr, rel_table, key_keep, pair_keep, out, lse, att_span, scale, bias, qc, dropout_t, dropout_seed,
-        dropout_bits,
+        dropout_bits, rel_saturated,
     )
     if dqc is not None:
         a.dqc = dqc.data_ptr()
@@ -475,6 +483,7 @@ def _dsa_bwd_impl(
     dropout_t: int = 0,
     dropout_seed: Optional[Tensor] = None,
     drop_bits: Optional[Tensor] = None,
+    rel_saturated: int = 0,
 ) -> tuple[Tensor, Tensor, Tensor, Tensor, Tensor, Tensor]:
     """Gradients (dq, dk, dv, dkr, dqr, dqc).  With ``dqkv`` (a contiguous
     ``[B, L, 3, H, D]`` buffer), dq, dk and dv are written into its three
@@ -513,7 +522,7 @@ def _dsa_bwd_impl(
         dout, q, k, v, kr, qr, rel_table, key_keep, pair_keep, out, lse, bias, att_span, scale,
         dq, dk, dv, dkr if kr is not None else None, dqr if qr is not None else None, dtab_overwrite=True,
         qc=qc, dqc=dqc if qc is not None else None, dropout_t=dropout_t, dropout_seed=dropout_seed,
-        dropout_bits=drop_bits, dtab_rows_first=rows_first,
+        dropout_bits=drop_bits, dtab_rows_first=rows_first, rel_saturated=rel_saturated,
     )
     ws = torch.empty((max(bwd_workspace_bytes(args), 16),), dtype=torch.uint8, device=q.device)
     args.workspace = ws.data_ptr()
@@ -531,7 +540,7 @@ dsa_bwd = torch.library.custom_op(
 @dsa_bwd.register_fake
 def _dsa_bwd_fake(
     dout, q, k, v, kr, qr, rel_table, key_keep, pair_keep, out, lse, bias, att_span, scale, qc=None, dqkv=None,
-    dropout_t=0, dropout_seed=None, drop_bits=None,
+    dropout_t=0, dropout_seed=None, drop_bits=None, rel_saturated=0,
 ):
     H, D = q.shape[2], q.shape[3]
     R = 2 * int(att_span)
@@ -550,8 +559,8 @@ def _dsa_bwd_fake(
 
 
 def _setup_context(ctx, inputs, output):
-    q, k, v, kr, qr, rel_table, key_keep, pair_keep, att_span, scale, save_bias, qc, dropout_t, dropout_seed = (
-        _with_dropout(inputs, 12)
+    q, k, v, kr, qr, rel_table, key_keep, pair_keep, att_span, scale, save_bias, qc, dropout_t, dropout_seed, sat = (
+        _with_trailing(inputs, 12)
     )
     out, lse, bias, drop_bits = output
     ctx.mark_non_differentiable(lse, bias, drop_bits)
@@ -562,25 +571,26 @@ def _setup_context(ctx, inputs, output):
     ctx.att_span = att_span
     ctx.scale = scale
     ctx.dropout_t = dropout_t
+    ctx.rel_saturated = sat
 
 
-def _with_dropout(inputs: tuple, n: int) -> tuple:
-    """The op's inputs with the two trailing dropout arguments filled in
-    (callers may leave them out)."""
-    return tuple(inputs) + (0, None)[len(inputs) - n:] if len(inputs) < n + 2 else tuple(inputs)
+def _with_trailing(inputs: tuple, n: int) -> tuple:
+    """The op's inputs with the trailing dropout and rel_saturated arguments
+    filled in (callers may leave them out)."""
+    return tuple(inputs) + (0, None, 0)[len(inputs) - n:] if len(inputs) < n + 3 else tuple(inputs)
 
 
 def _backward(ctx, dout, dlse, dbias, ddrop):
     q, k, v, kr, qr, rel_table, key_keep, pair_keep, out, lse, bias, qc, dropout_seed, drop_bits = ctx.saved_tensors
     if dout is None:  # the output itself received no gradient
-        return (None,) * 14
+        return (None,) * 15
     dq, dk, dv, dkr, dqr, dqc = _eager.on_eager(ctx, dsa_bwd, _dsa_bwd_impl)(
         dout, q, k, v, kr, qr, rel_table, key_keep, pair_keep, out, lse, bias, ctx.att_span, ctx.scale, qc, None,
-        ctx.dropout_t, dropout_seed, drop_bits,
+        ctx.dropout_t, dropout_seed, drop_bits, ctx.rel_saturated,
     )
     return (
         dq, dk, dv, (dkr if kr is not None else None), (dqr if qr is not None else None),
-        None, None, None, None, None, None, (dqc if qc is not None else None), None, None,
+        None, None, None, None, None, None, (dqc if qc is not None else None), None, None, None,
     )
 
 
@@ -603,16 +613,19 @@ def attention(
     qc: Optional[Tensor] = None,
     dropout_t: int = 0,
     dropout_seed: Optional[Tensor] = None,
+    rel_saturated: int = 0,
 ) -> tuple[Tensor, Tensor, Tensor, Tensor]:
     """``deberta_amd::dsa_fwd`` with its autograd: the op itself under
     torch.compile or tracing, its implementation in a torch.autograd.Function
     in plain eager mode (the same kernels, less host time)."""
     if _eager.eager(q):
         return _DsaFwdFunction.apply(
-            q, k, v, kr, qr, rel_table, key_keep, pair_keep, att_span, scale, save_bias, qc, dropout_t, dropout_seed
+            q, k, v, kr, qr, rel_table, key_keep, pair_keep, att_span, scale, save_bias, qc, dropout_t, dropout_seed,
+            rel_saturated,
         )
     return torch.ops.deberta_amd.dsa_fwd(
-        q, k, v, kr, qr, rel_table, key_keep, pair_keep, att_span, scale, save_bias, qc, dropout_t, dropout_seed
+        q, k, v, kr, qr, rel_table, key_keep, pair_keep, att_span, scale, save_bias, qc, dropout_t, dropout_seed,
+        rel_saturated,
     )
 
 
@@ -636,13 +649,15 @@ def _dsa_fwd_packed_impl(
     qc: Optional[Tensor] = None,
     dropout_t: int = 0,
     dropout_seed: Optional[Tensor] = None,
+    rel_saturated: int = 0,
 ) -> tuple[Tensor, Tensor, Tensor, Tensor]:
     """``dsa_fwd`` on ``q, k, v = qkv.unbind(2)`` (qkv ``[B, L, 3, H, D]``)."""
     if qkv.dim() != 5 or qkv.shape[2] != 3:
         raise ValueError(f"dsa: qkv must be [B, L, 3, H, D], got {tuple(qkv.shape)}")
     q, k, v = qkv.unbind(2)
     return _dsa_fwd_impl(
-        q, k, v, kr, qr, rel_table, key_keep, pair_keep, att_span, scale, save_bias, qc, dropout_t, dropout_seed
+        q, k, v, kr, qr, rel_table, key_keep, pair_keep, att_span, scale, save_bias, qc, dropout_t, dropout_seed,
+        rel_saturated,
     )
 
 
@@ -654,11 +669,12 @@ dsa_fwd_packed = torch.library.custom_op(
 @dsa_fwd_packed.register_fake
 def _dsa_fwd_packed_fake(
     qkv, kr, qr, rel_table, key_keep, pair_keep, att_span, scale, save_bias=True, qc=None, dropout_t=0,
-    dropout_seed=None,
+    dropout_seed=None, rel_saturated=0,
 ):
     q, k, _ = qkv.unbind(2)
     return _dsa_fwd_fake(
-        q, k, k, kr, qr, rel_table, key_keep, pair_keep, att_span, scale, save_bias, qc, dropout_t, dropout_seed
+        q, k, k, kr, qr, rel_table, key_keep, pair_keep, att_span, scale, save_bias, qc, dropout_t, dropout_seed,
+        rel_saturated,
     )
 
 
@@ -679,6 +695,7 @@ def _dsa_bwd_packed_impl(
     dropout_t: int = 0,
     dropout_seed: Optional[Tensor] = None,
     drop_bits: Optional[Tensor] = None,
+    rel_saturated: int = 0,
 ) -> tuple[Tensor, Tensor, Tensor, Tensor]:
     """Gradients (dqkv, dkr, dqr, dqc) of ``dsa_fwd_packed``: dqkv a
     contiguous ``[B, L, 3, H, D]`` tensor in qkv's dtype."""
@@ -686,7 +703,7 @@ def _dsa_bwd_packed_impl(
     dqkv = torch.empty(qkv.shape, dtype=qkv.dtype, device=qkv.device)
     _, _, _, dkr, dqr, dqc = _dsa_bwd_impl(
         dout, q, k, v, kr, qr, rel_table, key_keep, pair_keep, out, lse, bias, att_span, scale, qc, dqkv=dqkv,
-        dropout_t=dropout_t, dropout_seed=dropout_seed, drop_bits=drop_bits,
+        dropout_t=dropout_t, dropout_seed=dropout_seed, drop_bits=drop_bits, rel_saturated=rel_saturated,
     )
     return dqkv, dkr, dqr, dqc
 
@@ -699,7 +716,7 @@ dsa_bwd_packed = torch.library.custom_op(
 @dsa_bwd_packed.register_fake
 def _dsa_bwd_packed_fake(
     dout, qkv, kr, qr, rel_table, key_keep, pair_keep, out, lse, bias, att_span, scale, qc=None, dropout_t=0,
-    dropout_seed=None, drop_bits=None,
+    dropout_seed=None, drop_bits=None, rel_saturated=0,
 ):
     q, k, v = qkv.unbind(2)
     _, _, _, dkr, dqr, dqc = _dsa_bwd_fake(
@@ -709,8 +726,8 @@ def _dsa_bwd_packed_fake(
 
 
 def _setup_context_packed(ctx, inputs, output):
-    qkv, kr, qr, rel_table, key_keep, pair_keep, att_span, scale, save_bias, qc, dropout_t, dropout_seed = (
-        _with_dropout(inputs, 10)
+    qkv, kr, qr, rel_table, key_keep, pair_keep, att_span, scale, save_bias, qc, dropout_t, dropout_seed, sat = (
+        _with_trailing(inputs, 10)
     )
     out, lse, bias, drop_bits = output
     ctx.mark_non_differentiable(lse, bias, drop_bits)
@@ -719,19 +736,20 @@ def _setup_context_packed(ctx, inputs, output):
     ctx.att_span = att_span
     ctx.scale = scale
     ctx.dropout_t = dropout_t
+    ctx.rel_saturated = sat
 
 
 def _backward_packed(ctx, dout, dlse, dbias, ddrop):
     qkv, kr, qr, rel_table, key_keep, pair_keep, out, lse, bias, qc, dropout_seed, drop_bits = ctx.saved_tensors
     if dout is None:
-        return (None,) * 12
+        return (None,) * 13
     dqkv, dkr, dqr, dqc = _eager.on_eager(ctx, dsa_bwd_packed, _dsa_bwd_packed_impl)(
         dout, qkv, kr, qr, rel_table, key_keep, pair_keep, out, lse, bias, ctx.att_span, ctx.scale, qc,
-        ctx.dropout_t, dropout_seed, drop_bits,
+        ctx.dropout_t, dropout_seed, drop_bits, ctx.rel_saturated,
     )
     return (
         dqkv, (dkr if kr is not None else None), (dqr if qr is not None else None),
-        None, None, None, None, None, None, (dqc if qc is not None else None), None, None,
+        None, None, None, None, None, None, (dqc if qc is not None else None), None, None, None,
     )
 
 
@@ -752,15 +770,18 @@ def attention_packed(
     qc: Optional[Tensor] = None,
     dropout_t: int = 0,
     dropout_seed: Optional[Tensor] = None,
+    rel_saturated: int = 0,
 ) -> tuple[Tensor, Tensor, Tensor, Tensor]:
     """``attention`` on packed ``qkv`` ``[B, L, 3, H, D]``: the gradient of
     qkv comes back as one tensor."""
     if _eager.eager(qkv):
         return _DsaFwdPackedFunction.apply(
-            qkv, kr, qr, rel_table, key_keep, pair_keep, att_span, scale, save_bias, qc, dropout_t, dropout_seed
+            qkv, kr, qr, rel_table, key_keep, pair_keep, att_span, scale, save_bias, qc, dropout_t, dropout_seed,
+            rel_saturated,
         )
     return torch.ops.deberta_amd.dsa_fwd_packed(
-        qkv, kr, qr, rel_table, key_keep, pair_keep, att_span, scale, save_bias, qc, dropout_t, dropout_seed
+        qkv, kr, qr, rel_table, key_keep, pair_keep, att_span, scale, save_bias, qc, dropout_t, dropout_seed,
+        rel_saturated,
     )
 
 

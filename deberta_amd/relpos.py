@@ -44,6 +44,17 @@ def make_log_bucket_position(relative_pos: torch.Tensor, bucket_size: int, max_p
     return bucket.to(torch.long)
 
 
+def saturation_distance(bucket_size: int, max_position: int, att_span: int) -> int:
+    """Offset distance from which on the tables' rows no longer change, from
+    the configuration alone: where log buckets clamp the offset, or where the
+    kernels clamp it to ``att_span`` (the kernels' hint ``rel_saturated``)."""
+    if int(bucket_size) > 0 and int(max_position) > 0:
+        if int(bucket_size) // 2 > 1:
+            return max(int(max_position) - 1, 1)
+        return max(min(int(max_position) - 1, int(att_span)), 1)
+    return max(int(att_span), 1)
+
+
 def build_relative_position(
     query_len: int,
     key_len: int,

@@ -106,7 +106,8 @@ typedef struct dsa_fwd_args {
                              contiguous: the relative score term c2p + p2c
                              (unscaled; fp16 for bf16 inputs, fp32 for fp32),
                              written for dsa_bwd, which reads what a call of
-                             the same extents and masks wrote: tiles a mask
+                             the same extents, masks and rel_saturated wrote:
+                             tiles a mask
                              skips and blocks past the tables' saturation on
                              both sides are left as they are.  NULL: not
                              written. */
@@ -187,6 +188,14 @@ typedef struct dsa_fwd_args {
      where the other sums cancel it.  NULL: no residual; ignored for fp32.
      (Version 11.) */
   void* out_lo;
+  /* Optional, a hint: an offset distance from which on rel_table holds its end
+     values on both sides, as far as the caller knows without reading it (e.g.
+     max_position - 1 of a log-bucketed table); 0: taken as 2 att_span.  It
+     only decides whether the call looks for blocks past the saturation, whose
+     kernels are the slower ones where there are few: the results are those of
+     rel_table whatever it says.  The same in dsa_fwd and the dsa_bwd that
+     reads its bias.  (Version 13.) */
+  int32_t rel_saturated;
 } dsa_fwd_args;
 
 typedef struct dsa_bwd_args {

@@ -1,5 +1,6 @@
 """Far blocks: 128 x 128 blocks of (query, key) pairs whose relative position
-has saturated, run without bands (FarSpan, dsa_tiles.h).  The op against the
+has saturated, run without bands (FarSpan, dsa_tiles.h) where a call has
+enough of them (far_call, dsa_launch.h).  The op against the
 CPU oracle where the rule or the span can go wrong: extents on both sides of
 the rule, a span on one side only, past the last query or key block or
 nowhere, every mask form that takes it, dropout and the p2p query rows; and
@@ -36,6 +37,8 @@ _CASES = [
     Case(B=2, H=2, L=500, D=64, buckets=32, max_pos=64, mask="dead", seed=14),
     Case(B=1, H=2, L=600, D=64, buckets=32, max_pos=64, dropout=0.1, seed=15),
     Case(B=2, H=1, L=700, D=64, buckets=32, max_pos=64, mask="seg", dropout=0.1, seed=16),
+    Case(B=1, H=2, L=512, D=64, buckets=-1, max_pos=1, seed=17),  # saturated beside the diagonal, 4 blocks
+    Case(B=2, H=2, L=700, D=32, buckets=32, max_pos=64, mask="seg_mixed", seed=18),
 ]
 
 
@@ -188,7 +191,7 @@ def _same(got, want):
 def test_far_dead_rows_overflow(kind, dtype, gpu):
     """Padded query rows whose products with the tables overflow, beside live
     ones of the same 32 rows, change nothing: as with zeros there."""
-    c = Case(B=2, H=2, L=640, D=64, buckets=32, max_pos=64, seed=22)
+    c = Case(B=2, H=2, L=768, D=64, buckets=32, max_pos=64, seed=22)
     x = _padded(c, 530, kind)
     x["q"][:, 530:] = 0
     want = _grads(c, x, dtype, gpu)
@@ -201,7 +204,7 @@ def test_far_dead_rows_overflow(kind, dtype, gpu):
 def test_far_dead_chunks(kind, dtype, gpu):
     """What the padded queries of 32-row chunks without a live one hold (NaN)
     reaches nothing, the far rows of dKr included."""
-    c = Case(B=2, H=2, L=640, D=64, buckets=32, max_pos=64, seed=23)
+    c = Case(B=2, H=2, L=768, D=64, buckets=32, max_pos=64, seed=23)
     x = _padded(c, 544, kind)
     for n in ("q", "dout"):
         x[n][:, 544:] = 0
@@ -256,3 +259,38 @@ def test_far_term_not_finite(value, dtype, gpu):
     assert torch.isfinite(got[0][0]).all()
     for a, b in zip(*got):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("D", [32, 64])
+@pytest.mark.parametrize("dropout", [0.0, 0.1])
+@pytest.mark.parametrize("types", ["c2p|p2c", "c2p|p2c|p2p"])
+@pytest.mark.parametrize("mask", ["none", "key", "seg", "pair"])
+def test_far_kernels(mask, types, dropout, D, dtype, gpu):
+    """Every form of the kernels with far blocks (66% of the blocks here)."""
+    c = Case(B=1, H=2, L=900, D=D, buckets=32, max_pos=64, types=types, mask=mask, dropout=dropout, seed=26)
+    _check(c, dtype, gpu, grads_to_scale=True)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("hint", [1, 100, 1 << 20])
+def test_far_hint(hint, dtype, gpu):
+    """What a caller says of the saturation (here at 255) decides the kernels
+    that run, not what they compute: too near, too far, none."""
+    from deberta_amd import ops  # noqa: F401
+    from deberta_amd.relpos import relative_offset_table
+
+    c = Case(B=1, H=2, L=700, D=64, buckets=64, max_pos=256, seed=27)
+    x = make_inputs(c)
+    table = relative_offset_table(c.L, c.L, bucket_size=c.buckets, max_position=c.max_pos, device=gpu)
+    runs = []
+    for h in (0, hint):
+        q, k, v, kr, qr = (x[n].to(gpu, dtype).requires_grad_() for n in ("q", "k", "v", "kr", "qr"))
+        out = torch.ops.deberta_amd.dsa_fwd(
+            q, k, v, kr, qr, table, None, None, c.A, 1 / math.sqrt(3 * c.D), True, None, 0, None, h
+        )[0]
+        runs.append([out.detach(), *torch.autograd.grad(out, [q, k, v, kr, qr], x["dout"].to(gpu, dtype))])
+    # far terms are fp32 sums where the bands are rounded (fp16 for bf16)
+    tol = 1e-5 if dtype == torch.float32 else 1e-2
+    for name, a, b in zip(("out", "dq", "dk", "dv", "dkr", "dqr"), *runs):
+        assert float((a.float() - b.float()).norm()) <= tol * float(a.float().norm()), name
