@@ -112,3 +112,37 @@ def test_forward_without_workspace_equals_bits(L, dtype, gpu):
     torch.cuda.synchronize(gpu)
     assert torch.equal(out, want)
     assert torch.equal(lse2, lse)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+def test_bytes_forward_bits_backward(dtype, gpu):
+    """A forward on the mask's bytes (no workspace) of a call long enough for
+    far blocks saves the bands everywhere; the backward takes the far blocks'
+    terms from its own products and the saved bands elsewhere."""
+    from deberta_amd import _lib, ops
+    from deberta_amd.masks import kernel_masks
+    from deberta_amd.relpos import relative_offset_table
+
+    c = Case(B=1, H=2, L=600, D=64, buckets=32, max_pos=64, seed=12)
+    x = make_inputs(c)
+    x["mask"] = _mask("mixed", c.B, c.L, c.H, torch.Generator().manual_seed(c.seed))
+    ref = oracle_run(c, x, dtype)
+    q, k, v, kr, qr, dout = (x[n].to(gpu, dtype) for n in ("q", "k", "v", "kr", "qr", "dout"))
+    table = relative_offset_table(c.L, c.L, bucket_size=c.buckets, max_position=c.max_pos, device=gpu)
+    _, pk = kernel_masks(x["mask"].to(gpu), c.B, c.L, c.L, gpu, segments_from_dense=False)
+    out = torch.empty_like(q)
+    lse = torch.empty(c.B, c.H, c.L, device=gpu)
+    bias = torch.empty(ops.bias_shape(q, k), dtype=ops.bias_dtype(dtype), device=gpu)
+    scale = 1 / math.sqrt(3 * c.D)
+    a = ops._fill_fwd_args(q, k, v, kr, qr, table, None, pk, out, lse, c.A, scale, bias)
+    n = _lib.load().dsa_fwd_workspace_bytes(ctypes.byref(a))
+    a.rel_saturated = 1 << 28
+    assert n == _lib.load().dsa_fwd_workspace_bytes(ctypes.byref(a)) + 256  # far blocks are looked for
+    a.rel_saturated = 0
+    _lib.check(_lib.load().dsa_fwd(ctypes.byref(a), ctypes.c_void_p(torch.cuda.current_stream(gpu).cuda_stream)), "dsa_fwd")
+    grads = torch.ops.deberta_amd.dsa_bwd(dout, q, k, v, kr, qr, table, None, pk, out, lse, bias, c.A, scale)
+    got = dict(zip(("out", "dq", "dk", "dv", "dkr", "dqr"), [out, *grads]))
+    for name, r in ref.items():
+        g = got[name].float().cpu()
+        err, tol = (max_rel(g, r), 1e-4) if dtype == torch.float32 else (min(max_rel(g, r), max_abs(g, r)), 2e-2)
+        assert err <= tol, (name, err)
