@@ -25,15 +25,17 @@ _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 def eager(t: torch.Tensor) -> bool:
     """True when a call with main input ``t`` may bypass ``torch.ops``: a
     plain tensor, or a module's parameter (the relative table's LayerNorm
-    reads one: 240 us of a layer step's 1700 us of host time went into its
-    custom op's wrappers, forward and backward)."""
+    reads one, and its custom op's wrappers, forward and backward, were host
+    time of every layer step)."""
     # is_compiling() first: dynamo folds it to True while tracing, and the
     # dispatch-stack query after it (a C function dynamo does not trace)
     # would otherwise break the graph
-    if torch.compiler.is_compiling() or _dispatch_depth() != 0:
-        return False
     # (torch.jit.trace records the op of a parameter)
-    return type(t) is torch.Tensor or (type(t) is torch.nn.Parameter and not torch.jit.is_tracing())
+    return (
+        not torch.compiler.is_compiling()
+        and _dispatch_depth() == 0
+        and (type(t) is torch.Tensor or (type(t) is torch.nn.Parameter and not torch.jit.is_tracing()))
+    )
 
 
 def refuse_capture(what: str) -> None:
@@ -74,7 +76,8 @@ def function(
     def forward(ctx, *inputs):
         output = impl(*inputs)
         ctx.eager = True
-        ctx.op_in_graph = type(inputs[0]) is torch.nn.Parameter
+        if type(inputs[0]) is torch.nn.Parameter:
+            ctx.op_in_graph = True
         setup_context(ctx, inputs, output)
         return output
 

@@ -367,6 +367,10 @@ class DisentangledSelfAttention(nn.Module):
         self.pos_ebd_size = self.max_relative_positions
         if self.position_buckets > 0:
             self.pos_ebd_size = self.position_buckets
+        # the kernels' hint of where the relative table saturates
+        self._rel_saturated = saturation_distance(
+            self.position_buckets, self.max_relative_positions, self.pos_ebd_size
+        )
 
         self.pos_dropout = nn.Dropout(float(getattr(config, "hidden_dropout_prob", 0.0)))
         self.attn_kernel = normalize_attention_kernel(getattr(config, "hf_attention_kernel", "dynamic"))
@@ -584,9 +588,9 @@ class DisentangledSelfAttention(nn.Module):
 
         # the op takes the packed projection whole (its gradient comes back
         # as one tensor)
-        sat = saturation_distance(self.position_buckets, self.max_relative_positions, att_span)
         ctx = fused_attention(
-            q, k, v, kr, qr, table, attention_mask, att_span, scale, qc, qkv=qkv, dropout_p=drop_p, rel_saturated=sat
+            q, k, v, kr, qr, table, attention_mask, att_span, scale, qc, qkv=qkv, dropout_p=drop_p,
+            rel_saturated=self._rel_saturated,
         )
         bsz, seq_len = ctx.shape[0], ctx.shape[1]
         context_layer = ctx.reshape(bsz, seq_len, self.all_head_size).to(dtype=model_dtype)

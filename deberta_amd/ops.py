@@ -204,7 +204,8 @@ def _fill_fwd_args(
     a.dtype = _DTYPES[q.dtype]
     a.flags = _flags(kr, qr)
     a.scale = float(scale)
-    a.rel_saturated = int(rel_saturated)
+    if rel_saturated:
+        a.rel_saturated = int(rel_saturated)
     if qc is not None:
         a.qc = qc.data_ptr()
         a.qc_strides[:] = _strides3(qc)
