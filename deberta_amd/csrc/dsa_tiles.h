@@ -190,9 +190,10 @@ DSA_DEV SegRange wg_seg_range(int s, bool has, int* red) {
 // blocks at L = 2048, 74% at L = 4096.  Whether blocks can be far is decided
 // on the host from the extents (far_call), so shorter calls search nothing.
 // One workgroup of the preparation before the forward, and one of the
-// backward's prep kernel, find the span for the kernels after them (2 us at
-// L = 4096, beside the preparation's other blocks); a forward without a
-// workspace finds it in each of its workgroups.
+// backward's prep kernel, find the span for the kernels after them (beside the
+// preparation's other blocks: the forward's 6.4 -> 7.5 us at L = 4096, 22 with
+// one offset a thread and round trip); a forward without a workspace finds it
+// in each of its workgroups.
 constexpr int kNoFar = 1 << 26;  // a block diagonal past every call's (and 4x it, the 32-query tiles, in range)
 struct FarSpan {
   int pos, neg;  // far iff delta >= pos or delta <= neg
@@ -224,21 +225,37 @@ DSA_DEV int offset_row(const int32_t* rel, int d, int Lq, int Lk, int A, bool p2
 DSA_DEV FarSpan far_span(const FwdParams& p, int* red) {
   FarSpan s{kNoFar, -kNoFar};
   if (!p.far) return s;
-  int last[2];  // the furthest offset of a side whose rows differ from the end's
+  // The furthest offset of a side whose rows differ from its end's.  Both
+  // sides' offsets are read eight a thread at a time (past a side's end, the
+  // end itself): two round trips at L = 4096 in place of one an offset.
+  int last[2] = {0, 0}, n[2], ce[2], pe[2];
 #pragma unroll
   for (int side = 0; side < 2; ++side) {
-    const int e = far_offset(p, side), n = side == 0 ? e : -e;
-    const int ce = offset_row(p.rel, e, p.Lq, p.Lk, p.A, false), pe = offset_row(p.rel, e, p.Lq, p.Lk, p.A, true);
-    int m = 0;
-#pragma unroll 8
-    for (int o = 1 + (int)threadIdx.x; o < n; o += 256) {
-      const int t = min(max(p.rel[(side == 0 ? o : -o) + p.Lk - 1], -p.A), p.A);
-      if (((p.flags & 1) && c2p_row(t, p.A) != ce) || ((p.flags & 2) && p2c_row(t, p.A) != pe)) m = o;
+    const int e = far_offset(p, side);
+    n[side] = side == 0 ? e : -e;
+    ce[side] = offset_row(p.rel, e, p.Lq, p.Lk, p.A, false);
+    pe[side] = offset_row(p.rel, e, p.Lq, p.Lk, p.A, true);
+  }
+  for (int o0 = 1 + (int)threadIdx.x; o0 < max(n[0], n[1]); o0 += 8 * 256) {
+    int t[2][8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      t[0][u] = p.rel[min(o0 + 256 * u, n[0]) + p.Lk - 1];
+      t[1][u] = p.rel[p.Lk - 1 - min(o0 + 256 * u, n[1])];
     }
 #pragma unroll
-    for (int k = 32; k >= 1; k >>= 1) m = max(m, __shfl_xor(m, k));
-    last[side] = m;
+    for (int side = 0; side < 2; ++side)
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int r = min(max(t[side][u], -p.A), p.A);
+        if (((p.flags & 1) && c2p_row(r, p.A) != ce[side]) || ((p.flags & 2) && p2c_row(r, p.A) != pe[side]))
+          last[side] = o0 + 256 * u;
+      }
   }
+#pragma unroll
+  for (int side = 0; side < 2; ++side)
+#pragma unroll
+    for (int k = 32; k >= 1; k >>= 1) last[side] = max(last[side], __shfl_xor(last[side], k));
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = last[0], red[4 + (threadIdx.x >> 6)] = last[1];
   __syncthreads();
   const int4 a = *reinterpret_cast<const int4*>(red), b = *reinterpret_cast<const int4*>(red + 4);
