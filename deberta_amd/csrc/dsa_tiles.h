@@ -228,6 +228,7 @@ DSA_DEV FarSpan far_span(const FwdParams& p, int* red) {
   // The furthest offset of a side whose rows differ from its end's.  Both
   // sides' offsets are read eight a thread at a time (past a side's end, the
   // end itself): two round trips at L = 4096 in place of one an offset.
+  const int c2p = (p.flags & 1) ? -1 : 0, p2c = (p.flags & 2) ? -1 : 0;
   int last[2] = {0, 0}, n[2], ce[2], pe[2];
 #pragma unroll
   for (int side = 0; side < 2; ++side) {
@@ -248,8 +249,9 @@ DSA_DEV FarSpan far_span(const FwdParams& p, int* red) {
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
         const int r = min(max(t[side][u], -p.A), p.A);
-        if (((p.flags & 1) && c2p_row(r, p.A) != ce[side]) || ((p.flags & 2) && p2c_row(r, p.A) != pe[side]))
-          last[side] = o0 + 256 * u;
+        // (without branches: hipcc lost the p2c side of a short-circuit here)
+        const int differs = ((c2p_row(r, p.A) ^ ce[side]) & c2p) | ((p2c_row(r, p.A) ^ pe[side]) & p2c);
+        last[side] = differs ? o0 + 256 * u : last[side];
       }
   }
 #pragma unroll

@@ -106,8 +106,9 @@ def test_far_stage_split(Lq, Lk, p2p, dtype, gpu):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("types", ["c2p|p2c", "c2p", "p2c"])
 @pytest.mark.parametrize("mask", ["none", "key"])
-def test_far_table_not_monotone(mask, dtype, gpu):
+def test_far_table_not_monotone(mask, types, dtype, gpu):
     """A table that comes back to its end's rows on every block diagonal but
     not on the offsets between them has no far block: out, dq, dk and dv are
     those of any Toeplitz table (dkr and dqr need a monotone one).  The forward
@@ -116,24 +117,26 @@ def test_far_table_not_monotone(mask, dtype, gpu):
     from deberta_amd.masks import kernel_masks
     from oracle import eager
 
-    c = Case(B=2, H=2, L=514, D=64, buckets=32, max_pos=64, mask=mask, seed=21)
+    c = Case(B=2, H=2, L=514, D=64, buckets=32, max_pos=64, mask=mask, types=types, seed=21)
     x = make_inputs(c)
     d = torch.arange(-(c.L - 1), c.L)
     table = (d + 32) % 64 - 32
     i = torch.arange(c.L)
     leaf = lambda t: t.to(dtype).float().requires_grad_()
     hm = lambda t: t.permute(0, 2, 1, 3)
-    rq, rk, rv, rkr, rqr = (leaf(x[n]) for n in ("q", "k", "v", "kr", "qr"))
+    rq, rk, rv = (leaf(x[n]) for n in ("q", "k", "v"))
+    rkr, rqr = (leaf(x[n]) if t in c.type_list else None for n, t in (("kr", "c2p"), ("qr", "p2c")))
     ctx, _ = eager.attend(
         hm(rq), hm(rk), hm(rv), rkr, rqr, table[i[:, None] - i[None] + c.L - 1], x["mask"], types=c.type_list,
         att_span=c.A, use_relative=True,
     )
     ref = [ctx, *torch.autograd.grad(ctx, [rq, rk, rv], hm(x["dout"].to(dtype).float()))]
 
-    q, k, v, kr, qr = (x[n].to(gpu, dtype).requires_grad_() for n in ("q", "k", "v", "kr", "qr"))
+    q, k, v = (x[n].to(gpu, dtype).requires_grad_() for n in ("q", "k", "v"))
+    kr, qr = (x[n].to(gpu, dtype).requires_grad_() if t in c.type_list else None for n, t in (("kr", "c2p"), ("qr", "p2c")))
     rel = table.to(gpu, torch.int32)
     kk, _ = kernel_masks(None if x["mask"] is None else x["mask"].to(gpu), c.B, c.L, c.L, gpu)
-    scale = 1 / math.sqrt(3 * c.D)
+    scale = 1 / math.sqrt((1 + len(c.type_list)) * c.D)
     out, lse, _, _ = torch.ops.deberta_amd.dsa_fwd(q, k, v, kr, qr, rel, kk, None, c.A, scale, True)
     got = [hm(out), *torch.autograd.grad(out, [q, k, v], x["dout"].to(gpu, dtype))]
     for name, a, b in zip(("out", "dq", "dk", "dv"), got, ref):
