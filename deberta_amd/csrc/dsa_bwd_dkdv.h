@@ -42,8 +42,11 @@ constexpr int NW = 4, WK = 32, BKW = 128, BQ = 32;
 // DROP: attention dropout with the forward's keep bits p.drop
 // (dsa_dropout.h): dV sums the kept probabilities, scaled by p.drop_scale,
 // and dP keeps the kept pairs' dO . v, scaled the same way.
-// FAR: calls that can have far blocks (FarSpan, p.far); kept out of the others'
-// code, whose registers are all taken (252 of 256).
+// FAR: calls that look for far blocks (FarSpan, p.far); kept out of the others'
+// code, whose registers are all taken (250 of 256).  Its near tiles are slower
+// than the others' (50 to 100 scalar registers spill to vector lanes): at B=4,
+// L=2048, H=12 with 52% of the blocks far, 286 -> 292 us where the forward goes
+// from 274 to 230 and DQ|TABLE from 326 to 224 (far_call has the rule).
 template <typename T, int D, int MASK, bool DROP, bool FAR>
 __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
   using namespace kvcfg;
@@ -256,13 +259,13 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
   if constexpr (DROP) dropw = p.drop + drop_word0(b, h, p.H, p.LqP / 32, NKT64, 0, jw / 64);
   // Issues the LDS copies of query tile qi into the given buffers (lane
   // order = physical chunk order; Q and dO rows are clamped to Lq - 1, where
-  // probabilities are zero anyway), and, with ring set, its qrgt block
-  // (whose ring slot was last read two tiles earlier); with dropout, the
-  // wave's keep words.
+  // probabilities are zero anyway) and the last nring blocks of its qrgt
+  // window (one from the tile before, whose ring slot was last read two tiles
+  // earlier; five for the first near tile after far ones); with dropout, the
+  // wave's keep words, under a pair mask its bits.  side: the far side of a
+  // far tile, or -1.
   uint4 pnext = {0, 0, 0, 0};  // pair bits in registers: the lane's words of the next tile
   int qseg_next = 0;  // MASK_SEG: query segment of lane (w = 1, lane < 32) in the next tile
-  // nring: the last blocks of the tile's qrgt window to copy; side: the far
-  // side of a far tile, or -1.
   auto issue = [&](int qi, int nring, int side, T* Qd, T* dOd, BT* Bd, float* Rd, uint32_t* Dd, uint32_t* Pd) {
     const int i0 = qi * BQ;
     if (MASK == MASK_SEG && w == 1 && lane < BQ) qseg_next = (i0 + lane < Lq) ? sv(i0 + lane) : 0;
@@ -305,8 +308,6 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
     if (DROP && lane < 16) copy16(dropw + (int64_t)qi * NKT64 * 64, lane * 16, (char*)(Dd + w * 64));
   };
 
-  // dS rows i of the wave's 32 keys: lane (g, c16) writes keys jw + 16 kk +
-  // 4g + [0, 4) of query i0 + 16 mi + c16.
   typedef T vec4 __attribute__((ext_vector_type(4)));
   // dS rows i of the wave's 32 keys: lane (g, c16) writes keys jw + 8g +
   // [0, 8) of query i0 + 16 mi + c16, one 16-byte store (bf16; two for
@@ -411,9 +412,8 @@ __global__ __launch_bounds__(256, 2) void dsa_bwd_dkdv_kernel(BwdParams bp) {
         if constexpr (far) issue(qn, n + 1 == n2 ? 5 : 0, n + 1 < n1 ? 1 : n + 1 < n2 ? 0 : -1, nQ, ndO, nBt, nR, nDw, nPw);
         else issue(qn, qn == qi + 1, -1, nQ, ndO, nBt, nR, nDw, nPw);
       }
-      // With segments, a tile whose queries all share the workgroup's single
-      // key segment needs no masking beyond the dead-row test.  Other modes:
-      // tiles without a kept (query, key) pair store zeros.
+      // A listed tile marked full needs no masking.  Without a list, a tile
+      // past Lq stores zeros.
       const bool full = LIST && (ent & 0x4000);
       const bool skip = !LIST && i0 >= Lq;
       if (skip) {
