@@ -561,7 +561,7 @@ def _dsa_bwd_fake(
 
 def _setup_context(ctx, inputs, output):
     q, k, v, kr, qr, rel_table, key_keep, pair_keep, att_span, scale, save_bias, qc, dropout_t, dropout_seed, sat = (
-        _with_trailing(inputs, 12)
+        inputs if len(inputs) == 15 else _with_trailing(inputs, 12)
     )
     out, lse, bias, drop_bits = output
     ctx.mark_non_differentiable(lse, bias, drop_bits)
@@ -578,7 +578,7 @@ def _setup_context(ctx, inputs, output):
 def _with_trailing(inputs: tuple, n: int) -> tuple:
     """The op's inputs with the trailing dropout and rel_saturated arguments
     filled in (callers may leave them out)."""
-    return tuple(inputs) + (0, None, 0)[len(inputs) - n:] if len(inputs) < n + 3 else tuple(inputs)
+    return tuple(inputs) + (0, None, 0)[len(inputs) - n:]
 
 
 def _backward(ctx, dout, dlse, dbias, ddrop):
@@ -728,7 +728,7 @@ def _dsa_bwd_packed_fake(
 
 def _setup_context_packed(ctx, inputs, output):
     qkv, kr, qr, rel_table, key_keep, pair_keep, att_span, scale, save_bias, qc, dropout_t, dropout_seed, sat = (
-        _with_trailing(inputs, 10)
+        inputs if len(inputs) == 13 else _with_trailing(inputs, 10)
     )
     out, lse, bias, drop_bits = output
     ctx.mark_non_differentiable(lse, bias, drop_bits)
