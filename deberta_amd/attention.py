@@ -339,6 +339,10 @@ class DisentangledSelfAttention(nn.Module):
     and shapes, same config attributes read with the same defaults).
     """
 
+    # the kernels' hint of where the relative table saturates (0, a module saved
+    # before it was kept: unknown)
+    _rel_saturated = 0
+
     def __init__(self, config: Any) -> None:
         super().__init__()
         hidden_size = int(config.hidden_size)
@@ -367,7 +371,6 @@ class DisentangledSelfAttention(nn.Module):
         self.pos_ebd_size = self.max_relative_positions
         if self.position_buckets > 0:
             self.pos_ebd_size = self.position_buckets
-        # the kernels' hint of where the relative table saturates
         self._rel_saturated = saturation_distance(
             self.position_buckets, self.max_relative_positions, self.pos_ebd_size
         )

@@ -202,7 +202,7 @@ struct FarSpan {
 };
 // Blocks past a saturation at distance sat, of the nq x nk blocks of a call.
 inline int64_t far_blocks(int nq, int nk, int sat) {
-  const int d = sat > 1 ? (sat + 254) / 128 : 1;  // the first diagonal with 128 d - 127 >= sat
+  const int64_t d = sat > 1 ? ((int64_t)sat + 254) / 128 : 1;  // the first diagonal with 128 d - 127 >= sat
   int64_t n = 0;
   for (int side = 0; side < 2; ++side) {
     const int64_t m = (side ? nk : nq) - d, k = m < (side ? nq : nk) ? m : (side ? nq : nk);

@@ -55,6 +55,10 @@ def test_rule(form, need):
                 assert _looks(Lq, Lk, sat // 2, **form) == (far > 0 and share >= need - 1e-9), (Lq, Lk, sat, share)
 
 
+def test_largest_hint():
+    assert not _looks(4096, 4096, 32, 2**31 - 1)
+
+
 @pytest.mark.parametrize("buckets,max_pos", [(256, 512), (64, 512), (32, 64), (-1, 64), (2, 64), (8, 4), (24, 2)])
 def test_saturation_distance(buckets, max_pos):
     """No offset past the distance reads another row than the last one."""

@@ -297,3 +297,41 @@ def test_far_hint(hint, dtype, gpu):
     tol = 1e-5 if dtype == torch.float32 else 1e-2
     for name, a, b in zip(("out", "dq", "dk", "dv", "dkr", "dqr"), *runs):
         assert float((a.float() - b.float()).norm()) <= tol * float(a.float().norm()), name
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("kind", ["key", "seg", "pair"])
+def test_far_stage_split_masked(kind, dtype, gpu):
+    """The dq kernel alone, whose key tiles a mask lists, with far blocks:
+    DKDV, DQ, TABLE and SUM in calls of their own against one call."""
+    from deberta_amd import _lib, ops
+    from deberta_amd.masks import SegmentMask, kernel_masks
+    from deberta_amd.relpos import relative_offset_table
+
+    c = Case(B=2, H=2, L=768, D=64, buckets=32, max_pos=64, seed=28)
+    x = _padded(c, 700, kind)
+    q, k, v, kr, qr, dout = (x[n].to(gpu, dtype) for n in ("q", "k", "v", "kr", "qr", "dout"))
+    table = relative_offset_table(c.L, c.L, bucket_size=c.buckets, max_position=c.max_pos, device=gpu)
+    mask = SegmentMask(x["seg"]) if x["seg"] is not None else x["mask"].to(gpu)
+    kk, pk = kernel_masks(mask, c.B, c.L, c.L, gpu, segments_from_dense=False)
+    scale = 1 / math.sqrt(3 * c.D)
+    out, lse, bias, aux = torch.ops.deberta_amd.dsa_fwd(q, k, v, kr, qr, table, kk, pk, c.A, scale, True)
+    stream = ctypes.c_void_p(torch.cuda.current_stream(gpu).cuda_stream)
+    runs = []
+    for calls in ([""], ["PREP", "DKDV", "DQ", "TABLE", "SUM"]):
+        grads = [torch.full_like(t, float("nan")) for t in (q, k, v)]
+        tabs = [torch.zeros((c.H, 2 * c.A, c.D), dtype=torch.float32, device=gpu) for _ in range(2)]
+        a = ops.fill_bwd_args(dout, q, k, v, kr, qr, table, kk, pk, out, lse, bias, c.A, scale, *grads, *tabs,
+                              dropout_bits=aux)
+        ws = torch.empty((ops.bwd_workspace_bytes(a),), dtype=torch.uint8, device=gpu)
+        a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
+        for n in calls:
+            a.stages = getattr(_lib, f"DSA_STAGE_{n}") if n else 0
+            _lib.check(_lib.load().dsa_bwd(ctypes.byref(a), stream), "dsa_bwd")
+        torch.cuda.synchronize(gpu)
+        runs.append(grads + tabs)
+    for name, a, b in zip(("dq", "dk", "dv", "dkr", "dqr"), *runs):
+        if name in ("dkr", "dqr"):  # fp32 sums in another order
+            assert float((a - b).abs().max()) <= 1e-5 * float(a.abs().max()), name
+        else:
+            assert torch.isfinite(a).all() and torch.equal(a, b), name
