@@ -44,7 +44,7 @@ constexpr int NW = 4, WK = 32, BKW = 128, BQ = 32;
 // and dP keeps the kept pairs' dO . v, scaled the same way.
 // FAR: calls that look for far blocks (FarSpan, p.far); kept out of the others'
 // code, whose registers are all taken (250 of 256).  Its near tiles are slower
-// than the others' (50 to 100 scalar registers spill to vector lanes): at B=4,
+// than the others' (49 to 90 scalar registers spill to vector lanes): at B=4,
 // L=2048, H=12 with 52% of the blocks far, 286 -> 292 us where the forward goes
 // from 274 to 230 and DQ|TABLE from 326 to 224 (far_call has the rule).
 template <typename T, int D, int MASK, bool DROP, bool FAR>
