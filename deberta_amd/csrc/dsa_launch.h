@@ -60,23 +60,25 @@ static int elem_bytes(int dtype) { return dtype == DSA_BF16 ? 2 : 4; }
 // planes), so that calls with few far blocks lose.  Training step at 12 heads,
 // buckets 256 / max_position 512, 8192 tokens, plain -> FAR in us:
 //   L (share)     1024 (19%)  1152 (25%)  1408 (35%)  1536 (39%)  2048 (52%)
-//   no mask       493 -> 514  579 -> 559  620 -> 600  718 -> 655  952 -> 806
-//   ... p2p       491 -> 512  546 -> 545  599 -> 587  680 -> 644  933 -> 775
-//   ... and drop  550 -> 579  615 -> 627  675 -> 683  778 -> 745  1018 -> 903
-//   padded rows   397 -> 400  311 -> 309  358 -> 344  471 -> 405  485 -> 424
-//   causal, bits  390 -> 381  400 -> 391  431 -> 401  531 -> 478  687 -> 574
-// Documents know no share: those of 2/3 of a row gain from 39% on (441 -> 437,
-// 654 -> 606 at 52%, 644 -> 560 at L = 3072), those of 250 tokens hold no far
-// pair and lose 5 to 7% at any length (290 -> 303, 262 -> 282), more with
-// dropout (dkdv's registers again): they take long rows.  In float32 (4096
-// tokens) the registers fit: 6% 1006 -> 1023, 12% 1149 -> 1121, 30% 1604 ->
-// 1477; documents 30% 1242 -> 1189 and 605 -> 622.
+//   no mask       489 -> 503  565 -> 555  616 -> 581  707 -> 643  930 -> 791
+//   ... p2p       482 -> 503  542 -> 539  600 -> 579  674 -> 630  921 -> 766
+//   ... and drop  537 -> 566  605 -> 615  662 -> 664  761 -> 722  1002 -> 868
+//   padded rows   392 -> 395  311 -> 308  358 -> 339  467 -> 387  474 -> 410
+//   causal, bits  389 -> 378  400 -> 394  430 -> 398  532 -> 473  689 -> 565
+//   window, bits  204 -> 214  226 -> 237  224 -> 235  236 -> 246  260 -> 265
+// Documents know no share: those of 2/3 of a row gain from half of the blocks
+// on (434 -> 439 at 39%, 646 -> 591 at 52%, 632 -> 546 at L = 3072), those of
+// 250 tokens hold no far pair and lose 2 to 4% at any length (288 -> 295, 265
+// -> 270), more with dropout (dkdv's registers again: 331 -> 346 for 748 ->
+// 653): they take long rows.  In float32 (4096 tokens) the registers fit: 6%
+// 1013 -> 1022, 12% 1148 -> 1112, 30% 1605 -> 1467; documents 30% 1244 -> 1193
+// and 606 -> 618.
 static bool far_call(const dsa_fwd_args* a) {
   if (!a->flags) return false;
   const int nq = round_up(a->Lq, 128) / 128, nk = round_up(a->Lk, 128) / 128;
   const int64_t far = dsa::far_blocks(nq, nk, a->rel_saturated > 0 ? a->rel_saturated : 2 * a->att_span);
   const bool bf = a->dtype == DSA_BF16, drop = a->dropout_threshold != 0;
-  const int need = a->seg ? (!bf ? 30 : drop ? 60 : 50) : !bf ? 10 : a->qc ? 38 : 25;
+  const int need = a->seg ? (!bf ? 30 : drop ? 60 : 50) : !bf ? 10 : a->qc ? 34 : 25;
   return far > 0 && far * 100 >= (int64_t)nq * nk * need;
 }
 

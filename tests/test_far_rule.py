@@ -41,7 +41,7 @@ def _share(Lq, Lk, sat):
 @pytest.mark.parametrize(
     "form,need",
     [
-        (dict(), 0.25), (dict(drop=6554), 0.25), (dict(qc=True), 0.38), (dict(seg=True), 0.5),
+        (dict(), 0.25), (dict(drop=6554), 0.25), (dict(qc=True), 0.34), (dict(seg=True), 0.5),
         (dict(seg=True, drop=6554), 0.6), (dict(dtype=_lib.DSA_F32), 0.1), (dict(dtype=_lib.DSA_F32, seg=True), 0.3),
         (dict(dtype=_lib.DSA_F32, qc=True), 0.1),
     ],
